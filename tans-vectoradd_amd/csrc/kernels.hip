@@ -1055,7 +1055,7 @@ __global__ __launch_bounds__(kDecBlock) void fused_add_kernel(
     const uint16_t* __restrict__ a_st, const v2u* __restrict__ a_sm,
     const uint32_t* __restrict__ b_comp, int64_t b_words, const int64_t* __restrict__ b_off,
     const uint16_t* __restrict__ b_st, const v2u* __restrict__ b_sm,
-    const v2u* __restrict__ table, int64_t K, int n_tiles, v4u* __restrict__ out) {
+    const v2u* __restrict__ table, int64_t K, int n_tiles, int waves, v4u* __restrict__ out) {
     constexpr uint32_t L = Alpha<SPS>::L;
     constexpr int C = 2 * G;
     __shared__ DecSmem<SPS, C> smem;
@@ -1068,10 +1068,12 @@ __global__ __launch_bounds__(kDecBlock) void fused_add_kernel(
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
     const int64_t n_groups = (K + kLanes - 1) / kLanes;
-    const int64_t grid_groups = (int64_t)gridDim.x * kDecWaves * G;   // groups per round
-    int64_t g0 = ((int64_t)blockIdx.x * kDecWaves + wave) * G;
+    // the first `waves` waves of each workgroup decode (spread_waves); the
+    // others only help load the table
+    const int64_t grid_groups = (int64_t)gridDim.x * waves * G;   // groups per round
+    int64_t g0 = wave < waves ? ((int64_t)blockIdx.x * waves + wave) * G : n_groups;
     const bool live = g0 < n_groups;   // wave-uniform
-    const int64_t wg_groups = n_groups - (int64_t)blockIdx.x * kDecWaves * G;
+    const int64_t wg_groups = n_groups - (int64_t)blockIdx.x * waves * G;
     constexpr bool PACKED = FIRST < 0;
     // segments loaded at a start, and sign/mantissa tiles loaded then
     constexpr int NSEG = FIRST > 0 ? FIRST : PACKED ? pack_segs(-FIRST) : kSlots;
@@ -1084,7 +1086,7 @@ __global__ __launch_bounds__(kDecBlock) void fused_add_kernel(
                   "a resident stream's sign/mantissa tiles are all loaded at its start");
     FusedWave<SPS, G, FIRST> w;
     w.progress = &smem.progress;
-    w.live = (uint32_t)(wg_groups >= (int64_t)kDecWaves * G ? kDecWaves : (wg_groups + G - 1) / G);
+    w.live = (uint32_t)(wg_groups >= (int64_t)waves * G ? waves : (wg_groups + G - 1) / G);
     w.lane = lane;
     w.n_tiles = n_tiles;
     w.tbl = tbl;
@@ -1117,7 +1119,8 @@ __global__ __launch_bounds__(kDecBlock) void fused_add_kernel(
     auto setup = [&](int64_t gbase, bool ahead) {
         #pragma unroll
         for (int j = 0; j < G; j++) {
-            // a wave past the last group repeats it with no lanes in range
+            // a wave past the last group repeats it with no lanes in range and
+            // empty streams: its loads read nothing
             const int64_t g = gbase + j < n_groups ? gbase + j : n_groups - 1;
             const int64_t k0 = g * kLanes;
             const int lanes = gbase + j < n_groups ? (K - k0 < kLanes ? (int)(K - k0) : kLanes) : 0;
@@ -1130,6 +1133,7 @@ __global__ __launch_bounds__(kDecBlock) void fused_add_kernel(
                 sa = noff_lane(0); ea = noff_lane(1); sb = noff_lane(2); eb = noff_lane(3);
             } else {
                 sa = a_off[g]; ea = a_off[g + 1]; sb = b_off[g]; eb = b_off[g + 1];
+                if (!lanes) { ea = sa; eb = sb; }
             }
             if constexpr (PACKED) {
                 plen[2 * j] = pk_fetch<NSEG>(a_comp, a_words, sa, ea, lane, first[2 * j]);
@@ -1493,7 +1497,8 @@ template <int SPS, int FIRST>
 __global__ __launch_bounds__(kDecBlock) void decode_kernel(
     const uint32_t* __restrict__ comp, int64_t words, const int64_t* __restrict__ off,
     const uint16_t* __restrict__ st, const v2u* __restrict__ sm,
-    const v2u* __restrict__ table, int64_t K, int64_t N, uint8_t* __restrict__ out) {
+    const v2u* __restrict__ table, int64_t K, int64_t N, int waves,
+    uint8_t* __restrict__ out) {
     constexpr uint32_t L = Alpha<SPS>::L;
     constexpr int C = kDecodeGroups;
     __shared__ DecodeSmem<SPS> dsmem;
@@ -1505,10 +1510,11 @@ __global__ __launch_bounds__(kDecBlock) void decode_kernel(
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
     const int64_t n_groups = (K + kLanes - 1) / kLanes;
-    const int64_t grid_groups = (int64_t)gridDim.x * kDecWaves * C;   // groups per round
-    int64_t g0 = ((int64_t)blockIdx.x * kDecWaves + wave) * C;
+    // the first `waves` waves decode, as in fused_add_kernel
+    const int64_t grid_groups = (int64_t)gridDim.x * waves * C;   // groups per round
+    int64_t g0 = wave < waves ? ((int64_t)blockIdx.x * waves + wave) * C : n_groups;
     const bool live = g0 < n_groups;   // wave-uniform
-    const int64_t wg_groups = n_groups - (int64_t)blockIdx.x * kDecWaves * C;
+    const int64_t wg_groups = n_groups - (int64_t)blockIdx.x * waves * C;
     // as in fused_add_kernel (a lazy start measured within noise here:
     // 2^30 elements at 1024 per lane -0.3%, at 128 per lane +0.6%)
     constexpr bool PACKED = FIRST < 0;
@@ -1520,7 +1526,7 @@ __global__ __launch_bounds__(kDecBlock) void decode_kernel(
                   "packed streams of up to 4 tiles");
     DecodeWave<SPS, FIRST> w;
     w.progress = &smem.progress;
-    w.live = (uint32_t)(wg_groups >= (int64_t)kDecWaves * C ? kDecWaves : (wg_groups + C - 1) / C);
+    w.live = (uint32_t)(wg_groups >= (int64_t)waves * C ? waves : (wg_groups + C - 1) / C);
     w.lane = lane;
     w.K = K;
     const int rag = (int)(N % kTile);
@@ -1541,13 +1547,15 @@ __global__ __launch_bounds__(kDecBlock) void decode_kernel(
     auto setup = [&](int64_t gbase) {
         bool full = true;
         w.out_tile = out + gbase * kLanes;
-        // a wave past the last group repeats it with no lanes in range
+        // a wave past the last group repeats it with no lanes in range and an
+        // empty stream
         int64_t os[C], oe[C];
         #pragma unroll
         for (int j = 0; j < C; j++) {
             const int64_t g = gbase + j < n_groups ? gbase + j : n_groups - 1;
             os[j] = off[g];
             oe[j] = off[g + 1];
+            if (gbase + j >= n_groups) oe[j] = os[j];
         }
         #pragma unroll
         for (int j = 0; j < C; j++) {
@@ -1633,7 +1641,6 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int kGemmChains = 2;                        // row groups per wave
 constexpr int kGemmGroupRows = 16;                    // rows of a group
-constexpr int kGemmGroupsPerBlock = kDecWaves * kGemmChains;
 constexpr int kGemmMaxBatch = 8;
 constexpr int kGemmMaxSegCols = 1024;                 // Nc limit
 constexpr int kGemmXStride = kGemmMaxSegCols + 16;    // bf16 per x stage row (32 bytes of pad)
@@ -1734,14 +1741,14 @@ struct GemmWave {
     }
 };
 
-// Grid: S * row_blocks workgroups; block (s, rb) decodes row groups
-// [32 rb, 32 rb + 32) of segment s (16 rows each).  R: rows, Rp: rows
+// Grid: S * row_blocks workgroups; block (s, rb) decodes the 2 `waves` row
+// groups from 2 `waves` rb on of segment s (16 rows each).  R: rows, Rp: rows
 // padded to 64, C: columns, Nc: columns per segment, NB: batch rows.
 template <int SPS>
 __global__ __launch_bounds__(kDecBlock) void gemm_fused_kernel(
     const uint32_t* __restrict__ comp, int64_t words, const int64_t* __restrict__ off,
     const uint16_t* __restrict__ st, const v2u* __restrict__ sm, const v2u* __restrict__ table,
-    int64_t Rp, int64_t C, int S, int Nc, int row_blocks, const uint16_t* __restrict__ x, int NB,
+    int64_t Rp, int64_t C, int S, int Nc, int row_blocks, int waves, const uint16_t* __restrict__ x, int NB,
     float* __restrict__ ws) {
     constexpr uint32_t L = Alpha<SPS>::L;
     constexpr int CH = kGemmChains;
@@ -1765,12 +1772,13 @@ __global__ __launch_bounds__(kDecBlock) void gemm_fused_kernel(
     table_fetch<L>(tr, table);
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
-    const int64_t rg0 = (int64_t)rb * kGemmGroupsPerBlock + (int64_t)wave * CH;
+    // the first `waves` waves decode, as in fused_add_kernel
+    const int64_t rg0 = wave < waves ? ((int64_t)rb * waves + wave) * CH : n_rg;
     const bool live = rg0 < n_rg;   // wave-uniform
-    const int64_t rg_left = n_rg - (int64_t)rb * kGemmGroupsPerBlock;
+    const int64_t rg_left = n_rg - (int64_t)rb * waves * CH;
     GemmWave<SPS> w;
     w.progress = &smem.dec.progress;
-    w.live = (uint32_t)(rg_left >= kGemmGroupsPerBlock ? kDecWaves : (rg_left + CH - 1) / CH);
+    w.live = (uint32_t)(rg_left >= (int64_t)waves * CH ? waves : (rg_left + CH - 1) / CH);
     w.lane = lane;
     w.q = lane >> 4;
     w.tbl = smem.dec.tbl;
@@ -1780,7 +1788,7 @@ __global__ __launch_bounds__(kDecBlock) void gemm_fused_kernel(
     const int rag = per_lane % kTile;                         // 0 or 8
     w.n_tiles = per_lane / kTile + (rag ? 1 : 0);
     last_tile_sched<SPS>(per_lane / SPS, w.n_tiles, w.last_segs, w.fin_pos);
-    w.sm_bytes = kLanes * 8u;
+    w.sm_bytes = live ? kLanes * 8u : 0u;
     Seg first[CH][kSlots];
     uint16_t st0[CH];
     // a wave with one row group left repeats it as its second chain and
@@ -1790,7 +1798,7 @@ __global__ __launch_bounds__(kDecBlock) void gemm_fused_kernel(
     for (int j = 0; j < CH; j++) {
         const int64_t g = (int64_t)s * n_rg + (rg0 + j < n_rg ? rg0 + j : n_rg - 1);
         os[j] = off[g];
-        oe[j] = off[g + 1];
+        oe[j] = live ? off[g + 1] : os[j];   // a wave without work reads nothing
     }
     #pragma unroll
     for (int j = 0; j < CH; j++) {
@@ -2324,8 +2332,22 @@ int sps_for(int32_t log2L) {
     return log2L == TANS_PAIR_LOG2L ? 2 : (log2L == TANS_NIBBLE_LOG2L ? 1 : 0);
 }
 
-template <int SPS>
 constexpr int kFusedGroups = 1;   // groups per wave in the fused kernel
+
+// Waves of each workgroup that decode, for `units` wave-sized pieces of work
+// (a wave takes one at a time) on `cus` workgroups, one per CU: as few as
+// keep the number of rounds.  The 16 waves of a full workgroup share the
+// CU's issue slots, and a wave with a SIMD to itself decodes a tile in 0.85
+// us instead of 1.9, so pieces that do not fill the chip are spread over all
+// CUs rather than packed into a few.  Fused add, 1024 per lane, 16 waves per
+// workgroup against this rule: 256 groups 91.6 -> 61.6 us, 1024 groups 93.8
+// -> 67 us, 2048 groups 96.4 -> 78 us, 5000 groups (two rounds of 10 waves
+// per CU, not 16 and then 16 on a fifth of the CUs) 210 -> 180 us.
+int spread_waves(int64_t units, int cus) {
+    const int64_t per_round = (int64_t)cus * kDecWaves;
+    const int64_t rounds = (units + per_round - 1) / per_round;
+    return (int)((units + cus * rounds - 1) / (cus * rounds));
+}
 
 int gemm_fused_launch(const void* comp, int64_t comp_bytes, const int64_t* offsets,
                       const uint16_t* states, const void* sm, const uint32_t* table,
@@ -2471,18 +2493,19 @@ int tans_fp8_vecadd_fused(const void* a_comp, int64_t a_comp_bytes, const int64_
         return fail(TANS_EINVAL, "vecadd_fused: misaligned buffer (comp and out 16, sm 8 bytes)");
     if (N / kTile > INT32_MAX) return fail(TANS_EINVAL, "vecadd_fused: N too large");
     const int64_t groups = (K + kLanes - 1) / kLanes;
-    const int64_t per_block = (int64_t)kDecWaves * (sps == 2 ? kFusedGroups<2> : kFusedGroups<1>);
     // one workgroup per CU at most; the waves loop over the groups
     const int cus = cu_count();
     if (cus <= 0) return fail(TANS_EHIP, "vecadd_fused: cannot query the device's CU count");
-    const int64_t blocks = std::min<int64_t>((groups + per_block - 1) / per_block, cus);
+    const int waves = spread_waves(groups, cus);
+    const int64_t blocks = std::min<int64_t>((groups + waves - 1) / waves, cus);
     const int n_tiles = (int)(N / kTile);
 #define TANS_LAUNCH_FUSED(S, FIRST)                                                               \
-    hipLaunchKernelGGL((fused_add_kernel<S, kFusedGroups<S>, FIRST>), dim3((unsigned)blocks),       \
+    hipLaunchKernelGGL((fused_add_kernel<S, kFusedGroups, FIRST>), dim3((unsigned)blocks),       \
                        dim3(kDecBlock), 0, (hipStream_t)stream, (const uint32_t*)a_comp,         \
                        a_comp_bytes / 4, a_offsets, a_states, (const v2u*)a_sm,                  \
                        (const uint32_t*)b_comp, b_comp_bytes / 4, b_offsets, b_states,           \
-                       (const v2u*)b_sm, (const v2u*)table, K, n_tiles, (v4u*)out)
+                       (const v2u*)b_sm, (const v2u*)table, K, n_tiles, waves,      \
+                       (v4u*)out)
     // streams that fit the ring are loaded whole at their start
     if (packed) {
         switch (n_tiles) {
@@ -2527,23 +2550,24 @@ int tans_decode(const void* comp, int64_t comp_bytes, const int64_t* offsets,
     // the stores address 4 rows of a tile with 32-bit offsets
     if (K > (int64_t(1) << 30)) return fail(TANS_EINVAL, "decode: more than 2^30 lanes");
     const int64_t groups = (K + kLanes - 1) / kLanes;
-    const int64_t per_block = (int64_t)kDecWaves * kDecodeGroups;
-    int64_t blocks = (groups + per_block - 1) / per_block;
+    // a wave takes two groups; those that do not fill the chip are spread
+    // over it (spread_waves)
+    const int cus = cu_count();
+    if (cus <= 0) return fail(TANS_EHIP, "decode: cannot query the device's CU count");
+    const int64_t pairs = (groups + kDecodeGroups - 1) / kDecodeGroups;
+    const int waves = spread_waves(pairs, cus);
+    int64_t blocks = (pairs + waves - 1) / waves;
     // Columns of one or two tiles: one workgroup per CU, the waves loop over
     // their group pairs (measured at 2^30 elements: 16 per column 923 ->
     // 616 us).  From 4 tiles on, one workgroup per 32 groups is as fast or
     // faster (64 per column: 472 vs 468 us; 256: 388 vs 400 us).
-    if ((N + kTile - 1) / kTile <= 2) {
-        const int cus = cu_count();
-        if (cus <= 0) return fail(TANS_EHIP, "decode: cannot query the device's CU count");
-        blocks = std::min<int64_t>(blocks, cus);
-    }
+    if ((N + kTile - 1) / kTile <= 2) blocks = std::min<int64_t>(blocks, cus);
     if (!grid_fits(blocks, kDecBlock)) return fail(TANS_EINVAL, "decode: K too large");
 #define TANS_LAUNCH_DECODE(S, FIRST)                                                              \
     hipLaunchKernelGGL((decode_kernel<S, FIRST>), dim3((unsigned)blocks),                        \
                        dim3(kDecBlock), 0, (hipStream_t)stream, (const uint32_t*)comp,           \
                        comp_bytes / 4, offsets, states, (const v2u*)sm, (const v2u*)table, K, N, \
-                       (uint8_t*)out)
+                       waves, (uint8_t*)out)
     // streams that fit the ring are loaded whole at their start
     const int64_t n_tiles = (N + kTile - 1) / kTile;
     if (packed) {
@@ -2620,7 +2644,14 @@ int gemm_fused_launch(const void* comp, int64_t comp_bytes, const int64_t* offse
     if (workspace_bytes < S * B * Rp * 4)
         return fail(TANS_EINVAL, "gemm_fused: workspace smaller than S * B * Rp * 4 bytes");
     const int64_t n_rg = Rp / kGemmGroupRows;
-    const int64_t row_blocks = (n_rg + kGemmGroupsPerBlock - 1) / kGemmGroupsPerBlock;
+    // a wave takes two row groups of a segment; those that do not fill the
+    // chip are spread over it (spread_waves, each segment's over its share of
+    // the CUs)
+    const int cus = cu_count();
+    if (cus <= 0) return fail(TANS_EHIP, "gemm_fused: cannot query the device's CU count");
+    const int64_t pairs = (n_rg + kGemmChains - 1) / kGemmChains;
+    const int waves = spread_waves(pairs, (int)std::max<int64_t>(1, cus / S));
+    const int64_t row_blocks = (pairs + waves - 1) / waves;
     const int64_t blocks = S * row_blocks;
     if (!grid_fits(blocks, kDecBlock) || !grid_fits(B * (Rp / kLanes), kFinWaves * kLanes))
         return fail(TANS_EINVAL, "gemm_fused: matrix too large");
@@ -2628,7 +2659,7 @@ int gemm_fused_launch(const void* comp, int64_t comp_bytes, const int64_t* offse
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kDecBlock), 0, st,
                            (const uint32_t*)comp, comp_bytes / 4, offsets, states, (const v2u*)sm,
-                           (const v2u*)table, Rp, C, (int)S, (int)Nc, (int)row_blocks,
+                           (const v2u*)table, Rp, C, (int)S, (int)Nc, (int)row_blocks, waves,
                            (const uint16_t*)x, (int)B, (float*)workspace);
     };
     if (sps == 2) launch(gemm_fused_kernel<2>); else launch(gemm_fused_kernel<1>);

@@ -1,0 +1,67 @@
+"""The launch rule that spreads groups over the CUs (spread_waves in
+kernels.hip): tensors of one group, of about one group per CU, around whole
+rounds of 16 waves per CU, and of two uneven rounds.  The outputs are bytes
+(fused add == raw add, decode == input) or, for the GEMM, the raw kernel's
+product to a bf16 step."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(msg):
+    print(msg, flush=True)
+
+
+@pytest.fixture(scope="module")
+def R():
+    import rans_vectoradd
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    return rans_vectoradd
+
+
+def _bytes(R, n, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return R.random_fp8_bytes(n, device="cuda", generator=g)
+
+
+# groups of 64 lanes against 256 CUs: one, fewer than CUs, one more than CUs
+# (two waves on one), a whole round of 16 and one group more or less, two
+# rounds of 10 waves; the lane count ragged in each
+@pytest.mark.parametrize("alphabet,N", [("pair", 16), ("pair", 48), ("pair", 80), ("nibble", 48)])
+@pytest.mark.parametrize("groups", [1, 100, 257, 4095, 4096, 4097, 5000])
+def test_groups_spread_over_cus(R, alphabet, N, groups):
+    from rans_vectoradd import tans_codec as T
+    K = groups * 64 - 3
+    _say(f"case: spread {groups} groups x {N} {alphabet}")
+    hist = torch.tensor(R.QWEN3_14B_FP8_EXP)
+    a, b = _bytes(R, K * N, groups).view(K, N), _bytes(R, K * N, groups + 1).view(K, N)
+    ea, eb = (T.encode_gpu(q, hist, alphabet=alphabet) for q in (a, b))
+    tbl = T.build_decode_table(ea[6].cpu().numpy(), ea[5].cpu().numpy()).cuda()
+    order = (0, 2, 1, 3, 4)
+    out = R.fp8_vecadd_fused_tans(*[ea[i] for i in order], *[eb[i] for i in order], tbl, N)
+    raw = R.fp8_vecadd_raw(a.view(-1), b.view(-1)).view(K, N // 16, 16).permute(1, 0, 2).reshape(-1)
+    assert torch.equal(out, raw)
+    dec = R.gpu_tans_decode(ea[0], ea[2], ea[1], ea[3], ea[4], ea[6], ea[5], N)
+    assert torch.equal(dec, a.t())
+
+
+# row groups of 16 rows per segment: one, an odd number, more than the CUs
+# of a segment's share hold in one round
+@pytest.mark.parametrize("rows,cols,segments", [(16, 512, 1), (1000, 2048, 8), (8272, 288, 1),
+                                                (140000, 64, 1)])
+def test_gemm_row_groups_spread_over_cus(R, rows, cols, segments):
+    from rans_vectoradd import tans_codec as T
+    _say(f"case: spread gemm {rows}x{cols} S={segments}")
+    w = _bytes(R, rows * cols, rows).view(rows, cols)
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    x = torch.randn(3, cols, generator=g, device="cuda").to(torch.bfloat16)
+    m = T.encode_matrix(w, torch.tensor(R.QWEN3_14B_FP8_EXP), segments=segments)
+    y = R.fp8_gemm_fused_tans(m, m.decode_table().cuda(), x, 2.0 ** -9).float()
+    y_raw = R.fp8_gemm_raw(w, x, 2.0 ** -9).float()
+    # both round an fp32 sum (whose order differs by at most cols * 2^-24 of
+    # the terms' magnitude) to bf16: one bf16 step (2^-7 relative) apart
+    mag = (x.abs().float() @ w.view(torch.float8_e4m3fn).float().nan_to_num(0).abs().t()) * 2.0 ** -9
+    same_nan = torch.isnan(y) == torch.isnan(y_raw)
+    ok = (y - y_raw).abs() <= 2.0 ** -7 * y_raw.abs() + cols * 2.0 ** -23 * mag
+    assert bool((same_nan & (ok | torch.isnan(y_raw))).all())
