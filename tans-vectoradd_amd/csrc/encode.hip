@@ -7,25 +7,27 @@
 // schedule ordering the words of a group's 64 lanes.
 //
 // Passes (all on the caller's stream):
-//   enc_backward_kernel  one thread per lane: step chunks [S][K] (u16:
-//                        value in bits 11:0, nb in bits 15:12), the
-//                        initial decoder state, and the number of stream
-//                        words the lane takes (a closed form of the refill
-//                        schedule in the lane's bit counts), summed per
-//                        group (padded to 4); for rows of whole 16-byte
-//                        tiles also the sign/mantissa tiles
+//   enc_walk_kernel      one wave per 64-lane group, one lane per row: the
+//                        backward walk, a 16-element tile at a time.  Each
+//                        tile of a lane becomes a 12-byte record (its
+//                        segments' bit counts and its first 64 bits; the
+//                        bits past 64 go to an overflow array, written
+//                        where a lane has any).  Also the sign/mantissa
+//                        tiles, the initial decoder states, and the number
+//                        of stream words the lane takes (a closed form of
+//                        the refill schedule in the lane's bit counts),
+//                        summed per group (padded to 4)
 //   enc_scan_kernel      exclusive prefix of the group counts -> offsets
-//   enc_place_kernel     one wave per group: replays the schedule while
-//                        each lane packs its chunks into words; a word's
-//                        place (offset + handed + rank) is fixed when the
-//                        lane takes it, and the word is stored there when
-//                        its last bit is packed
-//   enc_sm_kernel        sign/mantissa tiles when rows are not whole tiles
+//   enc_place_kernel     one wave per group: replays the schedule from the
+//                        records' counts while each lane joins its tiles'
+//                        bits into words; a word's place (offset + handed +
+//                        rank) is fixed when the lane takes it, and the
+//                        word is stored there when its last bit is known
 //
 // The packed layout of short streams (pair alphabet, at most 32 steps per
-// lane; schedule.h, tans_pack) reuses the backward pass, which then records
-// each lane's bit count and state in the workspace and sums the group's
-// bits into its stream size; enc_place_packed_kernel assembles each group's
+// lane; schedule.h, tans_pack) reuses the walk, which then records each
+// lane's bit count and state in the workspace and sums the group's bits
+// into its stream size; enc_place_packed_kernel assembles each group's
 // stream (header of lane-pair counts, bit area) in LDS and copies it out.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -44,6 +46,7 @@ constexpr int kLanes = 64;
 constexpr int kTile = 16;
 constexpr int64_t kTailWords = 256;
 constexpr int kEncBlock = 256;
+static_assert(kTailWords <= kEncBlock, "one workgroup zeroes the tail");
 
 int fail(int code, const std::string& msg) {
     tans_internal_set_error(msg.c_str());
@@ -66,124 +69,199 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
-// Workspace layout: chunks u16 [S][K], glen u32 [G].
-struct WsLayout {
-    int64_t chunks, glen, plen, pstate, total;
+// Workspace: the tile records u32 [tiles][K][3], their overflow words
+// u32 [tiles][overflow words][K], group lengths u32 [G], and for the packed
+// layout each lane's bit count and initial state (u16 [K] each).
+constexpr int kRecWords = 3;       // counts, bits 0-31, bits 32-63
+constexpr uint32_t kRecBits = 64;  // bits of a tile the record holds
+
+// A tile of 16 elements: 8 steps in four segments of 2 (pair alphabet) or 16
+// steps in six of 3, 3, 2, 3, 3, 2 (schedule.h).  A segment's bit count
+// (at most 24 or 30) takes 5 bits of the record's first word; a tile holds
+// at most 96 or 160 bits.
+template <int SPS>
+struct TileFmt {
+    static constexpr bool kTriple = SPS == 1;
+    static constexpr int kSteps = kTile / SPS;
+    static constexpr int kSegs = kTriple ? 6 : 4;
+    static constexpr int kOvf = kTriple ? 3 : 1;   // overflow words
+    static constexpr int seg_first(int q) { return kTriple ? 8 * (q / 3) + 3 * (q % 3) : 2 * q; }
+    static constexpr int seg_len(int q) { return kTriple ? (q % 3 == 2 ? 2 : 3) : 2; }
+    static_assert(kSteps == (int)tans_sched::tile_steps(kTriple), "the schedule's tile");
 };
 
-// chunks [S][K] u16, glen [G] u32, and for the packed layout each lane's
-// bit count and initial state (u16 [K] each)
-WsLayout ws_layout(int64_t K, int64_t S) {
+struct WsLayout {
+    int64_t rec, ovf, glen, plen, pstate, total;
+};
+
+WsLayout ws_layout(int64_t K, int64_t N, int32_t log2L) {
     const int64_t G = (K + kLanes - 1) / kLanes;
+    const int64_t tiles = (N + kTile - 1) / kTile;
+    const int64_t n_ovf = log2L == TANS_PAIR_LOG2L ? TileFmt<2>::kOvf : TileFmt<1>::kOvf;
     WsLayout l;
-    l.chunks = 0;
-    l.glen = align256(S * K * 2);
+    l.rec = 0;
+    l.ovf = align256(tiles * K * kRecWords * 4);
+    l.glen = l.ovf + align256(tiles * K * n_ovf * 4);
     l.plen = l.glen + align256(G * 4);
     l.pstate = l.plen + align256(K * 2);
     l.total = l.pstate + align256(K * 2);
     return l;
 }
 
-// Exponent symbol of step i of lane k: the pair e0 * 16 + e1 of bytes 2i,
-// 2i + 1, or the exponent of byte i.  Both bytes of a pair lie in the same
-// aligned dword (2i is even and so is the row start, N being even); the
-// tensor's last dword, which may end past its `total` bytes, is read bytewise.
-template <int SPS>
-__device__ __forceinline__ uint32_t symbol_at(const uint8_t* __restrict__ fp8, int64_t byte,
-                                              int64_t total) {
-    const int64_t a = byte & ~int64_t(3);
-    uint32_t w;
-    if (a + 4 <= total) {
-        w = *reinterpret_cast<const uint32_t*>(fp8 + a);
-    } else {
-        w = 0;
-        for (int64_t j = a; j < total; j++) w |= (uint32_t)fp8[j] << (8 * (j - a));
-    }
-    const uint32_t sh = (uint32_t)(byte & 3) * 8u;
-    if constexpr (SPS == 2) {
-        return (((w >> (sh + 3)) & 0xFu) << 4) | ((w >> (sh + 11)) & 0xFu);
-    } else {
-        return (w >> (sh + 3)) & 0xFu;
-    }
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef uint32_t v3u __attribute__((ext_vector_type(3)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+typedef uint64_t Mask;   // a lane mask of the wave
+constexpr int kNT = 2;   // cache policy: non-temporal
+
+// A buffer resource of `bytes` from a wave-uniform base: loads past it
+// return zero, stores past it are dropped.
+__device__ __forceinline__ Rsrc rsrc(const void* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
+                                             0x00020000);
 }
 
 // Per-symbol step constants (the FSE formulation of the same construction).
 // For x in [L, 2L) the step emits the nb low bits of x with x >> nb in
-// [f, 2f): nb = (x + dnb) >> 16 with maxb = log2L - floor(log2(f - 1))
+// [f, 2f): nb = (x + x.dnb) >> 16 with maxb = log2L - floor(log2(f - 1))
 // (log2L for f = 1) and dnb = (maxb << 16) - (f << maxb); then x = next[idx]
-// with idx = start + (x >> nb) - f = (x >> nb) + dfind.  This gives the same
-// nb as floor(log2 x) - floor(log2 f), less one when x >> nb < f, for every
-// f in [1, L] and x in [L, 2L).  A symbol of frequency 0 is encoded as if
-// f = 1 (every index stays in range) and flagged in bit 31 of dnb.
+// with idx = start + (x >> nb) - f, kept as a byte offset: y = 2 (start - f).
+// This gives the same nb as floor(log2 x) - floor(log2 f), less one when
+// x >> nb < f, for every f in [1, L] and x in [L, 2L), and idx is in [start,
+// start + f).  f and start are clamped so that it is inside the table
+// whatever enc_tab holds.  A symbol of frequency 0 takes nb = log2L plus
+// kBadNb, a multiple of 32: shifts and field widths see log2L (so x >> nb is
+// 1 and idx = start), and the tile's bit count shows it.
+constexpr uint32_t kBadNb = 1024;
+
 __device__ __forceinline__ uint2 enc_consts(uint32_t e, int log2L) {
+    const uint32_t L = 1u << log2L;
     uint32_t f = e & 0xFFFFu;
-    const uint32_t start = e >> 16;
-    const uint32_t bad = f == 0 ? 1u : 0u;
-    if (f == 0) f = 1;
+    uint32_t start = e >> 16;
+    f = f > L ? L : f;
+    const bool bad = f == 0;
+    if (bad) f = 1;
+    start = start > L - f ? L - f : start;
     const uint32_t maxb = f == 1 ? (uint32_t)log2L
                                  : (uint32_t)log2L - (31u - (uint32_t)__builtin_clz(f - 1u));
-    const uint32_t dnb = (maxb << 16) - (f << maxb);
-    return uint2{dnb | (bad << 31), start - f};
+    const uint32_t dnb = bad ? ((uint32_t)log2L + kBadNb) << 16 : (maxb << 16) - (f << maxb);
+    return uint2{dnb, 2u * (start - f)};
 }
 
-// One backward encode step of symbol s: emit the chunk of step i (value in
-// bits 11:0, nb in bits 15:12), then x = L + the slot of s's rank-th
-// occurrence.  bad collects the flags of the symbols seen.
-// The chunk goes to row i of chunks [S][K] through a buffer resource on that
-// row (a scalar base; the lane's offset k * 2 is fixed), so the store costs
-// no per-step address arithmetic.
-__device__ __forceinline__ void enc_step(uint32_t s, const uint2* tab, const uint16_t* nx,
-                                         uint32_t L, uint32_t& x, uint32_t& bad, uint32_t& bits,
-                                         uint16_t* __restrict__ chunks, int64_t i, int64_t K,
-                                         uint32_t koff) {
-    const uint2 e = tab[s];
-    bad |= e.x;
-    const uint32_t nb = __builtin_amdgcn_ubfe(x + e.x, 16u, 5u);
-    bits += nb;
-    const uint32_t ch = __builtin_amdgcn_ubfe(x, 0u, nb) | (nb << 12);
-    __builtin_amdgcn_raw_buffer_store_b16((uint16_t)ch,
-                                          __builtin_amdgcn_make_buffer_rsrc(chunks + i * K, (short)0,
-                                                                            (int)(K * 2),
-                                                                            0x00020000),
-                                          koff, 0, 0);
-    uint32_t idx = (x >> nb) + e.y;
-    idx = idx < L ? idx : L - 1u;
-    x = nx[idx];
+// LDS tables of the walk.  tab is indexed by the symbol's bits as they lie
+// in the FP8 bytes: entry e (nibble) or e1 * 16 + e0 (pair), so an entry's
+// byte offset is a shift and a mask away (sym_offsets).  nx holds the next
+// states, each brought into [L, 2L).
+template <int SPS>
+struct EncTab {
+    uint2 tab[SPS == 2 ? 256 : 16];
+    uint16_t nx[1 << TANS_PAIR_LOG2L];
+};
+
+template <int SPS>
+__device__ __forceinline__ void load_tables(EncTab<SPS>& t, const uint32_t* __restrict__ enc_tab,
+                                            const uint16_t* __restrict__ next, int log2L) {
+    constexpr int NSYM = SPS == 2 ? 256 : 16;
+    const uint32_t L = 1u << log2L;
+    for (int i = threadIdx.x; i < NSYM; i += blockDim.x)
+        t.tab[SPS == 2 ? ((i & 15) << 4 | i >> 4) : i] = enc_consts(enc_tab[i], log2L);
+    for (uint32_t i = threadIdx.x; i < L; i += blockDim.x)
+        t.nx[i] = (uint16_t)(L + (next[i] & (L - 1u)));
 }
 
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-typedef uint64_t Mask;   // a lane mask of the wave
-constexpr int kEncBlockChunks = 8;   // 16-byte chunks per 128-byte block of a row
-
-// Symbol of step q of a 16-byte chunk: bytes 2q, 2q + 1 (pair) or byte q.
+// Byte offset in tab of step Q's symbol of a tile (16 FP8 bytes in c): the
+// exponents of bytes 2Q, 2Q + 1 (bits 6:3 of each) as e1 << 7 | e0 << 3, or
+// of byte Q as e << 3.
 template <int SPS, int Q>
-__device__ __forceinline__ uint32_t chunk_symbol(const v4u& c) {
+__device__ __forceinline__ uint32_t sym_offset(const v4u& c) {
     const uint32_t w = c[Q * SPS / 4];
     constexpr uint32_t sh = (uint32_t)((Q * SPS) % 4) * 8u;
     if constexpr (SPS == 2) {
-        return (((w >> (sh + 3)) & 0xFu) << 4) | ((w >> (sh + 11)) & 0xFu);
+        const uint32_t u = w & 0x78787878u;
+        return ((u | u >> 4) >> sh) & 0x7F8u;   // (u is shared by the word's two symbols)
     } else {
-        return (w >> (sh + 3)) & 0xFu;
+        return (w >> sh) & 0x78u;
     }
 }
 
 // The two sign/mantissa words of a 16-byte tile: sign and mantissa bits
 // (mask 0x87 of each byte) of bytes 0-3 in place and of bytes 4-7 rotated
 // by 4 bits into the exponent positions, the same for bytes 8-15.
-__device__ __forceinline__ void sm_words(const uint32_t (&b)[4], uint32_t& w0, uint32_t& w1) {
+__device__ __forceinline__ v2u sm_words(const v4u& b) {
     const uint32_t m = 0x87878787u;
-    w0 = (b[0] & m) | __builtin_amdgcn_alignbit(b[1] & m, b[1] & m, 28u);
-    w1 = (b[2] & m) | __builtin_amdgcn_alignbit(b[3] & m, b[3] & m, 28u);
+    return v2u{(b.x & m) | __builtin_amdgcn_alignbit(b.y & m, b.y & m, 28u),
+               (b.z & m) | __builtin_amdgcn_alignbit(b.w & m, b.w & m, 28u)};
 }
 
-// Chunks top - 1, top - 2, ... of a row into b[0], b[1], ... (zero below 0).
-__device__ __forceinline__ void load_block(v4u (&b)[kEncBlockChunks], const v4u* rp,
-                                           int64_t top) {
-    #pragma unroll
-    for (int c = 0; c < kEncBlockChunks; c++) {
-        const int64_t j = top - 1 - c;
-        b[c] = j >= 0 ? rp[j] : v4u{0u, 0u, 0u, 0u};   // wave-uniform condition
+// The bits of one tile of a lane, in decode order (LSB first).
+template <int SPS>
+struct TileBits {
+    uint32_t cnt[TileFmt<SPS>::kSegs];   // bits of each segment
+    uint32_t total;                      // their sum
+    uint64_t lo;                         // bits 0 .. 63
+    uint32_t ovf[TileFmt<SPS>::kOvf];    // the bits past 64 (only when total > 64)
+};
+
+// Walk one tile backwards from state x (steps steps - 1 .. 0; GUARD false: all
+// kSteps).  A step emits the nb low bits of x above the bits of the steps
+// before it; the segments are then joined, and the bits past 64 are formed
+// only when a lane of the wave has some.
+template <int SPS, bool GUARD>
+__device__ __forceinline__ void enc_tile(const v4u& c, int steps, const EncTab<SPS>& t,
+                                         uint32_t& x, TileBits<SPS>& o) {
+    using F = TileFmt<SPS>;
+    uint32_t val[F::kSegs];
+    static_for<0, F::kSegs>([&](auto I) {
+        constexpr int s = F::kSegs - 1 - decltype(I)::value;
+        val[s] = 0u;
+        o.cnt[s] = 0u;
+        static_for<0, F::seg_len(s)>([&](auto J) {
+            constexpr int q = F::seg_first(s) + F::seg_len(s) - 1 - decltype(J)::value;
+            if (GUARD && q >= steps) return;   // wave-uniform
+            const uint2 e = *reinterpret_cast<const uint2*>(
+                reinterpret_cast<const char*>(t.tab) + sym_offset<SPS, q>(c));
+            const uint32_t nb = (x + e.x) >> 16;
+            val[s] = (val[s] << (nb & 31u)) | __builtin_amdgcn_ubfe(x, 0u, nb);
+            o.cnt[s] += nb;
+            x = *reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(t.nx) +
+                                                   (((x >> (nb & 31u)) << 1) + e.y));
+        });
+    });
+    if constexpr (!F::kTriple) {
+        const uint32_t n01 = o.cnt[0] + o.cnt[1];
+        o.total = n01 + o.cnt[2] + o.cnt[3];
+        const uint64_t b01 = (uint64_t)val[1] << (o.cnt[0] & 63u) | val[0];
+        const uint64_t b23 = (uint64_t)val[3] << (o.cnt[2] & 63u) | val[2];
+        o.lo = b23 << (n01 & 63u) | b01;   // n01 <= 48
+        o.ovf[0] = 0u;
+        if (__any(o.total > kRecBits))     // (n01 > 0 in the lanes that keep it)
+            o.ovf[0] = o.total > kRecBits ? (uint32_t)(b23 >> ((64u - n01) & 63u)) : 0u;
+    } else {
+        // two halves of three segments (at most 30 + 30 + 20 bits)
+        uint64_t lo[2];
+        uint32_t hi[2], n[2];
+        #pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint32_t n01 = o.cnt[3 * h] + o.cnt[3 * h + 1];
+            n[h] = n01 + o.cnt[3 * h + 2];
+            lo[h] = (uint64_t)val[3 * h + 2] << (n01 & 63u) |
+                    (uint64_t)val[3 * h + 1] << (o.cnt[3 * h] & 63u) | val[3 * h];
+            // bits 64 .. 79 (n01 > 44 where there are any)
+            hi[h] = n[h] > 64u ? val[3 * h + 2] >> ((64u - n01) & 31u) : 0u;
+        }
+        o.total = n[0] + n[1];
+        o.lo = n[0] < 64u ? lo[1] << (n[0] & 63u) | lo[0] : lo[0];
+        o.ovf[0] = o.ovf[1] = o.ovf[2] = 0u;
+        if (__any(o.total > kRecBits)) {
+            const unsigned __int128 h1 = (unsigned __int128)hi[1] << 64 | lo[1];
+            unsigned __int128 up = 0;
+            if (o.total > kRecBits)
+                up = n[0] >= 64u ? h1 << ((n[0] - 64u) & 63u) | hi[0] : h1 >> ((64u - n[0]) & 127u);
+            o.ovf[0] = (uint32_t)up;
+            o.ovf[1] = (uint32_t)(up >> 32);
+            o.ovf[2] = (uint32_t)(up >> 64);
+        }
     }
 }
 
@@ -213,134 +291,248 @@ __device__ __forceinline__ uint32_t lane_words(int64_t S, bool triple, uint32_t 
     return t + (32u * t - c2 < (uint32_t)tans_sched::final_below(S, triple) ? 1u : 0u);
 }
 
-// One thread per lane walks its row backwards.  When rows are 16-byte
-// aligned (N % 16 == 0) a lane loads its row 128 bytes at a time and the
-// next 128 bytes while it encodes the current ones: a step then waits on
-// LDS only, not on a global load, and each line of the row is fetched in
-// one go (the lanes' rows are N bytes apart, so a line read piecewise over
-// many steps could leave the cache in between).  A wave is one 64-lane
-// group (blocks hold four); its lanes' word counts are summed into
-// glen[group], padded to a multiple of 4.  PACKED (the packed layout):
-// plen[k] gets the lane's bits (12 for the state + its steps' nb), and
-// glen[group] the words of the group's stream (header, bits, padding to 16
-// bytes); `states` is then the workspace's state array.
-template <int SPS, bool PACKED = false>
-__global__ __launch_bounds__(kEncBlock) void enc_backward_kernel(
-    const uint8_t* __restrict__ fp8, int64_t K, int64_t N, const uint32_t* __restrict__ enc_tab,
-    const uint16_t* __restrict__ next, int log2L, uint16_t* __restrict__ chunks,
-    uint16_t* __restrict__ states, uint32_t* __restrict__ glen, uint32_t* __restrict__ sm,
-    int* __restrict__ status, uint16_t* __restrict__ plen) {
-    static_assert(kEncBlock % kLanes == 0, "blocks hold whole groups");
-    constexpr int NSYM = SPS == 2 ? 256 : 16;
-    __shared__ uint2 tab[NSYM];
-    __shared__ uint16_t nx[1 << TANS_PAIR_LOG2L];
-    const uint32_t L = 1u << log2L;
-    for (int i = threadIdx.x; i < NSYM; i += blockDim.x) tab[i] = enc_consts(enc_tab[i], log2L);
-    for (uint32_t i = threadIdx.x; i < L; i += blockDim.x) nx[i] = next[i];
-    __syncthreads();
-    const int64_t k = (int64_t)blockIdx.x * kEncBlock + threadIdx.x;
-    if (k - (threadIdx.x & (kLanes - 1)) >= K) return;   // the whole group is out of range
-    const int64_t S = N / SPS;
-    constexpr bool kTriple = SPS == 1;   // 2^11-state tables: 3-3-2 segments
-    uint32_t words = 0;
-    if (k < K) {
-        const int64_t row = k * N;
-        uint32_t x = L;
-        uint32_t bad = 0;    // bit 31: a symbol of frequency 0
-        uint32_t bits = 0;          // the lane's stream bits
-        uint32_t b1 = 0, b2 = 0;    // bits of the last segment, of the last two (lane_words)
-        const uint32_t koff = (uint32_t)k * 2u;   // K <= INT32_MAX (checked by the launcher)
-        if (N % 16 == 0) {   // kernel-uniform
-            // S is a multiple of 8 (pair) or 16 (nibble), so the last two
-            // segments (steps S - 4 .. or S - 5 ..) are the walk's first
-            // steps, all in the row's last chunk
-            constexpr int kQ = 16 / SPS;   // steps per chunk
-            constexpr int kB2 = kTriple ? kQ - 5 : kQ - 4;   // first step of the last two
-            const v4u* rp = reinterpret_cast<const v4u*>(fp8 + row);
-            const int64_t nch = N / 16;
-            v4u cur[kEncBlockChunks], nxt[kEncBlockChunks];
-            load_block(cur, rp, nch);
-            for (int64_t hi = nch; hi > 0; hi -= kEncBlockChunks) {
-                load_block(nxt, rp, hi - kEncBlockChunks);
-                #pragma unroll
-                for (int c = 0; c < kEncBlockChunks; c++) {
-                    const int64_t j = hi - 1 - c;
-                    if (j < 0) break;   // wave-uniform
-                    static_for<0, kQ>([&](auto Q) {
-                        constexpr int q = kQ - 1 - decltype(Q)::value;
-                        enc_step(chunk_symbol<SPS, q>(cur[c]), tab, nx, L, x, bad, bits, chunks,
-                                 j * kQ + q, K, koff);
-                        if constexpr (q == kQ - 2) {
-                            if (j == nch - 1) b1 = bits;   // wave-uniform
-                        } else if constexpr (q == kB2) {
-                            if (j == nch - 1) b2 = bits;
-                        }
-                    });
-                    // the chunk is tile j: its sign/mantissa words (a wave's
-                    // stores cover 512 contiguous bytes)
-                    const uint32_t tb[4] = {cur[c].x, cur[c].y, cur[c].z, cur[c].w};
-                    uint32_t w0, w1;
-                    sm_words(tb, w0, w1);
-                    *reinterpret_cast<uint2*>(sm + (j * K + k) * 2) = uint2{w0, w1};
-                }
-                #pragma unroll
-                for (int c = 0; c < kEncBlockChunks; c++) cur[c] = nxt[c];
-            }
+// The rows of an FP8 tensor [K, N].  Rows of whole 16-byte tiles start
+// 16-byte aligned; others start on any even byte, and their tiles are
+// unaligned 16-byte loads (gfx950 takes any alignment).
+typedef v4u v4u_any __attribute__((aligned(1)));
+
+struct RowSrc {
+    const uint8_t* fp8;
+    int64_t K, N;
+
+    const uint8_t* row;   // the lane's row
+    int64_t left;         // bytes from it to the tensor's end
+
+    __device__ __forceinline__ void start(int64_t k) {
+        row = fp8 + k * N;
+        left = K * N - k * N;
+    }
+    __device__ __forceinline__ v4u tile(int64_t t) const {
+        return *reinterpret_cast<const v4u_any*>(row + t * kTile);
+    }
+    // the last tile's n < 16 bytes (zeros after them): one load where the
+    // tensor goes on past it, else byte by byte
+    __device__ __forceinline__ v4u last(int64_t t, int n) const {
+        v4u v = {0u, 0u, 0u, 0u};
+        const uint8_t* p = row + t * kTile;
+        if (left >= t * kTile + kTile) {
+            v = *reinterpret_cast<const v4u_any*>(p);
         } else {
-            // first steps of the last segment and of the one before it
-            const int64_t n_seg = tans_sched::segments(S, kTriple);
-            const int64_t last = tans_sched::seg_start(n_seg - 1, kTriple);
-            const int64_t last2 = n_seg >= 2 ? tans_sched::seg_start(n_seg - 2, kTriple) : -1;
-            for (int64_t i = S - 1; i >= 0; i--) {
-                enc_step(symbol_at<SPS>(fp8, row + i * SPS, K * N), tab, nx, L, x, bad, bits,
-                         chunks, i, K, koff);
-                if (i == last) b1 = bits;
-                if (i == last2) b2 = bits;
-            }
+            #pragma unroll
+            for (int i = 0; i < kTile; i++)
+                if (i < n) v[i / 4] |= (uint32_t)p[i] << (8 * (i % 4));
         }
-        states[k] = (uint16_t)x;
-        if (bad >> 31) *status = TANS_ESYMBOL;   // vector store: any failing lane may write it
+        #pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const int b = n - 4 * w;   // bytes of this word (wave-uniform)
+            v[w] &= b >= 4 ? 0xFFFFFFFFu : b <= 0 ? 0u : (1u << (8 * b)) - 1u;
+        }
+        return v;
+    }
+};
+
+// One wave per 64-lane group; each lane walks its row backwards, a tile at a
+// time, and stores per tile its 12-byte record (768 contiguous bytes per
+// wave) and its sign/mantissa words (512).  A lane loads its row 128 bytes
+// (8 tiles) at a time and the next 128 while it encodes the current ones: a
+// step then waits on LDS only, not on a global load, and each line of the
+// row is fetched in one go (the lanes' rows are N bytes apart, so a line
+// read piecewise over many steps could leave the cache in between).
+//
+// What bounds it: memory.  2^29 elements at 1024 per lane take 252 us (284 us
+// with 2-byte chunks stored per step, 0.54 GB of them) for 1.21 GB read and
+// written; the same accesses without the walk take 230 us, the walk without
+// its loads and stores 97 us.  Conflict-free table reads change nothing.  The
+// sign/mantissa stores are non-temporal: nothing here reads them again, and
+// the place pass, which finds more of the records still cached, takes 142
+// instead of 149 us.  Non-temporal records: this kernel 268, the place pass
+// 131 us.
+//
+// The lanes' word counts are summed into glen[group], padded to a multiple
+// of 4.  PACKED (the packed layout): plen[k] gets the lane's bits (12 for
+// the state + its steps' nb), and glen[group] the words of the group's
+// stream (header, bits, padding to 16 bytes); `states` is then the
+// workspace's state array.
+constexpr int kBlockTiles = 8;   // tiles per 128-byte block of a row
+
+template <int SPS, bool PACKED, class Src>
+__global__ __launch_bounds__(kEncBlock) void enc_walk_kernel(
+    Src src, int64_t K, int64_t N, const uint32_t* __restrict__ enc_tab,
+    const uint16_t* __restrict__ next, int log2L, uint32_t* __restrict__ rec,
+    uint32_t* __restrict__ ovf, uint16_t* __restrict__ states, uint32_t* __restrict__ glen,
+    uint32_t* __restrict__ sm, int* __restrict__ status, uint16_t* __restrict__ plen) {
+    using F = TileFmt<SPS>;
+    static_assert(kEncBlock % kLanes == 0, "blocks hold whole groups");
+    __shared__ EncTab<SPS> tab;
+    load_tables<SPS>(tab, enc_tab, next, log2L);
+    __syncthreads();
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int64_t g = (int64_t)blockIdx.x * (kEncBlock / kLanes) +
+                      __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int64_t k0 = g * kLanes;
+    if (k0 >= K) return;
+    const uint32_t lanes = (uint32_t)(K - k0 < kLanes ? K - k0 : kLanes);
+    const bool active = (uint32_t)lane < lanes;
+    src.start(active ? k0 + lane : K - 1);   // lanes out of range repeat the last row, unstored
+    const int64_t S = N / SPS;
+    const int nt = (int)((N + kTile - 1) / kTile);   // S <= 2^24 (checked by the launcher)
+    const int rag = (int)(N % kTile);
+    const int last_steps = (rag ? rag : kTile) / SPS;
+    const int last_segs = (int)tans_sched::last_tile_segments(S, F::kTriple);
+    uint32_t x = 1u << log2L;
+    uint32_t bits = 0;          // the lane's stream bits
+    uint32_t bad = 0;           // kBadNb or more: a symbol of frequency 0
+    uint32_t b1 = 0, b2 = 0;    // bits of the last segment, of the last two (lane_words)
+    // the group's part of tile t's records, overflow words and sm rows (wave-uniform)
+    const char* rec_t = reinterpret_cast<const char*>(rec) +
+                        ((int64_t)(nt - 1) * K + k0) * (kRecWords * 4);
+    const char* ovf_t = reinterpret_cast<const char*>(ovf) +
+                        ((int64_t)(nt - 1) * F::kOvf * K + k0) * 4;
+    const char* sm_t = reinterpret_cast<const char*>(sm) + ((int64_t)(nt - 1) * K + k0) * 8;
+    // tiles 8 b .. 8 b + 7 of the row
+    auto load = [&](v4u (&buf)[kBlockTiles], int b) {
+        #pragma unroll
+        for (int c = kBlockTiles - 1; c >= 0; c--) buf[c] = src.tile(b * kBlockTiles + c);
+    };
+    // tile t; FIRST: it may be the row's last (the walk's first)
+    auto tile = [&](const v4u& c, int t, auto FIRST) {
+        constexpr bool kFirst = decltype(FIRST)::value;
+        TileBits<SPS> o;
+        enc_tile<SPS, kFirst>(c, kFirst && t == nt - 1 ? last_steps : F::kSteps, tab, x, o);
+        uint32_t counts = o.cnt[0];
+        #pragma unroll
+        for (int s = 1; s < F::kSegs; s++) counts |= o.cnt[s] << (5 * s);
+        const v3u r = {counts, (uint32_t)o.lo, (uint32_t)(o.lo >> 32)};
+        __builtin_amdgcn_raw_buffer_store_b96(r, rsrc(rec_t, lanes * (kRecWords * 4)),
+                                              (uint32_t)lane * (kRecWords * 4), 0, 0);
+        if (__any(o.total > kRecBits)) {
+            #pragma unroll
+            for (int i = 0; i < F::kOvf; i++)
+                if (o.total > kRecBits + 32u * i)
+                    __builtin_amdgcn_raw_buffer_store_b32(o.ovf[i],
+                                                          rsrc(ovf_t + (int64_t)i * K * 4, lanes * 4),
+                                                          (uint32_t)lane * 4, 0, 0);
+        }
+        __builtin_amdgcn_raw_buffer_store_b64(sm_words(c), rsrc(sm_t, lanes * 8),
+                                              (uint32_t)lane * 8, 0, kNT);
+        rec_t -= K * (kRecWords * 4);
+        ovf_t -= K * (F::kOvf * 4);
+        sm_t -= K * 8;
+        bits += o.total;
+        bad |= o.total;
+        if (kFirst && t == nt - 1) {
+            #pragma unroll
+            for (int s = 0; s < F::kSegs; s++) {
+                if (s == last_segs - 1) b1 = o.cnt[s];
+                if (s == last_segs - 2) b2 = o.cnt[s];
+            }
+            b2 += b1;
+        } else if (t == nt - 2 && last_segs == 1) {
+            b2 += o.cnt[F::kSegs - 1];
+        }
+    };
+    v4u cur[kBlockTiles], nxt[kBlockTiles];
+    int b = (nt - 1) / kBlockTiles;
+    const int full = nt - (rag ? 1 : 0);   // whole tiles
+    #pragma unroll
+    for (int c = kBlockTiles - 1; c >= 0; c--)
+        if (b * kBlockTiles + c < full) cur[c] = src.tile(b * kBlockTiles + c);   // wave-uniform
+    v4u ragged = {0u, 0u, 0u, 0u};
+    if (rag) ragged = src.last(nt - 1, rag);
+    if (b > 0) load(nxt, b - 1);
+    #pragma unroll
+    for (int c = kBlockTiles - 1; c >= 0; c--) {
+        const int t = b * kBlockTiles + c;
+        if (t < nt) tile(rag && t == nt - 1 ? ragged : cur[c], t, std::true_type{});
+    }
+    for (b--; b >= 0; b--) {
+        #pragma unroll
+        for (int c = 0; c < kBlockTiles; c++) cur[c] = nxt[c];
+        if (b > 0) load(nxt, b - 1);
+        #pragma unroll
+        for (int c = kBlockTiles - 1; c >= 0; c--)
+            tile(cur[c], b * kBlockTiles + c, std::false_type{});
+    }
+    uint32_t words = 0;
+    if (active) {
+        states[k0 + lane] = (uint16_t)x;
+        if (bad >= kBadNb) {
+            *status = TANS_ESYMBOL;   // vector store: any failing lane may write it
+            bits = b1 = b2 = 0;       // its bit counts mean nothing
+        }
         if constexpr (PACKED) {
             words = (uint32_t)tans_pack::kStateBits + bits;   // the lane's bits
-            plen[k] = (uint16_t)words;
+            plen[k0 + lane] = (uint16_t)words;
         } else {
-            words = lane_words(S, kTriple, bits, b1, b2);
+            words = lane_words(S, F::kTriple, bits, b1, b2);
         }
     }
     #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) words += __shfl_xor(words, m, kLanes);
-    if ((threadIdx.x & (kLanes - 1)) == 0) {
+    if (lane == 0) {
         if constexpr (PACKED)   // header + bits, padded to 16 bytes
-            glen[k / kLanes] = ((uint32_t)tans_pack::hdr_total(S) + (words + 7u) / 8u + 15u) / 16u * 4u;
+            glen[g] = ((uint32_t)tans_pack::hdr_total(S) + (words + 7u) / 8u + 15u) / 16u * 4u;
         else
-            glen[k / kLanes] = (words + 3u) & ~3u;
+            glen[g] = (words + 3u) & ~3u;
     }
 }
 
-// offsets[g] = sum of glen[0..g), offsets[G] = total; one workgroup: each
-// thread sums a contiguous run, then a Hillis-Steele scan over the threads.
-__global__ __launch_bounds__(1024) void enc_scan_kernel(const uint32_t* __restrict__ glen,
-                                                        int64_t G, int64_t* __restrict__ offsets) {
-    __shared__ int64_t part[1024];
-    const int tid = threadIdx.x;
-    const int64_t per = (G + 1023) / 1024;
-    const int64_t b = tid * per;
-    int64_t sum = 0;
-    for (int64_t i = b; i < b + per && i < G; i++) sum += glen[i];
-    part[tid] = sum;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        const int64_t v = tid >= off ? part[tid - off] : 0;
+// offsets[g] = sum of glen[0..g), offsets[G] = total.  One workgroup takes
+// kScanItems groups per thread and round; a round's loads are issued before
+// the previous round is summed.  A thread's items are a contiguous run, the
+// waves scan their threads' sums by shuffles and the 16 wave totals meet in
+// LDS.  (8192 groups: 12.9 us with one contiguous run per thread, read word
+// by word, 8.9 us now.)
+constexpr int kScanBlock = 1024;
+constexpr int kScanItems = 8;
+
+__global__ __launch_bounds__(kScanBlock) void enc_scan_kernel(const uint32_t* __restrict__ glen,
+                                                              int64_t G,
+                                                              int64_t* __restrict__ offsets) {
+    constexpr int kWaves = kScanBlock / kLanes;
+    constexpr int64_t kRound = (int64_t)kScanBlock * kScanItems;
+    __shared__ int64_t wave_sum[2][kWaves];
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int wave = threadIdx.x / kLanes;
+    auto load = [&](int64_t base, uint32_t (&v)[kScanItems]) {
+        const int64_t i0 = base + (int64_t)threadIdx.x * kScanItems;
+        #pragma unroll
+        for (int i = 0; i < kScanItems; i++) v[i] = i0 + i < G ? glen[i0 + i] : 0u;
+    };
+    uint32_t v[kScanItems], n[kScanItems];
+    load(0, v);
+    int64_t carry = 0;
+    int buf = 0;
+    for (int64_t base = 0; base < G; base += kRound) {
+        load(base + kRound, n);
+        int64_t sum = 0;
+        #pragma unroll
+        for (int i = 0; i < kScanItems; i++) sum += v[i];
+        int64_t inc = sum;   // inclusive scan over the wave
+        #pragma unroll
+        for (int d = 1; d < kLanes; d <<= 1) {
+            const int64_t y = __shfl_up(inc, d, kLanes);
+            if (lane >= d) inc += y;
+        }
+        if (lane == kLanes - 1) wave_sum[buf][wave] = inc;
         __syncthreads();
-        part[tid] += v;
-        __syncthreads();
+        int64_t run = carry + inc - sum;
+        #pragma unroll
+        for (int w = 0; w < kWaves; w++) {
+            const int64_t s = wave_sum[buf][w];
+            if (w < wave) run += s;
+            carry += s;
+        }
+        const int64_t i0 = base + (int64_t)threadIdx.x * kScanItems;
+        #pragma unroll
+        for (int i = 0; i < kScanItems; i++) {
+            if (i0 + i < G) offsets[i0 + i] = run;
+            run += v[i];
+            v[i] = n[i];
+        }
+        buf ^= 1;   // the next round writes the other buffer: one barrier per round
     }
-    if (tid == 1023) offsets[G] = part[1023];
-    int64_t run = part[tid] - sum;
-    for (int64_t i = b; i < b + per && i < G; i++) {
-        offsets[i] = run;
-        run += glen[i];
-    }
+    if (threadIdx.x == 0) offsets[G] = carry;
 }
 
 // Zero n words (a kernel rather than hipMemsetAsync, so a caller may
@@ -350,146 +542,226 @@ __global__ __launch_bounds__(kEncBlock) void zero_words_kernel(uint32_t* __restr
     if (i < n) p[i] = 0u;
 }
 
-// One wave per group replays the refill schedule while each lane packs its
-// chunks into 32-bit words, LSB first.  A word's place in the stream is
-// fixed when the lane takes it: the first two words of every lane are the
-// first 2 x lanes words (first words in lane order, then the second), and
-// a word taken after a segment goes to handed + rank (ballot + mbcnt, the
-// order the decoders read it).  A word is stored when its last bit is
-// packed, which comes after it is taken (a segment adds at most 30 bits,
-// and a lane takes a word only once it holds at most 32), so each lane
-// keeps the places of at most two taken, unfinished words.  Words taken
-// past the lane's bits, and the group's padding to 4 words, are zero.  The
-// stores go through a buffer resource bounded by the group's length.
-// TRIPLE: 2^11-state tables, segments of 3, 3, 2 steps (schedule.h).
-constexpr int kPlaceSteps = 16;   // steps whose chunks are loaded together (whole segments)
+// x += y with the carry out of every lane as a lane mask (v_add_co_u32 with
+// an SGPR carry).
+__device__ __forceinline__ Mask add_carry(uint32_t& x, uint32_t y) {
+    Mask c;
+    asm("v_add_co_u32 %0, %1, %2, %3" : "=v"(x), "=s"(c) : "v"(x), "v"(y));
+    return c;
+}
 
-template <bool TRIPLE>
+// m's lanes take if_set, the others if_clear (v_cndmask_b32 on the mask).
+__device__ __forceinline__ uint32_t select(Mask m, uint32_t if_set, uint32_t if_clear) {
+    return __builtin_amdgcn_inverse_ballot_w64(m) ? if_set : if_clear;
+}
+
+// Place in the lane's mask order (how many of m's lanes come before it).
+__device__ __forceinline__ uint32_t rank_in(Mask m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// One wave per group replays the refill schedule from the tile records while
+// each lane joins its tiles' bits into 32-bit words, LSB first.  A word's
+// place in the stream is fixed when the lane takes it: the first two words
+// of every lane are the first 2 x lanes words (first words in lane order,
+// then the second), and a word taken after a segment goes to handed + rank
+// (in lane order, as the decoders read it).  A lane takes a word whenever
+// its consumed bits cross a multiple of 32, which is also when its oldest
+// word is complete: it then stores that word at the place it took for it
+// (f0), and the newly taken place becomes the younger of its two (f1).  The
+// position in the oldest word is kept in the top 5 bits of `pos`, so adding
+// a segment's count there carries out exactly at a crossing.
+//
+// A tile's bits are appended to the unfinished word by one 64-bit shift per
+// word; the words come out of them in order, one at most per segment.  Words
+// taken past the lane's bits, and the group's padding to 4 words, are zero.
+// The stores go through a buffer resource bounded by the group's length.
+//
+// What bounds it: the vector-memory path, by its instructions: one scattered
+// store per segment.  2^29 elements at 1024 per lane, 0.58 GB: 142 us (201 us
+// with a 2-byte load per step and the bits joined step by step).
+constexpr int kPlaceAhead = 4;   // tiles whose records are in flight
+
+template <int SPS>
 __global__ __launch_bounds__(kEncBlock) void enc_place_kernel(
-    const uint16_t* __restrict__ chunks, int64_t K, int64_t S,
-    const int64_t* __restrict__ offsets, uint32_t* __restrict__ comp) {
-    // segments per kPlaceSteps steps, and their first steps and lengths
-    constexpr int kSegs = TRIPLE ? 6 : 8;
-    constexpr auto seg_first = [](int q) { return TRIPLE ? 8 * (q / 3) + 3 * (q % 3) : 2 * q; };
-    constexpr auto seg_len = [](int q) { return TRIPLE ? (q % 3 == 2 ? 2 : 3) : 2; };
-    static_assert(seg_first(kSegs - 1) + seg_len(kSegs - 1) == kPlaceSteps, "whole segments");
+    const uint32_t* __restrict__ rec, const uint32_t* __restrict__ ovf, int64_t K, int64_t N,
+    const int64_t* __restrict__ offsets, uint32_t* __restrict__ comp, int64_t words_total) {
+    using F = TileFmt<SPS>;
+    constexpr int NQ = (F::kTriple ? 160 : 96) / 32 + 1;   // words a tile's bits can touch
     const int lane = threadIdx.x & (kLanes - 1);
     // the group (wave-uniform, so the output resource stays in SGPRs)
     const int64_t g = (int64_t)blockIdx.x * (kEncBlock / kLanes) +
                       __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
-    const int64_t G = (K + kLanes - 1) / kLanes;
-    if (g >= G) return;
-    const int64_t k = g * kLanes + lane;
-    const bool active = k < K;
-    const int64_t kk = active ? k : K - 1;
-    const uint32_t lanes = (uint32_t)(K - g * kLanes < kLanes ? K - g * kLanes : kLanes);
+    const int64_t k0 = g * kLanes;
+    if (blockIdx.x == 0 && threadIdx.x < kTailWords) comp[words_total + threadIdx.x] = 0u;
+    if (k0 >= K) return;
+    const uint32_t lanes = (uint32_t)(K - k0 < kLanes ? K - k0 : kLanes);
+    const bool active = (uint32_t)lane < lanes;
     const int64_t base = offsets[g];
     const int64_t glen = offsets[g + 1] - base;
-    const Rsrc out = __builtin_amdgcn_make_buffer_rsrc(
-        comp + base, (short)0, (int)(glen > 0x1FFFFFFF ? 0x7FFFFFFF : glen * 4), 0x00020000);
-    // S <= 2^24 (checked by the launcher)
-    const int n_seg = (int)tans_sched::segments(S, TRIPLE);
-    const int32_t fin_below = S > 0 ? tans_sched::final_below(S, TRIPLE) : 0;
-    uint64_t acc = 0;   // packed bits not yet stored
-    uint32_t n = 0;     // how many
-    uint32_t f0 = (uint32_t)lane, f1 = lanes + (uint32_t)lane;   // places of unfinished words
-    uint32_t fc = S > 0 && active ? 2u : 0u;                      // how many
-    int32_t held = 64;  // bits the lane holds
-    uint32_t handed = S > 0 ? 2u * lanes : 0u;
-    // the chunks of steps t0 .. t0 + kPlaceSteps - 1 (zero past step S; the
-    // loads stay in bounds and unconditional, so a batch's loads leave
-    // together), one batch ahead of the packing
-    const uint32_t koff = (uint32_t)kk * 2u;   // K <= INT32_MAX (checked by the launcher)
-    const int steps = (int)S;
-    auto load = [&](uint32_t (&c)[kPlaceSteps], int t0) {
+    const Rsrc out = rsrc(comp + base, glen > 0x1FFFFFFF ? 0x7FFFFFFFu : (uint32_t)(glen * 4));
+    const int64_t S = N / SPS;
+    const int nt = (int)((N + kTile - 1) / kTile);   // S <= 2^24 (checked by the launcher)
+    const int last_segs = (int)tans_sched::last_tile_segments(S, F::kTriple);
+    // the final check: a lane that crossed takes a word when it then holds
+    // 32 - position < final_below bits
+    const uint32_t fin_pos = (uint32_t)(32 - tans_sched::final_below(S, F::kTriple));   // may be -1
+    uint32_t pos = 0;     // bits of the oldest word already known, in bits 31:27
+    uint32_t acc = 0;     // those bits
+    uint32_t f0 = (uint32_t)lane * 4u, f1 = (lanes + (uint32_t)lane) * 4u;   // places (bytes)
+    uint32_t handed = 8u * lanes;   // bytes handed out
+    // tile t's record (zero past the last tile and in lanes out of range)
+    const int64_t rec_stride = K * (kRecWords * 4);
+    auto load = [&](int t) {
+        const int tt = t < nt ? t : nt - 1;
+        return __builtin_amdgcn_raw_buffer_load_b96(
+            rsrc(reinterpret_cast<const char*>(rec) + (int64_t)tt * rec_stride +
+                     k0 * (kRecWords * 4),
+                 t < nt ? lanes * (kRecWords * 4) : 0u),
+            (uint32_t)lane * (kRecWords * 4), 0, 0);
+    };
+    // the words tile t's bits make, the unfinished one first
+    auto words_of = [&](const v3u& r, int t, uint32_t (&q)[NQ]) {
+        const uint32_t n = pos >> 27;
+        const uint64_t a = (uint64_t)r.y << n;
+        const uint64_t b = ((uint64_t)r.z << 32 | r.y) << n;
+        q[0] = (uint32_t)a | acc;
+        q[1] = (uint32_t)(b >> 32);
+        q[2] = (uint32_t)(((uint64_t)r.z << n) >> 32);
         #pragma unroll
-        for (int u = 0; u < kPlaceSteps; u++) {
-            const int t = t0 + u;
-            const char* row =
-                reinterpret_cast<const char*>(chunks + (int64_t)(t < steps ? t : steps - 1) * K);
-            const uint32_t v = *reinterpret_cast<const uint16_t*>(row + koff);
-            c[u] = t < steps ? v : 0u;   // wave-uniform
+        for (int i = 3; i < NQ; i++) q[i] = 0u;
+        uint32_t total = 0;
+        #pragma unroll
+        for (int s = 0; s < F::kSegs; s++) total += (r.x >> (5 * s)) & 31u;
+        if (__any(total > kRecBits)) {
+            uint32_t prev = r.z;
+            #pragma unroll
+            for (int i = 0; i < F::kOvf; i++) {
+                // words past the lane's bits were not written: zero
+                const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(
+                    rsrc(ovf + ((int64_t)t * F::kOvf + i) * K + k0,
+                         lanes * 4),
+                    (uint32_t)lane * 4, 0, 0);
+                const uint32_t w = total > kRecBits + 32u * i ? v : 0u;
+                q[2 + i] = (uint32_t)((((uint64_t)w << 32 | prev) << n) >> 32);
+                prev = w;
+            }
+            q[2 + F::kOvf] = (uint32_t)(((uint64_t)prev << n) >> 32);
         }
     };
-    uint32_t c[kPlaceSteps], cn[kPlaceSteps];
-    if (steps > 0) load(c, 0);
-    for (int t0 = 0; t0 < steps; t0 += kPlaceSteps) {
-        if (t0 + kPlaceSteps < steps) load(cn, t0 + kPlaceSteps);   // wave-uniform
-        const int j0 = t0 / kPlaceSteps * kSegs;
-        #pragma unroll
-        for (int q = 0; q < kSegs; q++) {
-            const int j = j0 + q;
-            if (j >= n_seg) break;   // wave-uniform
+    auto tile = [&](const v3u& r, int t) {
+        uint32_t q[NQ];
+        words_of(r, t, q);
+        static_for<0, F::kSegs>([&](auto I) {
+            constexpr int s = decltype(I)::value;
+            const Mask m = add_carry(pos, (r.x << (27 - 5 * s)) & 0xF8000000u);
+            if (__builtin_amdgcn_inverse_ballot_w64(m))
+                __builtin_amdgcn_raw_buffer_store_b32(q[0], out, f0, 0, 0);
+            f0 = select(m, f1, f0);
+            f1 = select(m, rank_in(m) * 4u + handed, f1);
+            handed += 4u * (uint32_t)__popcll(m);
+            // (the words left can be no more than the segments left, plus one)
             #pragma unroll
-            for (int u = seg_first(q); u < seg_first(q) + seg_len(q); u++) {
-                const uint32_t nb = c[u] >> 12;
-                acc |= (uint64_t)(c[u] & 0xFFFu) << n;
-                n += nb;
-                held -= (int32_t)nb;
-            }
-            if (n >= 32) {   // at most one word per segment (n < 32 + 30)
-                if (active)
-                    __builtin_amdgcn_raw_buffer_store_b32((uint32_t)acc, out, f0 * 4u, 0, 0);
-                f0 = f1;
-                fc--;
-                acc >>= 32;
-                n -= 32;
-            }
-            if (j + 1 < n_seg) {   // wave-uniform: no check after the last segment
-                const int32_t below = j + 2 == n_seg ? fin_below : tans_sched::kAtMost + 1;
-                const bool need = active && held < below;
-                const Mask m = __ballot(need);
-                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-                    (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                if (need) {
-                    if (fc == 0) f0 = handed + rank; else f1 = handed + rank;
-                    fc++;
-                    held += 32;
-                }
-                handed += (uint32_t)__popcll(m);
-            }
-        }
+            for (int i = 0; i < F::kSegs - s && i + 1 < NQ; i++) q[i] = select(m, q[i + 1], q[i]);
+        });
+        acc = q[0];
+    };
+    v3u r[kPlaceAhead];
+    #pragma unroll
+    for (int i = 0; i < kPlaceAhead; i++) r[i] = load(i);
+    int t = 0;
+    for (; t + kPlaceAhead < nt; t += kPlaceAhead) {
         #pragma unroll
-        for (int u = 0; u < kPlaceSteps; u++) c[u] = cn[u];
+        for (int i = 0; i < kPlaceAhead; i++) {
+            tile(r[i], t + i);
+            r[i] = load(t + i + kPlaceAhead);
+        }
+    }
+    // the last 1 .. kPlaceAhead tiles; the last one ends the streams
+    uint32_t fc = active ? 2u : 0u;   // places held
+    #pragma unroll
+    for (int i = 0; i < kPlaceAhead; i++) {
+        if (t + i >= nt) break;   // wave-uniform
+        if (t + i < nt - 1) {
+            tile(r[i], t + i);
+            continue;
+        }
+        uint32_t q[NQ];
+        words_of(r[i], nt - 1, q);
+        #pragma unroll
+        for (int s = 0; s < F::kSegs; s++) {
+            if (s >= last_segs) break;   // wave-uniform
+            const Mask m = add_carry(pos, (r[i].x << (27 - 5 * s)) & 0xF8000000u);
+            // after the last segment no word is taken, after the one before
+            // it only by the lanes that the final check names
+            const Mask take = s == last_segs - 1 ? Mask(0)
+                              : s == last_segs - 2
+                                  ? m & __ballot((int32_t)(pos >> 27) > (int32_t)fin_pos)
+                                  : m;
+            if (__builtin_amdgcn_inverse_ballot_w64(m))
+                __builtin_amdgcn_raw_buffer_store_b32(q[0], out, f0, 0, 0);
+            f0 = select(m, f1, f0);
+            f1 = select(take, rank_in(take) * 4u + handed, f1);
+            fc -= select(m & ~take, 1u, 0u);
+            handed += 4u * (uint32_t)__popcll(take);
+            #pragma unroll
+            for (int j = 0; j + 1 < NQ; j++) q[j] = select(m, q[j + 1], q[j]);
+        }
+        acc = q[0];
     }
     if (active) {
-        if (n > 0) {   // the last, partial word
-            __builtin_amdgcn_raw_buffer_store_b32((uint32_t)acc, out, f0 * 4u, 0, 0);
+        if (pos >> 27) {   // the last, partial word
+            __builtin_amdgcn_raw_buffer_store_b32(acc, out, f0, 0, 0);
             f0 = f1;
             fc--;
         }
-        if (fc >= 1) __builtin_amdgcn_raw_buffer_store_b32(0u, out, f0 * 4u, 0, 0);
-        if (fc >= 2) __builtin_amdgcn_raw_buffer_store_b32(0u, out, f1 * 4u, 0, 0);
+        if (fc >= 1) __builtin_amdgcn_raw_buffer_store_b32(0u, out, f0, 0, 0);
+        if (fc >= 2) __builtin_amdgcn_raw_buffer_store_b32(0u, out, f1, 0, 0);
     }
     // padding up to the 4-word boundary
-    if ((int64_t)handed + lane < glen)
-        __builtin_amdgcn_raw_buffer_store_b32(0u, out, (handed + (uint32_t)lane) * 4u, 0, 0);
+    if ((int64_t)handed + 4 * lane < glen * 4)
+        __builtin_amdgcn_raw_buffer_store_b32(0u, out, handed + 4u * (uint32_t)lane, 0, 0);
 }
 
 // The packed layout: one wave per group.  Each lane reads its bit count
 // (plen), the pair's count is the two lanes' sum, and a scan of the counts
 // over the wave gives each pair's end; the wave then ORs the header and
-// every lane's bits (state minus L, then each step's chunk; even lanes
-// forwards from the pair's start, odd lanes bit-reversed backwards from its
-// end) into its LDS buffer, which holds the longest possible stream, and
-// copies the group's stream words out (zeros past the bits).
+// every lane's bits (state minus L, then each tile's; even lanes forwards
+// from the pair's start, odd lanes bit-reversed backwards from its end) into
+// its LDS buffer, which holds the longest possible stream, and copies the
+// group's stream words out (zeros past the bits).  A tile goes in as up to
+// three 32-bit fields, not step by step.
 constexpr int kPackWords = (int)(tans_pack::max_stream_bytes(tans_pack::kMaxSteps) / 4);
+constexpr int kPackTiles = (int)(2 * tans_pack::kMaxSteps / kTile);
 
 __global__ __launch_bounds__(kEncBlock) void enc_place_packed_kernel(
-    const uint16_t* __restrict__ chunks, const uint16_t* __restrict__ pstate,
-    const uint16_t* __restrict__ plen, int64_t K, int64_t S, uint32_t L,
-    const int64_t* __restrict__ offsets, uint32_t* __restrict__ comp) {
+    const uint32_t* __restrict__ rec, const uint32_t* __restrict__ ovf,
+    const uint16_t* __restrict__ pstate, const uint16_t* __restrict__ plen, int64_t K, int64_t N,
+    uint32_t L, const int64_t* __restrict__ offsets, uint32_t* __restrict__ comp,
+    int64_t words_total) {
+    using F = TileFmt<2>;
     __shared__ uint32_t bufs[kEncBlock / kLanes][kPackWords];
     const int lane = threadIdx.x & (kLanes - 1);
-    const int wave = threadIdx.x / kLanes;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
     const int64_t g = (int64_t)blockIdx.x * (kEncBlock / kLanes) + wave;
-    const int64_t G = (K + kLanes - 1) / kLanes;
-    if (g >= G) return;
+    if (blockIdx.x == 0 && threadIdx.x < kTailWords) comp[words_total + threadIdx.x] = 0u;
+    const int64_t k0 = g * kLanes;
+    if (k0 >= K) return;
+    const uint32_t lanes = (uint32_t)(K - k0 < kLanes ? K - k0 : kLanes);
+    const bool active = (uint32_t)lane < lanes;
+    const int nt = (int)((N + kTile - 1) / kTile);   // at most kPackTiles (checked by the launcher)
+    v3u r[kPackTiles];
+    #pragma unroll
+    for (int t = 0; t < kPackTiles; t++)
+        r[t] = __builtin_amdgcn_raw_buffer_load_b96(
+            rsrc(rec + ((int64_t)(t < nt ? t : nt - 1) * K + k0) * kRecWords,
+                 t < nt ? lanes * (kRecWords * 4) : 0u),
+            (uint32_t)lane * (kRecWords * 4), 0, 0);
     uint32_t* b = bufs[wave];
     for (int i = lane; i < kPackWords; i += kLanes) b[i] = 0u;
-    const int64_t k = g * kLanes + lane;
-    const bool active = k < K;
-    const uint32_t len = active ? plen[k] : 0u;
+    const uint32_t len = active ? plen[k0 + lane] : 0u;
+    const uint32_t st = active ? (uint32_t)pstate[k0 + lane] - L : 0u;
     const uint32_t cnt = len + (uint32_t)__shfl_xor((int)len, 1, kLanes);   // the pair's bits
     uint32_t v = (lane & 1) ? 0u : cnt;
     #pragma unroll
@@ -497,6 +769,7 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_packed_kernel(
         const uint32_t y = (uint32_t)__shfl_up((int)v, d, kLanes);
         if (lane >= d) v += y;
     }
+    const int64_t S = N / 2;
     const int hb = tans_pack::hdr_bytes(S);
     const uint32_t end = (uint32_t)tans_pack::hdr_total(S) * 8u + v;
     const uint32_t start = end - cnt;
@@ -508,6 +781,7 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_packed_kernel(
     if (active) {
         const bool odd = lane & 1;
         uint32_t o = 0;   // bits of the lane placed so far
+        // the low nb <= 32 bits of val (the others zero) as the lane's next bits
         auto put = [&](uint32_t val, uint32_t nb) {
             if (nb == 0) return;
             // odd lanes: the field's bits run backwards, so it sits reversed
@@ -515,79 +789,30 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_packed_kernel(
             const uint32_t p = odd ? end - o - nb : start + o;
             const uint32_t f = odd ? __builtin_bitreverse32(val) >> (32u - nb) : val;
             const uint32_t sh = p & 31u;
-            atomicOr(&b[p >> 5], f << sh);
-            if (sh + nb > 32u) atomicOr(&b[(p >> 5) + 1], f >> (32u - sh));
+            if (p + nb <= (uint32_t)kPackWords * 32u) {   // (a well-formed stream always fits)
+                atomicOr(&b[p >> 5], f << sh);
+                if (sh + nb > 32u) atomicOr(&b[(p >> 5) + 1], f >> (32u - sh));
+            }
             o += nb;
         };
-        put((uint32_t)pstate[k] - L, (uint32_t)tans_pack::kStateBits);
-        for (int64_t s = 0; s < S; s++) {
-            const uint32_t c = chunks[s * K + k];
-            put(c & 0xFFFu, c >> 12);
+        put(st, (uint32_t)tans_pack::kStateBits);
+        #pragma unroll
+        for (int t = 0; t < kPackTiles; t++) {
+            if (t >= nt) break;   // wave-uniform
+            uint32_t total = 0;
+            #pragma unroll
+            for (int s = 0; s < F::kSegs; s++) total += (r[t].x >> (5 * s)) & 31u;
+            put(r[t].y, total < 32u ? total : 32u);
+            if (total > 32u) put(r[t].z, total < 64u ? total - 32u : 32u);
+            if (total > 64u) {
+                const uint32_t w = total < 96u ? total - 64u : 32u;
+                put(ovf[(int64_t)t * K + k0 + lane] , w);
+            }
         }
     }
     const int64_t base = offsets[g];
     const int64_t glen = offsets[g + 1] - base;
     for (int64_t i = lane; i < glen && i < kPackWords; i += kLanes) comp[base + i] = b[i];
-}
-
-// Sign/mantissa tiles: sm[(t K + k) * 8] from bytes [16t, 16t + 16) of row
-// k (zero past N).  A workgroup of 4 waves takes 32 rows x 64 tiles: each
-// wave reads 8 rows, one row segment of 1 KiB per instruction (lane = tile),
-// turns each 16 bytes into the tile's two sm words, and stages them in LDS
-// by [tile][row]; after a barrier each wave writes 16 tiles as contiguous
-// 256-byte runs of 32 rows.
-constexpr int kSmRows = 32;                      // rows per workgroup
-constexpr int kSmCols = kLanes;                  // tiles per workgroup
-constexpr int kSmPad = kSmRows + 1;              // LDS row stride (records): 2-way banks at most
-
-__global__ __launch_bounds__(kEncBlock) void enc_sm_kernel(const uint8_t* __restrict__ fp8,
-                                                           int64_t K, int64_t N, int64_t n_tiles,
-                                                           uint32_t* __restrict__ sm) {
-    static_assert(kEncBlock == 4 * kLanes && kSmRows % 4 == 0, "4 waves, 8 rows each");
-    __shared__ uint2 st[kSmCols * kSmPad];
-    const int lane = threadIdx.x & (kLanes - 1);
-    const int wave = threadIdx.x / kLanes;
-    const int64_t col_blocks = (n_tiles + kSmCols - 1) / kSmCols;
-    const int64_t rb = blockIdx.x / col_blocks, cb = blockIdx.x % col_blocks;
-    const int64_t k0 = rb * kSmRows, t0 = cb * kSmCols;
-    const int64_t t = t0 + lane;   // this lane's tile in the load phase
-    constexpr int kPerWave = kSmRows / 4;
-    #pragma unroll
-    for (int u = 0; u < kPerWave; u++) {
-        const int r = wave * kPerWave + u;
-        const int64_t k = k0 + r;
-        uint32_t b[4] = {0u, 0u, 0u, 0u};
-        if (k < K && t < n_tiles) {
-            const uint8_t* row = fp8 + k * N;
-            if (N % kTile == 0) {   // whole, 16-byte aligned tiles
-                const uint4 v = *reinterpret_cast<const uint4*>(row + t * kTile);
-                b[0] = v.x; b[1] = v.y; b[2] = v.z; b[3] = v.w;
-            } else {
-                #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    #pragma unroll
-                    for (int y = 0; y < 4; y++) {
-                        const int64_t c = t * kTile + 4 * q + y;
-                        if (c < N) b[q] |= (uint32_t)row[c] << (8 * y);
-                    }
-                }
-            }
-        }
-        uint32_t w0, w1;
-        sm_words(b, w0, w1);
-        st[lane * kSmPad + r] = uint2{w0, w1};
-    }
-    __syncthreads();
-    // store phase: each instruction writes two tiles x 32 rows (lane / 32, lane % 32)
-    const int r = lane % kSmRows;
-    const int64_t k = k0 + r;
-    #pragma unroll
-    for (int v = 0; v < kSmCols / 8; v++) {
-        const int tt = (wave * (kSmCols / 8) + v) * 2 + lane / kSmRows;
-        const int64_t tg = t0 + tt;
-        if (k < K && tg < n_tiles)
-            *reinterpret_cast<uint2*>(sm + (tg * K + k) * 2) = st[tt * kSmPad + r];
-    }
 }
 
 }  // namespace
@@ -599,8 +824,7 @@ int tans_gpu_encode_workspace(int64_t K, int64_t N, int32_t log2L, int64_t* work
         return fail(TANS_EINVAL, "gpu_encode: need K >= 0 and even N >= 0");
     if (log2L != TANS_PAIR_LOG2L && log2L != TANS_NIBBLE_LOG2L)
         return fail(TANS_EINVAL, "gpu_encode: log2L must be 12 (pair) or 11 (nibble)");
-    const int64_t S = log2L == TANS_PAIR_LOG2L ? N / 2 : N;
-    *workspace_bytes = ws_layout(K, S).total;
+    *workspace_bytes = ws_layout(K, N, log2L).total;
     return TANS_OK;
 }
 
@@ -635,39 +859,29 @@ int gpu_encode_begin(const void* fp8, int64_t K, int64_t N, const uint32_t* enc_
     const int sps = log2L == TANS_PAIR_LOG2L ? 2 : 1;
     const int64_t S = N / sps;
     const int64_t G = (K + kLanes - 1) / kLanes;
-    const int64_t n_tiles = (N + kTile - 1) / kTile;
-    // K within int32 (the kernels' lane offsets) and every grid within the
-    // 32-bit work-item count of a launch
-    const int64_t sm_blocks = (K + kSmRows - 1) / kSmRows * ((n_tiles + kSmCols - 1) / kSmCols);
-    if (K > INT32_MAX || S > (int64_t(1) << 24) || sm_blocks > int64_t(UINT32_MAX) / kEncBlock)
+    // K within int32 keeps every grid within a launch's 32-bit work-item count
+    if (K > INT32_MAX || S > (int64_t(1) << 24))
         return fail(TANS_EINVAL, "gpu_encode: tensor too large");
-    const WsLayout l = ws_layout(K, S);
+    const WsLayout l = ws_layout(K, N, log2L);
     char* ws = static_cast<char*>(workspace);
-    uint16_t* chunks = reinterpret_cast<uint16_t*>(ws + l.chunks);
+    uint32_t* rec = reinterpret_cast<uint32_t*>(ws + l.rec);
+    uint32_t* ovf = reinterpret_cast<uint32_t*>(ws + l.ovf);
     uint32_t* glen = reinterpret_cast<uint32_t*>(ws + l.glen);
     uint16_t* plen = reinterpret_cast<uint16_t*>(ws + l.plen);
+    uint16_t* st_out = packed ? reinterpret_cast<uint16_t*>(ws + l.pstate) : states;
     hipStream_t st = (hipStream_t)stream;
-    const unsigned lane_blocks = (unsigned)((K + kEncBlock - 1) / kEncBlock);
-    if (packed)
-        hipLaunchKernelGGL((enc_backward_kernel<2, true>), dim3(lane_blocks), dim3(kEncBlock), 0,
-                           st, (const uint8_t*)fp8, K, N, enc_tab, enc_next, (int)log2L, chunks,
-                           reinterpret_cast<uint16_t*>(ws + l.pstate), glen, (uint32_t*)sm,
-                           status, plen);
-    else if (sps == 2)
-        hipLaunchKernelGGL(enc_backward_kernel<2>, dim3(lane_blocks), dim3(kEncBlock), 0, st,
-                           (const uint8_t*)fp8, K, N, enc_tab, enc_next, (int)log2L, chunks,
-                           states, glen, (uint32_t*)sm, status, plen);
-    else
-        hipLaunchKernelGGL(enc_backward_kernel<1>, dim3(lane_blocks), dim3(kEncBlock), 0, st,
-                           (const uint8_t*)fp8, K, N, enc_tab, enc_next, (int)log2L, chunks,
-                           states, glen, (uint32_t*)sm, status, plen);
-    if ((rc = hip_check(hipGetLastError(), "enc_backward_kernel launch"))) return rc;
-    hipLaunchKernelGGL(enc_scan_kernel, dim3(1), dim3(1024), 0, st, glen, G, offsets);
-    if ((rc = hip_check(hipGetLastError(), "enc_scan_kernel launch"))) return rc;
-    if (N % 16 == 0) return TANS_OK;   // the backward pass wrote the sign/mantissa tiles
-    hipLaunchKernelGGL(enc_sm_kernel, dim3((unsigned)sm_blocks), dim3(kEncBlock), 0, st,
-                       (const uint8_t*)fp8, K, N, n_tiles, (uint32_t*)sm);
-    return hip_check(hipGetLastError(), "enc_sm_kernel launch");
+    const dim3 grid((unsigned)((G + kEncBlock / kLanes - 1) / (kEncBlock / kLanes)));
+    const RowSrc src{(const uint8_t*)fp8, K, N, nullptr, 0};
+    auto walk = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kEncBlock), 0, st, src, K, N, enc_tab, enc_next,
+                           (int)log2L, rec, ovf, st_out, glen, (uint32_t*)sm, status, plen);
+    };
+    if (packed) walk(enc_walk_kernel<2, true, RowSrc>);
+    else if (sps == 2) walk(enc_walk_kernel<2, false, RowSrc>);
+    else walk(enc_walk_kernel<1, false, RowSrc>);
+    if ((rc = hip_check(hipGetLastError(), "enc_walk_kernel launch"))) return rc;
+    hipLaunchKernelGGL(enc_scan_kernel, dim3(1), dim3(kScanBlock), 0, st, glen, G, offsets);
+    return hip_check(hipGetLastError(), "enc_scan_kernel launch");
 }
 
 int gpu_encode_finish(int64_t K, int64_t N, int32_t log2L, const void* workspace,
@@ -685,25 +899,25 @@ int gpu_encode_finish(int64_t K, int64_t N, int32_t log2L, const void* workspace
     const int64_t words_total = comp_bytes / 4 - kTailWords;
     uint32_t* c32 = static_cast<uint32_t*>(comp);
     if (K > 0 && N > 0) {
-        const int sps = log2L == TANS_PAIR_LOG2L ? 2 : 1;
-        const int64_t S = N / sps;
         const int64_t G = (K + kLanes - 1) / kLanes;
-        const WsLayout l = ws_layout(K, S);
+        const WsLayout l = ws_layout(K, N, log2L);
         const char* ws = static_cast<const char*>(workspace);
         const dim3 grid((unsigned)((G + kEncBlock / kLanes - 1) / (kEncBlock / kLanes)));
-        const uint16_t* ch = reinterpret_cast<const uint16_t*>(ws + l.chunks);
+        const uint32_t* rec = reinterpret_cast<const uint32_t*>(ws + l.rec);
+        const uint32_t* ovf = reinterpret_cast<const uint32_t*>(ws + l.ovf);
+        // (the place kernels zero the tail words too)
         if (packed)
-            hipLaunchKernelGGL(enc_place_packed_kernel, grid, dim3(kEncBlock), 0, st, ch,
+            hipLaunchKernelGGL(enc_place_packed_kernel, grid, dim3(kEncBlock), 0, st, rec, ovf,
                                reinterpret_cast<const uint16_t*>(ws + l.pstate),
-                               reinterpret_cast<const uint16_t*>(ws + l.plen), K, S,
-                               (uint32_t)(1u << log2L), offsets, c32);
-        else if (sps == 1)   // 2^11-state tables: the 3-3-2 schedule
-            hipLaunchKernelGGL(enc_place_kernel<true>, grid, dim3(kEncBlock), 0, st, ch, K, S,
-                               offsets, c32);
+                               reinterpret_cast<const uint16_t*>(ws + l.plen), K, N,
+                               (uint32_t)(1u << log2L), offsets, c32, words_total);
+        else if (log2L == TANS_NIBBLE_LOG2L)
+            hipLaunchKernelGGL(enc_place_kernel<1>, grid, dim3(kEncBlock), 0, st, rec, ovf, K, N,
+                               offsets, c32, words_total);
         else
-            hipLaunchKernelGGL(enc_place_kernel<false>, grid, dim3(kEncBlock), 0, st, ch, K, S,
-                               offsets, c32);
-        if ((rc = hip_check(hipGetLastError(), "enc_place_kernel launch"))) return rc;
+            hipLaunchKernelGGL(enc_place_kernel<2>, grid, dim3(kEncBlock), 0, st, rec, ovf, K, N,
+                               offsets, c32, words_total);
+        return hip_check(hipGetLastError(), "enc_place_kernel launch");
     }
     hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((kTailWords + kEncBlock - 1) / kEncBlock)),
                        dim3(kEncBlock), 0, st, c32 + words_total, kTailWords);
