@@ -224,6 +224,19 @@ int tans_gpu_encode_begin(const void* fp8, int64_t K, int64_t N, const uint32_t*
 int tans_gpu_encode_finish(int64_t K, int64_t N, int32_t log2L, const void* workspace,
                            const int64_t* offsets, void* comp, int64_t comp_bytes, void* stream);
 
+/* tans_gpu_encode_begin of a matrix W [R, C] (device, row-major, any
+ * alignment, C >= 16) in the layout tans_fp8_gemm_fused reads (below): rows
+ * padded to Rp, S segments of Nc columns, rows past R and columns past C
+ * read as the byte `pad`, without a copy of W in lane order.  K = 4 * S * Rp
+ * lanes of N = Nc / 4 elements: the workspace is tans_gpu_encode_workspace's
+ * for that K and N, and tans_gpu_encode_finish(K, N, ..) completes it.  No
+ * counterpart in the reference.                                          */
+int tans_gpu_encode_matrix_begin(const void* w, int64_t R, int64_t C, int64_t S, int64_t Nc,
+                                 int32_t pad, const uint32_t* enc_tab, const uint16_t* enc_next,
+                                 int32_t log2L, void* workspace, int64_t workspace_bytes,
+                                 int64_t* offsets, uint16_t* states, void* sm, int32_t* status,
+                                 void* stream);
+
 /* The GPU encoder into the packed layout of short streams (log2L 12, N <= 64):
  * the same bytes as tans_encode_packed_begin/finish, with the same
  * workspace, the same calls and no states output.  Replaces, like those,

@@ -295,6 +295,7 @@ __device__ __forceinline__ uint32_t lane_words(int64_t S, bool triple, uint32_t 
 // 16-byte aligned; others start on any even byte, and their tiles are
 // unaligned 16-byte loads (gfx950 takes any alignment).
 typedef v4u v4u_any __attribute__((aligned(1)));
+typedef v2u v2u_any __attribute__((aligned(1)));
 
 struct RowSrc {
     const uint8_t* fp8;
@@ -329,6 +330,67 @@ struct RowSrc {
         }
         return v;
     }
+};
+
+// The lanes of a matrix W [R, C] in the decode-GEMM's layout (the lane streams
+// of rans_vectoradd.tans_codec.gemm_slab, read where they lie): lane ((s *
+// n_rg + g) * 4 + q) * 16 + r holds row 16 g + r of segment s (columns s Nc
+// on): its tile t is columns 16 q .. 16 q + 15 of the segment's 64-column
+// block t, and of a last block of 32 columns it has the 8 columns 8 q on.
+// Rows past R and columns past C read as the byte `pad`.  C >= 16.
+struct MatSrc {
+    const uint8_t* w;
+    int64_t R, C;
+    int n_rg, Nc;
+    uint32_t pad4;        // `pad` in each byte
+
+    const uint8_t* p;     // the lane's columns of block 0
+    const uint8_t* p8;    // its columns of a last 32-column block
+    int lim, lim8;        // columns of W from p, p8 on (0 in rows past R)
+    bool inside;          // every whole tile of the wave's lanes lies in W
+
+    __device__ __forceinline__ void start(int64_t k) {
+        const uint32_t grp = __builtin_amdgcn_readfirstlane((uint32_t)(k / kLanes));
+        const int j = (int)(k % kLanes), q = j >> 4;
+        const uint32_t s = grp / (uint32_t)n_rg;
+        const int64_t row = (int64_t)(grp % (uint32_t)n_rg) * 16 + (j & 15);
+        const int64_t col0 = (int64_t)s * Nc;
+        const int blocks = Nc / 64;
+        p = w + (row < R ? row * C : 0) + col0 + 16 * q;
+        p8 = p + 64 * blocks - 8 * q;
+        const int64_t left = row < R ? C - col0 : 0;
+        auto clamp = [](int64_t v) { return (int)(v < 0 ? 0 : v > kMaxCols ? kMaxCols : v); };
+        lim = clamp(left - 16 * q);
+        lim8 = clamp(left - 64 * blocks - 8 * q);
+        inside = __all(lim >= 64 * (blocks - 1) + 16);
+    }
+    // the n bytes (8 or 16) at a, of which `avail` lie in W: loaded as the
+    // n bytes that end with them (inside the row, as C >= 16), shifted down
+    // and padded
+    template <int n>
+    __device__ __forceinline__ v4u edge(const uint8_t* a, int avail) const {
+        avail = avail < 0 ? 0 : avail > n ? n : avail;
+        const uint8_t* from = avail ? a - (n - avail) : w;
+        unsigned __int128 v = 0, fill = 0;
+        if constexpr (n == 16) {
+            v = __builtin_bit_cast(unsigned __int128, *reinterpret_cast<const v4u_any*>(from));
+            fill = __builtin_bit_cast(unsigned __int128, v4u{pad4, pad4, pad4, pad4});
+        } else {
+            v = __builtin_bit_cast(uint64_t, *reinterpret_cast<const v2u_any*>(from));
+            fill = __builtin_bit_cast(unsigned __int128, v4u{pad4, pad4, 0u, 0u});
+        }
+        const uint32_t up = (uint32_t)avail * 8u, down = (uint32_t)(n - avail) * 8u;
+        const unsigned __int128 kept = avail ? v >> (down & 127u) : 0;
+        // the pad bytes sit above the kept ones, below byte n
+        const unsigned __int128 above = avail < n ? (fill >> (up & 127u)) << (up & 127u) : 0;
+        return __builtin_bit_cast(v4u, kept | above);
+    }
+    __device__ __forceinline__ v4u tile(int64_t t) const {
+        if (inside) return *reinterpret_cast<const v4u_any*>(p + 64 * t);   // wave-uniform
+        return edge<16>(p + 64 * t, lim - 64 * (int)t);
+    }
+    __device__ __forceinline__ v4u last(int64_t, int) const { return edge<8>(p8, lim8); }
+    static constexpr int kMaxCols = 1 << 20;   // more than any segment's columns
 };
 
 // One wave per 64-lane group; each lane walks its row backwards, a tile at a
@@ -832,11 +894,13 @@ int tans_gpu_encode_workspace(int64_t K, int64_t N, int32_t log2L, int64_t* work
 
 namespace {
 
-// begin of both layouts; packed: states == NULL (the workspace keeps them)
-int gpu_encode_begin(const void* fp8, int64_t K, int64_t N, const uint32_t* enc_tab,
-                     const uint16_t* enc_next, int32_t log2L, void* workspace,
-                     int64_t workspace_bytes, int64_t* offsets, uint16_t* states, void* sm,
-                     int32_t* status, void* stream, bool packed) {
+// begin of every source and layout; packed: states == NULL (the workspace
+// keeps them)
+template <class Src>
+int gpu_encode_begin(const Src& src, const void* data, int64_t K, int64_t N,
+                     const uint32_t* enc_tab, const uint16_t* enc_next, int32_t log2L,
+                     void* workspace, int64_t workspace_bytes, int64_t* offsets, uint16_t* states,
+                     void* sm, int32_t* status, void* stream, bool packed) {
     int64_t need = 0;
     int rc = tans_gpu_encode_workspace(K, N, log2L, &need);
     if (rc) return rc;
@@ -850,12 +914,10 @@ int gpu_encode_begin(const void* fp8, int64_t K, int64_t N, const uint32_t* enc_
         }
         return fail(TANS_EINVAL, "gpu_encode: N must be positive when K > 0");
     }
-    if (!fp8 || !enc_tab || !enc_next || !workspace || !offsets || (!states && !packed) || !sm ||
+    if (!data || !enc_tab || !enc_next || !workspace || !offsets || (!states && !packed) || !sm ||
         !status)
         return fail(TANS_EINVAL, "gpu_encode: null pointer");
     if (workspace_bytes < need) return fail(TANS_EINVAL, "gpu_encode: workspace too small");
-    if (reinterpret_cast<uintptr_t>(fp8) % 16)
-        return fail(TANS_EINVAL, "gpu_encode: fp8 must be 16-byte aligned");
     const int sps = log2L == TANS_PAIR_LOG2L ? 2 : 1;
     const int64_t S = N / sps;
     const int64_t G = (K + kLanes - 1) / kLanes;
@@ -871,17 +933,32 @@ int gpu_encode_begin(const void* fp8, int64_t K, int64_t N, const uint32_t* enc_
     uint16_t* st_out = packed ? reinterpret_cast<uint16_t*>(ws + l.pstate) : states;
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid((unsigned)((G + kEncBlock / kLanes - 1) / (kEncBlock / kLanes)));
-    const RowSrc src{(const uint8_t*)fp8, K, N, nullptr, 0};
     auto walk = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(kEncBlock), 0, st, src, K, N, enc_tab, enc_next,
                            (int)log2L, rec, ovf, st_out, glen, (uint32_t*)sm, status, plen);
     };
-    if (packed) walk(enc_walk_kernel<2, true, RowSrc>);
-    else if (sps == 2) walk(enc_walk_kernel<2, false, RowSrc>);
-    else walk(enc_walk_kernel<1, false, RowSrc>);
+    if constexpr (std::is_same_v<Src, RowSrc>) {
+        if (packed) walk(enc_walk_kernel<2, true, Src>);
+    }
+    if (!packed) {
+        if (sps == 2) walk(enc_walk_kernel<2, false, Src>);
+        else walk(enc_walk_kernel<1, false, Src>);
+    }
     if ((rc = hip_check(hipGetLastError(), "enc_walk_kernel launch"))) return rc;
     hipLaunchKernelGGL(enc_scan_kernel, dim3(1), dim3(kScanBlock), 0, st, glen, G, offsets);
     return hip_check(hipGetLastError(), "enc_scan_kernel launch");
+}
+
+// begin of a tensor's rows
+int gpu_encode_rows(const void* fp8, int64_t K, int64_t N, const uint32_t* enc_tab,
+                    const uint16_t* enc_next, int32_t log2L, void* workspace,
+                    int64_t workspace_bytes, int64_t* offsets, uint16_t* states, void* sm,
+                    int32_t* status, void* stream, bool packed) {
+    if (reinterpret_cast<uintptr_t>(fp8) % 16)
+        return fail(TANS_EINVAL, "gpu_encode: fp8 must be 16-byte aligned");
+    return gpu_encode_begin(RowSrc{(const uint8_t*)fp8, K, N, nullptr, 0}, fp8, K, N, enc_tab,
+                            enc_next, log2L, workspace, workspace_bytes, offsets, states, sm,
+                            status, stream, packed);
 }
 
 int gpu_encode_finish(int64_t K, int64_t N, int32_t log2L, const void* workspace,
@@ -932,8 +1009,29 @@ int tans_gpu_encode_begin(const void* fp8, int64_t K, int64_t N, const uint32_t*
                           const uint16_t* enc_next, int32_t log2L, void* workspace,
                           int64_t workspace_bytes, int64_t* offsets, uint16_t* states, void* sm,
                           int32_t* status, void* stream) {
-    return gpu_encode_begin(fp8, K, N, enc_tab, enc_next, log2L, workspace, workspace_bytes,
+    return gpu_encode_rows(fp8, K, N, enc_tab, enc_next, log2L, workspace, workspace_bytes,
                             offsets, states, sm, status, stream, false);
+}
+
+int tans_gpu_encode_matrix_begin(const void* w, int64_t R, int64_t C, int64_t S, int64_t Nc,
+                                 int32_t pad, const uint32_t* enc_tab, const uint16_t* enc_next,
+                                 int32_t log2L, void* workspace, int64_t workspace_bytes,
+                                 int64_t* offsets, uint16_t* states, void* sm, int32_t* status,
+                                 void* stream) {
+    if (R <= 0 || C < 16 || S <= 0 || Nc <= 0 || Nc % 32 || Nc > 1024)
+        return fail(TANS_EINVAL, "gpu_encode_matrix: need R > 0, C >= 16 and segments of at most "
+                                 "1024 columns, a multiple of 32");
+    if (S > INT32_MAX || S * Nc < C || (S - 1) * Nc >= C)
+        return fail(TANS_EINVAL, "gpu_encode_matrix: S segments of Nc columns must cover C exactly");
+    if (pad < 0 || pad > 255) return fail(TANS_EINVAL, "gpu_encode_matrix: pad must be a byte");
+    // (R and S within int32 and K checked against it: no product overflows)
+    if (R > INT32_MAX) return fail(TANS_EINVAL, "gpu_encode_matrix: matrix too large");
+    const int64_t Rp = (R + kLanes - 1) / kLanes * kLanes;
+    if (S > INT32_MAX / (4 * Rp)) return fail(TANS_EINVAL, "gpu_encode_matrix: matrix too large");
+    const MatSrc src{(const uint8_t*)w, R, C, (int)(Rp / 16), (int)Nc,
+                     (uint32_t)pad * 0x01010101u, nullptr, nullptr, 0, 0, false};
+    return gpu_encode_begin(src, w, 4 * S * Rp, Nc / 4, enc_tab, enc_next, log2L, workspace,
+                            workspace_bytes, offsets, states, sm, status, stream, false);
 }
 
 int tans_gpu_encode_finish(int64_t K, int64_t N, int32_t log2L, const void* workspace,
@@ -945,7 +1043,7 @@ int tans_gpu_encode_packed_begin(const void* fp8, int64_t K, int64_t N, const ui
                                  const uint16_t* enc_next, int32_t log2L, void* workspace,
                                  int64_t workspace_bytes, int64_t* offsets, void* sm,
                                  int32_t* status, void* stream) {
-    return gpu_encode_begin(fp8, K, N, enc_tab, enc_next, log2L, workspace, workspace_bytes,
+    return gpu_encode_rows(fp8, K, N, enc_tab, enc_next, log2L, workspace, workspace_bytes,
                             offsets, nullptr, sm, status, stream, true);
 }
 

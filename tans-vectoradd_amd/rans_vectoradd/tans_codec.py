@@ -318,14 +318,16 @@ def encode_matrix(w_fp8: torch.Tensor, exp_freqs, *, segments: int | None = None
     lane holding a quarter of every 64-column block of its row (the A
     operand of the kernel's 16x16x32 matrix-core products).  Padding bytes
     hold the most frequent exponent (a finite value with a nonzero
-    frequency); the kernel multiplies them by zero.  A GPU tensor is laid
-    out and encoded on its GPU (encode_gpu: the same bytes), and the
-    result's tensors stay there; a CPU tensor is encoded on the CPU."""
+    frequency); the kernel multiplies them by zero.  A GPU tensor is
+    encoded on its GPU (the same bytes), and the result's tensors stay
+    there; a CPU tensor is encoded on the CPU."""
     if not (isinstance(w_fp8, torch.Tensor) and w_fp8.dim() == 2 and w_fp8.dtype == torch.uint8):
         raise ValueError("w_fp8 must be a 2-D uint8 tensor [R, C]")
     R, C = w_fp8.shape
     if R == 0 or C == 0:
         raise ValueError("empty matrix")
+    if alphabet not in ALPHABETS:
+        raise ValueError(f"alphabet must be one of {sorted(ALPHABETS)}")
     S = segments if segments is not None else gemm_segments(R, C)
     if S < 1:
         raise ValueError("segments must be >= 1")
@@ -337,17 +339,26 @@ def encode_matrix(w_fp8: torch.Tensor, exp_freqs, *, segments: int | None = None
     if isinstance(exp_freqs, torch.Tensor):
         exp_freqs = exp_freqs.detach().cpu().double().numpy()
     pad = int(np.argmax(np.asarray(exp_freqs, dtype=np.float64))) << 3
-    w = w_fp8
-    if Rp != R or S * Nc != C:
-        wp = torch.full((Rp, S * Nc), pad, dtype=torch.uint8, device=w.device)
-        wp[:R, :C] = w
-        w = wp
-    slab = gemm_slab(w, S, Nc)
     # the GEMM kernel reads the refill-schedule layout
-    if slab.is_cuda:
-        enc = encode_gpu(slab, exp_freqs, alphabet=alphabet, layout="words")
+    if w_fp8.is_cuda and C >= 16:
+        # the walk reads the lanes where they lie in W: no padded copy, no slab
+        w = w_fp8.contiguous()
+
+        def begin(log2L, tab, nxt, ws, offsets, states, sm, status, stream):
+            return lib.tans_gpu_encode_matrix_begin(w.data_ptr(), R, C, S, Nc, pad, tab, nxt,
+                                                    log2L, ws.data_ptr(), ws.numel(), offsets,
+                                                    states, sm, status, stream)
+
+        enc = _encode_lanes_gpu(begin, 4 * S * Rp, Nc // 4, exp_freqs, alphabet, w.device, False)
     else:
-        enc = encode(slab, exp_freqs, alphabet=alphabet, layout="words")
+        w = w_fp8
+        if Rp != R or S * Nc != C:
+            wp = torch.full((Rp, S * Nc), pad, dtype=torch.uint8, device=w.device)
+            wp[:R, :C] = w
+            w = wp
+        slab = gemm_slab(w, S, Nc)
+        enc = (encode_gpu if slab.is_cuda else encode)(slab, exp_freqs, alphabet=alphabet,
+                                                       layout="words")
     comp, states, offsets, partial, sm, freqs, spread = enc
     return TansMatrix(comp, states, offsets, partial, sm, freqs, spread, rows=R, cols=C,
                       segments=S, seg_cols=Nc, alphabet=alphabet)
@@ -415,13 +426,28 @@ def encode_gpu(fp8_bytes: torch.Tensor, exp_freqs, tile: int = 0, *, alphabet: s
     packed = packed_layout(N, alphabet, layout)
     if isinstance(exp_freqs, torch.Tensor):
         exp_freqs = exp_freqs.detach().cpu().float().numpy()
-    nsym, L, _ = ALPHABETS[alphabet]
-    log2L = L.bit_length() - 1
-    dev = fp8_bytes.device
-    freqs, spread, tab_d, next_d = _encode_tables(exp_freqs, alphabet, dev)
     x = fp8_bytes.contiguous()
-    if x.data_ptr() % 16:            # the kernels read 4- and 16-byte words
+    if x.data_ptr() % 16:            # the kernels read 16-byte words
         x = x.clone()
+
+    def begin(log2L, tab, nxt, ws, offsets, states, sm, status, stream):
+        if packed and K:
+            return lib.tans_gpu_encode_packed_begin(x.data_ptr(), K, N, tab, nxt, log2L,
+                                                    ws.data_ptr(), ws.numel(), offsets, sm,
+                                                    status, stream)
+        return lib.tans_gpu_encode_begin(x.data_ptr(), K, N, tab, nxt, log2L, ws.data_ptr(),
+                                         ws.numel(), offsets, states, sm, status, stream)
+
+    return _encode_lanes_gpu(begin, K, N, exp_freqs, alphabet, x.device, packed)
+
+
+def _encode_lanes_gpu(begin, K: int, N: int, exp_freqs, alphabet: str, dev: torch.device,
+                      packed: bool):
+    """The GPU encoder's passes over K lanes of N elements: `begin` starts
+    them on its source (an encode begin of the C ABI), the stream length is
+    read back, and finish writes the streams.  Returns the 7-tuple."""
+    log2L = ALPHABETS[alphabet][1].bit_length() - 1
+    freqs, spread, tab_d, next_d = _encode_tables(exp_freqs, alphabet, dev)
     G = -(-K // TANS_LANES)
     with torch.cuda.device(dev):
         ws_bytes = ctypes.c_int64()
@@ -432,16 +458,8 @@ def encode_gpu(fp8_bytes: torch.Tensor, exp_freqs, tile: int = 0, *, alphabet: s
         sm = torch.empty(((N + 15) // 16, K, 8), dtype=torch.uint8, device=dev)
         status = torch.zeros(1, dtype=torch.int32, device=dev)
         stream = torch.cuda.current_stream(dev).cuda_stream
-        if packed and K:
-            check(lib.tans_gpu_encode_packed_begin(
-                x.data_ptr(), K, N, tab_d.data_ptr(), next_d.data_ptr(), log2L, ws.data_ptr(),
-                ws.numel(), offsets.data_ptr(), sm.data_ptr(), status.data_ptr(), stream),
-                "encode_gpu")
-        else:
-            check(lib.tans_gpu_encode_begin(
-                x.data_ptr(), K, N, tab_d.data_ptr(), next_d.data_ptr(), log2L, ws.data_ptr(),
-                ws.numel(), offsets.data_ptr(), states.data_ptr(), sm.data_ptr(),
-                status.data_ptr(), stream), "encode_gpu")
+        check(begin(log2L, tab_d.data_ptr(), next_d.data_ptr(), ws, offsets.data_ptr(),
+                    states.data_ptr(), sm.data_ptr(), status.data_ptr(), stream), "encode_gpu")
         total, bad = (int(v) for v in torch.stack([offsets[G], status[0].to(torch.int64)]).tolist())
         if bad:
             raise RuntimeError("encode_gpu: data holds a symbol whose frequency is 0")

@@ -159,6 +159,29 @@ def test_encode_matrix_on_gpu_equals_cpu(R, alphabet, rows, cols, segments):
         assert torch.equal(getattr(a, part).cpu(), getattr(b, part)), part
 
 
+@pytest.mark.parametrize("alphabet", ALPHABETS)
+@pytest.mark.parametrize("rows,cols,segments", [(16, 16, 1), (17, 17, 1), (65, 95, 2), (64, 96, 1),
+                                                (63, 1033, None), (200, 4100, None), (3, 40, 2),
+                                                (64, 2048, 2), (10, 8, 1)])
+def test_encode_matrix_reads_w_in_place(R, alphabet, rows, cols, segments):
+    """The walk reads W's rows where they lie: columns that end inside a
+    16-column chunk, a half tile or a segment, odd row lengths (unaligned
+    rows), rows past R, a segment whose width is one half tile, fewer columns
+    than a chunk, and a matrix that starts at an odd address and ends with its
+    storage.  Bytes equal the CPU encoder's."""
+    from rans_vectoradd import data as D, tans_codec as T
+    _say(f"case: encode_matrix in place {rows}x{cols} S={segments} {alphabet}")
+    q, _ = D.gaussian_fp8_bytes((rows + 1) * cols, seed=rows * cols)
+    w = q[cols:].reshape(rows, cols)
+    hist = D.exp_histogram(q) + 1
+    big = q.cuda()
+    for wg in (w.cuda(), big[cols:].view(rows, cols), w.t().contiguous().cuda().t()):
+        a = T.encode_matrix(wg, hist, segments=segments, alphabet=alphabet)
+        b = T.encode_matrix(w, hist, segments=segments, alphabet=alphabet)
+        for part in ("comp", "states", "offsets", "sm", "freqs", "spread"):
+            assert torch.equal(getattr(a, part).cpu(), getattr(b, part)), part
+
+
 def test_checkpoint_container_on_gpu(R, tmp_path):
     """A checkpoint encoded with the GPU encoder into a container, loaded on
     the GPU: the lane tensor decodes to its bytes and the matrix gives the
