@@ -224,7 +224,18 @@ int tans_gpu_encode_begin(const void* fp8, int64_t K, int64_t N, const uint32_t*
 int tans_gpu_encode_finish(int64_t K, int64_t N, int32_t log2L, const void* workspace,
                            const int64_t* offsets, void* comp, int64_t comp_bytes, void* stream);
 
-/* tans_gpu_encode_begin of a matrix W [R, C] (device, row-major, any
+/* tans_gpu_encode_begin, or with packed != 0 tans_gpu_encode_packed_begin
+ * (below; states unused), that reports through result instead of status:
+ * int64 {stream words, 1 if a symbol has frequency 0 else 0}, written in
+ * stream order.  It may be device memory or pinned host memory, which a
+ * caller that waits for the stream reads without a copy.  No counterpart in
+ * the reference, whose encoder runs on the host (csrc/tans_codec.cpp:69-196). */
+int tans_gpu_encode_lanes_begin(const void* fp8, int64_t K, int64_t N, int32_t packed,
+                                const uint32_t* enc_tab, const uint16_t* enc_next, int32_t log2L,
+                                void* workspace, int64_t workspace_bytes, int64_t* offsets,
+                                uint16_t* states, void* sm, int64_t* result, void* stream);
+
+/* tans_gpu_encode_lanes_begin of a matrix W [R, C] (device, row-major, any
  * alignment, C >= 16) in the layout tans_fp8_gemm_fused reads (below): rows
  * padded to Rp, S segments of Nc columns, rows past R and columns past C
  * read as the byte `pad`, without a copy of W in lane order.  K = 4 * S * Rp
@@ -234,7 +245,7 @@ int tans_gpu_encode_finish(int64_t K, int64_t N, int32_t log2L, const void* work
 int tans_gpu_encode_matrix_begin(const void* w, int64_t R, int64_t C, int64_t S, int64_t Nc,
                                  int32_t pad, const uint32_t* enc_tab, const uint16_t* enc_next,
                                  int32_t log2L, void* workspace, int64_t workspace_bytes,
-                                 int64_t* offsets, uint16_t* states, void* sm, int32_t* status,
+                                 int64_t* offsets, uint16_t* states, void* sm, int64_t* result,
                                  void* stream);
 
 /* The GPU encoder into the packed layout of short streams (log2L 12, N <= 64):

@@ -134,6 +134,7 @@ __device__ __forceinline__ Rsrc rsrc(const void* base, uint32_t bytes) {
 // kBadNb, a multiple of 32: shifts and field widths see log2L (so x >> nb is
 // 1 and idx = start), and the tile's bit count shows it.
 constexpr uint32_t kBadNb = 1024;
+constexpr uint32_t kBadGroup = 0x80000000u;   // in glen: the group holds such a symbol
 
 __device__ __forceinline__ uint2 enc_consts(uint32_t e, int log2L) {
     const uint32_t L = 1u << log2L;
@@ -422,7 +423,7 @@ __global__ __launch_bounds__(kEncBlock) void enc_walk_kernel(
     Src src, int64_t K, int64_t N, const uint32_t* __restrict__ enc_tab,
     const uint16_t* __restrict__ next, int log2L, uint32_t* __restrict__ rec,
     uint32_t* __restrict__ ovf, uint16_t* __restrict__ states, uint32_t* __restrict__ glen,
-    uint32_t* __restrict__ sm, int* __restrict__ status, uint16_t* __restrict__ plen) {
+    uint32_t* __restrict__ sm, uint16_t* __restrict__ plen) {
     using F = TileFmt<SPS>;
     static_assert(kEncBlock % kLanes == 0, "blocks hold whole groups");
     __shared__ EncTab<SPS> tab;
@@ -518,10 +519,7 @@ __global__ __launch_bounds__(kEncBlock) void enc_walk_kernel(
     uint32_t words = 0;
     if (active) {
         states[k0 + lane] = (uint16_t)x;
-        if (bad >= kBadNb) {
-            *status = TANS_ESYMBOL;   // vector store: any failing lane may write it
-            bits = b1 = b2 = 0;       // its bit counts mean nothing
-        }
+        if (bad >= kBadNb) bits = b1 = b2 = 0;   // its bit counts mean nothing
         if constexpr (PACKED) {
             words = (uint32_t)tans_pack::kStateBits + bits;   // the lane's bits
             plen[k0 + lane] = (uint16_t)words;
@@ -531,12 +529,12 @@ __global__ __launch_bounds__(kEncBlock) void enc_walk_kernel(
     }
     #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) words += __shfl_xor(words, m, kLanes);
-    if (lane == 0) {
-        if constexpr (PACKED)   // header + bits, padded to 16 bytes
-            glen[g] = ((uint32_t)tans_pack::hdr_total(S) + (words + 7u) / 8u + 15u) / 16u * 4u;
-        else
-            glen[g] = (words + 3u) & ~3u;
-    }
+    if constexpr (PACKED)   // header + bits, padded to 16 bytes
+        words = ((uint32_t)tans_pack::hdr_total(S) + (words + 7u) / 8u + 15u) / 16u * 4u;
+    else
+        words = (words + 3u) & ~3u;
+    if (__any(bad >= kBadNb)) words |= kBadGroup;
+    if (lane == 0) glen[g] = words;
 }
 
 // offsets[g] = sum of glen[0..g), offsets[G] = total.  One workgroup takes
@@ -544,13 +542,18 @@ __global__ __launch_bounds__(kEncBlock) void enc_walk_kernel(
 // the previous round is summed.  A thread's items are a contiguous run, the
 // waves scan their threads' sums by shuffles and the 16 wave totals meet in
 // LDS.  (8192 groups: 12.9 us with one contiguous run per thread, read word
-// by word, 8.9 us now.)
+// by word, 8.9 us now.)  It also reports: *status = TANS_ESYMBOL if a group
+// is marked kBadGroup, and result = {total, 1 if any is}, which may be host
+// memory, so that a caller waiting for the stream needs no copy.  Either may
+// be null.
 constexpr int kScanBlock = 1024;
 constexpr int kScanItems = 8;
 
 __global__ __launch_bounds__(kScanBlock) void enc_scan_kernel(const uint32_t* __restrict__ glen,
                                                               int64_t G,
-                                                              int64_t* __restrict__ offsets) {
+                                                              int64_t* __restrict__ offsets,
+                                                              int* __restrict__ status,
+                                                              int64_t* __restrict__ result) {
     constexpr int kWaves = kScanBlock / kLanes;
     constexpr int64_t kRound = (int64_t)kScanBlock * kScanItems;
     __shared__ int64_t wave_sum[2][kWaves];
@@ -564,12 +567,17 @@ __global__ __launch_bounds__(kScanBlock) void enc_scan_kernel(const uint32_t* __
     uint32_t v[kScanItems], n[kScanItems];
     load(0, v);
     int64_t carry = 0;
+    uint32_t marks = 0;
     int buf = 0;
     for (int64_t base = 0; base < G; base += kRound) {
         load(base + kRound, n);
         int64_t sum = 0;
         #pragma unroll
-        for (int i = 0; i < kScanItems; i++) sum += v[i];
+        for (int i = 0; i < kScanItems; i++) {
+            marks |= v[i];
+            v[i] &= ~kBadGroup;
+            sum += v[i];
+        }
         int64_t inc = sum;   // inclusive scan over the wave
         #pragma unroll
         for (int d = 1; d < kLanes; d <<= 1) {
@@ -594,7 +602,15 @@ __global__ __launch_bounds__(kScanBlock) void enc_scan_kernel(const uint32_t* __
         }
         buf ^= 1;   // the next round writes the other buffer: one barrier per round
     }
-    if (threadIdx.x == 0) offsets[G] = carry;
+    const bool bad = __syncthreads_or((int)(marks & kBadGroup)) != 0;
+    if (threadIdx.x == 0) {
+        offsets[G] = carry;
+        if (bad && status) *status = TANS_ESYMBOL;
+        if (result) {
+            result[0] = carry;
+            result[1] = bad ? 1 : 0;
+        }
+    }
 }
 
 // Zero n words (a kernel rather than hipMemsetAsync, so a caller may
@@ -900,22 +916,22 @@ template <class Src>
 int gpu_encode_begin(const Src& src, const void* data, int64_t K, int64_t N,
                      const uint32_t* enc_tab, const uint16_t* enc_next, int32_t log2L,
                      void* workspace, int64_t workspace_bytes, int64_t* offsets, uint16_t* states,
-                     void* sm, int32_t* status, void* stream, bool packed) {
+                     void* sm, int32_t* status, int64_t* result, void* stream, bool packed) {
     int64_t need = 0;
     int rc = tans_gpu_encode_workspace(K, N, log2L, &need);
     if (rc) return rc;
     if (packed && (log2L != TANS_PAIR_LOG2L || N > 2 * tans_pack::kMaxSteps))
         return fail(TANS_EINVAL, "gpu_encode_packed: needs log2L 12 and N <= 64");
     if (K == 0 || N == 0) {
-        if (K == 0 && offsets) {   // offsets = {0}
-            hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(kEncBlock), 0, (hipStream_t)stream,
-                               reinterpret_cast<uint32_t*>(offsets), (int64_t)2);
+        if (K == 0 && offsets) {   // offsets = {0}: the scan of no groups
+            hipLaunchKernelGGL(enc_scan_kernel, dim3(1), dim3(kScanBlock), 0, (hipStream_t)stream,
+                               nullptr, (int64_t)0, offsets, status, result);
             return hip_check(hipGetLastError(), "gpu_encode offsets");
         }
         return fail(TANS_EINVAL, "gpu_encode: N must be positive when K > 0");
     }
     if (!data || !enc_tab || !enc_next || !workspace || !offsets || (!states && !packed) || !sm ||
-        !status)
+        (!status && !result))
         return fail(TANS_EINVAL, "gpu_encode: null pointer");
     if (workspace_bytes < need) return fail(TANS_EINVAL, "gpu_encode: workspace too small");
     const int sps = log2L == TANS_PAIR_LOG2L ? 2 : 1;
@@ -935,7 +951,7 @@ int gpu_encode_begin(const Src& src, const void* data, int64_t K, int64_t N,
     const dim3 grid((unsigned)((G + kEncBlock / kLanes - 1) / (kEncBlock / kLanes)));
     auto walk = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(kEncBlock), 0, st, src, K, N, enc_tab, enc_next,
-                           (int)log2L, rec, ovf, st_out, glen, (uint32_t*)sm, status, plen);
+                           (int)log2L, rec, ovf, st_out, glen, (uint32_t*)sm, plen);
     };
     if constexpr (std::is_same_v<Src, RowSrc>) {
         if (packed) walk(enc_walk_kernel<2, true, Src>);
@@ -945,7 +961,8 @@ int gpu_encode_begin(const Src& src, const void* data, int64_t K, int64_t N,
         else walk(enc_walk_kernel<1, false, Src>);
     }
     if ((rc = hip_check(hipGetLastError(), "enc_walk_kernel launch"))) return rc;
-    hipLaunchKernelGGL(enc_scan_kernel, dim3(1), dim3(kScanBlock), 0, st, glen, G, offsets);
+    hipLaunchKernelGGL(enc_scan_kernel, dim3(1), dim3(kScanBlock), 0, st, glen, G, offsets,
+                       status, result);
     return hip_check(hipGetLastError(), "enc_scan_kernel launch");
 }
 
@@ -953,12 +970,12 @@ int gpu_encode_begin(const Src& src, const void* data, int64_t K, int64_t N,
 int gpu_encode_rows(const void* fp8, int64_t K, int64_t N, const uint32_t* enc_tab,
                     const uint16_t* enc_next, int32_t log2L, void* workspace,
                     int64_t workspace_bytes, int64_t* offsets, uint16_t* states, void* sm,
-                    int32_t* status, void* stream, bool packed) {
+                    int32_t* status, int64_t* result, void* stream, bool packed) {
     if (reinterpret_cast<uintptr_t>(fp8) % 16)
         return fail(TANS_EINVAL, "gpu_encode: fp8 must be 16-byte aligned");
     return gpu_encode_begin(RowSrc{(const uint8_t*)fp8, K, N, nullptr, 0}, fp8, K, N, enc_tab,
                             enc_next, log2L, workspace, workspace_bytes, offsets, states, sm,
-                            status, stream, packed);
+                            status, result, stream, packed);
 }
 
 int gpu_encode_finish(int64_t K, int64_t N, int32_t log2L, const void* workspace,
@@ -1010,14 +1027,24 @@ int tans_gpu_encode_begin(const void* fp8, int64_t K, int64_t N, const uint32_t*
                           int64_t workspace_bytes, int64_t* offsets, uint16_t* states, void* sm,
                           int32_t* status, void* stream) {
     return gpu_encode_rows(fp8, K, N, enc_tab, enc_next, log2L, workspace, workspace_bytes,
-                            offsets, states, sm, status, stream, false);
+                            offsets, states, sm, status, nullptr, stream, false);
+}
+
+int tans_gpu_encode_lanes_begin(const void* fp8, int64_t K, int64_t N, int32_t packed,
+                                const uint32_t* enc_tab, const uint16_t* enc_next, int32_t log2L,
+                                void* workspace, int64_t workspace_bytes, int64_t* offsets,
+                                uint16_t* states, void* sm, int64_t* result, void* stream) {
+    if (!result) return fail(TANS_EINVAL, "gpu_encode_lanes: null result");
+    return gpu_encode_rows(fp8, K, N, enc_tab, enc_next, log2L, workspace, workspace_bytes,
+                           offsets, states, sm, nullptr, result, stream, packed != 0);
 }
 
 int tans_gpu_encode_matrix_begin(const void* w, int64_t R, int64_t C, int64_t S, int64_t Nc,
                                  int32_t pad, const uint32_t* enc_tab, const uint16_t* enc_next,
                                  int32_t log2L, void* workspace, int64_t workspace_bytes,
-                                 int64_t* offsets, uint16_t* states, void* sm, int32_t* status,
+                                 int64_t* offsets, uint16_t* states, void* sm, int64_t* result,
                                  void* stream) {
+    if (!result) return fail(TANS_EINVAL, "gpu_encode_matrix: null result");
     if (R <= 0 || C < 16 || S <= 0 || Nc <= 0 || Nc % 32 || Nc > 1024)
         return fail(TANS_EINVAL, "gpu_encode_matrix: need R > 0, C >= 16 and segments of at most "
                                  "1024 columns, a multiple of 32");
@@ -1031,7 +1058,7 @@ int tans_gpu_encode_matrix_begin(const void* w, int64_t R, int64_t C, int64_t S,
     const MatSrc src{(const uint8_t*)w, R, C, (int)(Rp / 16), (int)Nc,
                      (uint32_t)pad * 0x01010101u, nullptr, nullptr, 0, 0, false};
     return gpu_encode_begin(src, w, 4 * S * Rp, Nc / 4, enc_tab, enc_next, log2L, workspace,
-                            workspace_bytes, offsets, states, sm, status, stream, false);
+                            workspace_bytes, offsets, states, sm, nullptr, result, stream, false);
 }
 
 int tans_gpu_encode_finish(int64_t K, int64_t N, int32_t log2L, const void* workspace,
@@ -1044,7 +1071,7 @@ int tans_gpu_encode_packed_begin(const void* fp8, int64_t K, int64_t N, const ui
                                  int64_t workspace_bytes, int64_t* offsets, void* sm,
                                  int32_t* status, void* stream) {
     return gpu_encode_rows(fp8, K, N, enc_tab, enc_next, log2L, workspace, workspace_bytes,
-                            offsets, nullptr, sm, status, stream, true);
+                            offsets, nullptr, sm, status, nullptr, stream, true);
 }
 
 int tans_gpu_encode_packed_finish(int64_t K, int64_t N, int32_t log2L, const void* workspace,

@@ -33,6 +33,7 @@ EXPORTS = (
     "tans_gpu_encode_workspace",
     "tans_gpu_encode_begin",
     "tans_gpu_encode_finish",
+    "tans_gpu_encode_lanes_begin",
     "tans_gpu_encode_matrix_begin",
     "tans_gpu_encode_packed_begin",
     "tans_gpu_encode_packed_finish",
@@ -82,6 +83,8 @@ for _name, _args in {
     "tans_build_encode_table": [_P, _P, _I32, _I32, _P, _P],
     "tans_gpu_encode_workspace": [_I64, _I64, _I32, ctypes.POINTER(_I64)],
     "tans_gpu_encode_begin": [_P, _I64, _I64, _P, _P, _I32, _P, _I64, _P, _P, _P, _P, _P],
+    "tans_gpu_encode_lanes_begin": [_P, _I64, _I64, _I32, _P, _P, _I32, _P, _I64, _P, _P, _P, _P,
+                                    _P],
     "tans_gpu_encode_matrix_begin": [_P, _I64, _I64, _I64, _I64, _I32, _P, _P, _I32, _P, _I64,
                                      _P, _P, _P, _P, _P],
     "tans_gpu_encode_finish": [_I64, _I64, _I32, _P, _P, _P, _I64, _P],

@@ -344,10 +344,10 @@ def encode_matrix(w_fp8: torch.Tensor, exp_freqs, *, segments: int | None = None
         # the walk reads the lanes where they lie in W: no padded copy, no slab
         w = w_fp8.contiguous()
 
-        def begin(log2L, tab, nxt, ws, offsets, states, sm, status, stream):
+        def begin(log2L, tab, nxt, ws, offsets, states, sm, result, stream):
             return lib.tans_gpu_encode_matrix_begin(w.data_ptr(), R, C, S, Nc, pad, tab, nxt,
                                                     log2L, ws.data_ptr(), ws.numel(), offsets,
-                                                    states, sm, status, stream)
+                                                    states, sm, result, stream)
 
         enc = _encode_lanes_gpu(begin, 4 * S * Rp, Nc // 4, exp_freqs, alphabet, w.device, False)
     else:
@@ -373,10 +373,10 @@ _ENC_TABLES_MAX = 16
 
 
 def _encode_tables(exp_freqs, alphabet: str, dev: torch.device):
-    """(freqs, spread, enc_tab on dev, enc_next on dev) for a histogram.  The
+    """(freqs, spread, enc_tab, enc_next) on dev for a histogram.  The
     quantization costs about a millisecond of host time, so the tables of the
-    last few (histogram, alphabet, device) keys are kept; the numpy arrays
-    are read-only so a caller cannot change a cached entry."""
+    last few (histogram, alphabet, device) keys are kept; callers get copies
+    of freqs and spread."""
     h = np.ascontiguousarray(np.asarray(exp_freqs, dtype=np.float64))
     key = (alphabet, h.shape, h.tobytes(), str(dev))
     hit = _ENC_TABLES.get(key)
@@ -393,15 +393,15 @@ def _encode_tables(exp_freqs, alphabet: str, dev: torch.device):
                                       ctypes.c_void_p(enc_tab.ctypes.data),
                                       ctypes.c_void_p(enc_next.ctypes.data)),
           "encode_gpu")
-    freqs.setflags(write=False)
-    spread.setflags(write=False)
     with torch.cuda.device(dev):
-        tab_d = torch.from_numpy(enc_tab.view(np.int32)).to(dev)
-        next_d = torch.from_numpy(enc_next.view(np.int16)).to(dev)
+        # (copies from pageable memory: done when they return, so any stream
+        # may read the tables)
+        tables = tuple(torch.from_numpy(t).to(dev) for t in
+                       (freqs, spread, enc_tab.view(np.int32), enc_next.view(np.int16)))
     if len(_ENC_TABLES) >= _ENC_TABLES_MAX:
         _ENC_TABLES.pop(next(iter(_ENC_TABLES)))
-    _ENC_TABLES[key] = (freqs, spread, tab_d, next_d)
-    return _ENC_TABLES[key]
+    _ENC_TABLES[key] = tables
+    return tables
 
 
 def encode_gpu(fp8_bytes: torch.Tensor, exp_freqs, tile: int = 0, *, alphabet: str = "pair",
@@ -430,13 +430,10 @@ def encode_gpu(fp8_bytes: torch.Tensor, exp_freqs, tile: int = 0, *, alphabet: s
     if x.data_ptr() % 16:            # the kernels read 16-byte words
         x = x.clone()
 
-    def begin(log2L, tab, nxt, ws, offsets, states, sm, status, stream):
-        if packed and K:
-            return lib.tans_gpu_encode_packed_begin(x.data_ptr(), K, N, tab, nxt, log2L,
-                                                    ws.data_ptr(), ws.numel(), offsets, sm,
-                                                    status, stream)
-        return lib.tans_gpu_encode_begin(x.data_ptr(), K, N, tab, nxt, log2L, ws.data_ptr(),
-                                         ws.numel(), offsets, states, sm, status, stream)
+    def begin(log2L, tab, nxt, ws, offsets, states, sm, result, stream):
+        return lib.tans_gpu_encode_lanes_begin(x.data_ptr(), K, N, packed and K > 0, tab, nxt,
+                                               log2L, ws.data_ptr(), ws.numel(), offsets, states,
+                                               sm, result, stream)
 
     return _encode_lanes_gpu(begin, K, N, exp_freqs, alphabet, x.device, packed)
 
@@ -449,27 +446,32 @@ def _encode_lanes_gpu(begin, K: int, N: int, exp_freqs, alphabet: str, dev: torc
     log2L = ALPHABETS[alphabet][1].bit_length() - 1
     freqs, spread, tab_d, next_d = _encode_tables(exp_freqs, alphabet, dev)
     G = -(-K // TANS_LANES)
-    with torch.cuda.device(dev):
+    with _C._on(dev):
         ws_bytes = ctypes.c_int64()
         check(lib.tans_gpu_encode_workspace(K, N, log2L, ctypes.byref(ws_bytes)), "encode_gpu")
         ws = torch.empty(max(ws_bytes.value, 1), dtype=torch.uint8, device=dev)
         offsets = torch.empty(G + 1, dtype=torch.int64, device=dev)
         states = torch.empty(0 if packed else K, dtype=torch.uint16, device=dev)
         sm = torch.empty(((N + 15) // 16, K, 8), dtype=torch.uint8, device=dev)
-        status = torch.zeros(1, dtype=torch.int32, device=dev)
-        stream = torch.cuda.current_stream(dev).cuda_stream
+        # the length and the error mark come back in pinned memory that the
+        # scan writes: one wait for the stream, no copies or launches for it
+        result = torch.empty(2, dtype=torch.int64, device="cpu", pin_memory=True)
+        stream = torch.cuda.current_stream(dev)
         check(begin(log2L, tab_d.data_ptr(), next_d.data_ptr(), ws, offsets.data_ptr(),
-                    states.data_ptr(), sm.data_ptr(), status.data_ptr(), stream), "encode_gpu")
-        total, bad = (int(v) for v in torch.stack([offsets[G], status[0].to(torch.int64)]).tolist())
+                    states.data_ptr(), sm.data_ptr(), result.data_ptr(), stream.cuda_stream),
+              "encode_gpu")
+        # (device copies of the cached tables, made while the passes run)
+        freqs_d, spread_d = freqs.clone(), spread.clone()
+        partial = torch.empty(0, dtype=torch.uint8, device=dev)
+        stream.synchronize()
+        total, bad = result.tolist()
         if bad:
             raise RuntimeError("encode_gpu: data holds a symbol whose frequency is 0")
         comp = torch.empty((total + 256) * 4, dtype=torch.uint8, device=dev)
         finish = lib.tans_gpu_encode_packed_finish if packed and K else lib.tans_gpu_encode_finish
         check(finish(K, N, log2L, ws.data_ptr(), offsets.data_ptr(), comp.data_ptr(),
-                     comp.numel(), stream), "encode_gpu")
-    partial = torch.empty(0, dtype=torch.uint8, device=dev)
-    return (comp, states, offsets, partial, sm, torch.from_numpy(freqs.copy()).to(dev),
-            torch.from_numpy(spread.copy()).to(dev))
+                     comp.numel(), stream.cuda_stream), "encode_gpu")
+    return comp, states, offsets, partial, sm, freqs_d, spread_d
 
 
 @dataclasses.dataclass
