@@ -1646,12 +1646,23 @@ constexpr int kGemmMaxSegCols = 1024;                 // Nc limit
 constexpr int kGemmXStride = kGemmMaxSegCols + 16;    // bf16 per x stage row (32 bytes of pad)
 static_assert(kGemmMaxSegCols == kDecBlock, "one x stage column per thread");
 
-template <int SPS>
+constexpr int kFinWaves = 4;   // partial orders of the segment sum (gemm_finalize_kernel)
+
+// WHOLE: a workgroup holds every segment of its row groups, one wave per
+// segment and two row groups, and x in all columns of the matrix: batch row b
+// at xs + b * whole_x_stride(S * Nc), zero past C.
+constexpr int kWholeXBytes = 24 * 1024 - 64;
+
+constexpr int whole_x_stride(int cols) { return (cols + 127) / 128 * 128 + 16; }   // bf16
+
+template <int SPS, bool WHOLE>
 struct GemmSmem {
     DecSmem<SPS, kGemmChains> dec;
-    alignas(16) __bf16 xs[kGemmMaxBatch][kGemmXStride];   // x columns of the segment
+    // x columns of the segment, kGemmXStride per batch row (or of the matrix)
+    alignas(16) __bf16 xs[WHOLE ? kWholeXBytes / 2 : kGemmMaxBatch * kGemmXStride];
 };
-static_assert(sizeof(GemmSmem<2>) <= 160 * 1024 && sizeof(GemmSmem<1>) <= 160 * 1024,
+static_assert(sizeof(GemmSmem<2, false>) <= 160 * 1024 && sizeof(GemmSmem<1, false>) <= 160 * 1024 &&
+                  sizeof(GemmSmem<2, true>) <= 160 * 1024 && sizeof(GemmSmem<1, true>) <= 160 * 1024,
               "the GEMM workgroup's LDS fits one CU");
 
 // Four bf16 pairs from 4 FP8 words (exact: every E4M3FN value is a bf16).
@@ -1741,54 +1752,75 @@ struct GemmWave {
     }
 };
 
+__device__ __forceinline__ uint16_t bf16_rne(float f) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, f);
+    if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (uint16_t)((u >> 16) | 0x40u);   // quiet NaN
+    return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
+}
+
 // Grid: S * row_blocks workgroups; block (s, rb) decodes the 2 `waves` row
 // groups from 2 `waves` rb on of segment s (16 rows each).  R: rows, Rp: rows
 // padded to 64, C: columns, Nc: columns per segment, NB: batch rows.
-template <int SPS>
+//
+// WHOLE: grid of row blocks alone; a workgroup takes `waves` / S pairs of row
+// groups in all S segments (wave w: pair w / S, segment w % S), adds the
+// segments' sums in LDS in gemm_finalize_kernel's order and writes y: no
+// partial sums in memory, no second kernel.
+template <int SPS, bool WHOLE>
 __global__ __launch_bounds__(kDecBlock) void gemm_fused_kernel(
     const uint32_t* __restrict__ comp, int64_t words, const int64_t* __restrict__ off,
     const uint16_t* __restrict__ st, const v2u* __restrict__ sm, const v2u* __restrict__ table,
     int64_t Rp, int64_t C, int S, int Nc, int row_blocks, int waves, const uint16_t* __restrict__ x, int NB,
-    float* __restrict__ ws) {
+    float* __restrict__ ws, int64_t R, float scale, uint16_t* __restrict__ y) {
     constexpr uint32_t L = Alpha<SPS>::L;
     constexpr int CH = kGemmChains;
-    __shared__ GemmSmem<SPS> smem;
-    const int s = (int)(blockIdx.x / (unsigned)row_blocks);
-    const int rb = (int)(blockIdx.x % (unsigned)row_blocks);
+    __shared__ GemmSmem<SPS, WHOLE> smem;
+    const int lane = threadIdx.x & (kLanes - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int s = WHOLE ? wave % S : (int)(blockIdx.x / (unsigned)row_blocks);
+    const int rb = WHOLE ? (int)blockIdx.x : (int)(blockIdx.x % (unsigned)row_blocks);
     const int64_t n_rg = Rp / kGemmGroupRows;               // row groups per segment
     // issue the x, table, stream, state and sign/mantissa loads together
     // (as in fused_add_kernel); a wave past the last row group loads the
     // last one and leaves after the barrier.  Thread i stages column i of
     // the segment for every batch row (zero past the segment, the matrix
     // or the batch).
+    // (WHOLE: thread i takes columns i, i + 1024, .. of the matrix, written
+    // as they come)
     const int xc = (int)threadIdx.x;
     const int64_t xcol = (int64_t)s * Nc + xc;
     const bool x_in = xc < Nc && xcol < C;
     uint16_t xv[kGemmMaxBatch];
-    #pragma unroll
-    for (int b = 0; b < kGemmMaxBatch; b++)
-        xv[b] = (b < NB && x_in) ? x[(int64_t)b * C + xcol] : (uint16_t)0;
+    if constexpr (!WHOLE) {
+        #pragma unroll
+        for (int b = 0; b < kGemmMaxBatch; b++)
+            xv[b] = (b < NB && x_in) ? x[(int64_t)b * C + xcol] : (uint16_t)0;
+    }
     TableRegs<L> tr;
     table_fetch<L>(tr, table);
-    const int lane = threadIdx.x & (kLanes - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
     // the first `waves` waves decode, as in fused_add_kernel
-    const int64_t rg0 = wave < waves ? ((int64_t)rb * waves + wave) * CH : n_rg;
-    const bool live = rg0 < n_rg;   // wave-uniform
-    const int64_t rg_left = n_rg - (int64_t)rb * waves * CH;
+    const int pairs = WHOLE ? waves / S : waves;   // row group pairs per workgroup
+    const int pair = WHOLE ? wave / S : wave;
+    const int64_t rg0 = ((int64_t)rb * pairs + pair) * CH;
+    const bool live = wave < waves && rg0 < n_rg;   // wave-uniform
+    const int64_t rg_left = n_rg - (int64_t)rb * pairs * CH;
+    const int xstride = WHOLE ? whole_x_stride(S * Nc) : kGemmXStride;
     GemmWave<SPS> w;
     w.progress = &smem.dec.progress;
-    w.live = (uint32_t)(rg_left >= (int64_t)waves * CH ? waves : (rg_left + CH - 1) / CH);
+    w.live = (uint32_t)(rg_left >= (int64_t)pairs * CH ? pairs : (rg_left + CH - 1) / CH);
+    if constexpr (WHOLE) w.live *= (uint32_t)S;
     w.lane = lane;
     w.q = lane >> 4;
     w.tbl = smem.dec.tbl;
-    w.xrow = &smem.xs[lane & (kGemmMaxBatch - 1)][0];
+    // (WHOLE stages the batch's rows alone: lanes past it read row 0)
+    w.xrow = WHOLE ? smem.xs + ((lane & 15) < NB ? lane & 15 : 0) * xstride + s * Nc
+                   : smem.xs + (lane & (kGemmMaxBatch - 1)) * xstride;
     w.sm_stride = (int64_t)S * n_rg * kLanes * 8;            // lanes: S * n_rg * 64
     const int per_lane = Nc / 4;                              // elements per lane (8 | per_lane)
     const int rag = per_lane % kTile;                         // 0 or 8
     w.n_tiles = per_lane / kTile + (rag ? 1 : 0);
     last_tile_sched<SPS>(per_lane / SPS, w.n_tiles, w.last_segs, w.fin_pos);
-    w.sm_bytes = live ? kLanes * 8u : 0u;
+    w.sm_bytes = kLanes * 8u;
     Seg first[CH][kSlots];
     uint16_t st0[CH];
     // a wave with one row group left repeats it as its second chain and
@@ -1798,7 +1830,7 @@ __global__ __launch_bounds__(kDecBlock) void gemm_fused_kernel(
     for (int j = 0; j < CH; j++) {
         const int64_t g = (int64_t)s * n_rg + (rg0 + j < n_rg ? rg0 + j : n_rg - 1);
         os[j] = off[g];
-        oe[j] = live ? off[g + 1] : os[j];   // a wave without work reads nothing
+        oe[j] = off[g + 1];
     }
     #pragma unroll
     for (int j = 0; j < CH; j++) {
@@ -1822,39 +1854,87 @@ __global__ __launch_bounds__(kDecBlock) void gemm_fused_kernel(
         w.pf[j] = row + tn * w.sm_stride;
         w.acc[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    #pragma unroll
-    for (int b = 0; b < kGemmMaxBatch; b++)
-        smem.xs[b][xc] = __builtin_bit_cast(__bf16, xv[b]);
-    if (xc < kGemmXStride - kGemmMaxSegCols) {
+    if constexpr (WHOLE) {
+        // four columns of every batch row at a time, loaded together
+        for (int c0 = xc; c0 < xstride; c0 += 4 * kDecBlock) {
+            for (int b = 0; b < NB; b++) {
+                uint16_t v[4];
+                #pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int c = c0 + i * kDecBlock;
+                    v[i] = c < C ? x[(int64_t)b * C + c] : (uint16_t)0;
+                }
+                #pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (c0 + i * kDecBlock < xstride)
+                        smem.xs[b * xstride + c0 + i * kDecBlock] = __builtin_bit_cast(__bf16, v[i]);
+            }
+        }
+    } else {
         #pragma unroll
         for (int b = 0; b < kGemmMaxBatch; b++)
-            smem.xs[b][kGemmMaxSegCols + xc] = __builtin_bit_cast(__bf16, (uint16_t)0);
+            smem.xs[b * kGemmXStride + xc] = __builtin_bit_cast(__bf16, xv[b]);
+        if (xc < kGemmXStride - kGemmMaxSegCols) {
+            #pragma unroll
+            for (int b = 0; b < kGemmMaxBatch; b++)
+                smem.xs[b * kGemmXStride + kGemmMaxSegCols + xc] =
+                    __builtin_bit_cast(__bf16, (uint16_t)0);
+        }
     }
     table_store<L>(smem.dec.tbl, tr);
     if (threadIdx.x == 0) smem.dec.init();
     __syncthreads();
-    if (!live) return;
-    #pragma unroll
-    for (int j = 0; j < CH; j++) {
-        feed_commit<kLazySegs>(w.ch.f[j], lane, first[j], w.ch.p[j]);
-        lane_init(w.ch.l[j], w.ch.f[j], lane, kLanes, st0[j], L, smem.dec.sink_off());
+    if (!WHOLE && !live) return;
+    if (live) {
+        #pragma unroll
+        for (int j = 0; j < CH; j++) {
+            feed_commit<kLazySegs>(w.ch.f[j], lane, first[j], w.ch.p[j]);
+            lane_init(w.ch.l[j], w.ch.f[j], lane, kLanes, st0[j], L, smem.dec.sink_off());
+        }
+        w.run(rag ? rag : kTile);
     }
-    w.run(rag ? rag : kTile);
     const int bn = lane & 15;   // the batch row of this lane's sums
-    if (bn >= NB) return;
-    #pragma unroll
-    for (int j = 0; j < CH; j++) {
-        if (rg0 + j >= n_rg) break;
-        const int64_t r = (rg0 + j) * kGemmGroupRows + 4 * w.q;
-        *reinterpret_cast<v4f*>(ws + ((int64_t)s * NB + bn) * Rp + r) = w.acc[j];
+    if constexpr (WHOLE) {
+        // the wave's sums go to its own rings (it has read the last of them):
+        // lane j's four of chain c at [c][j]
+        v4f* part = reinterpret_cast<v4f*>(&smem.dec.rings[wave][0][0]);
+        static_assert(CH * kLanes * sizeof(v4f) <= sizeof(smem.dec.rings[0]), "a wave's sums fit");
+        asm volatile("" ::: "memory");
+        if (live) {
+            #pragma unroll
+            for (int j = 0; j < CH; j++) part[j * kLanes + lane] = w.acc[j];
+        }
+        __syncthreads();
+        // rows of the workgroup, consecutive per thread, one batch row after
+        // the other: segments s, s + 4, .. of each in turn, then the four sums
+        const int rows = (int)(rg_left < (int64_t)pairs * CH ? rg_left : pairs * CH) * kGemmGroupRows;
+        const int64_t row0 = (int64_t)rb * pairs * CH * kGemmGroupRows;
+        for (int t = (int)threadIdx.x; t < rows * NB; t += kDecBlock) {
+            const int b = t / rows, r = t % rows;
+            const int rg = r / kGemmGroupRows, rr = r % kGemmGroupRows;
+            const int at = ((rg % CH) * kLanes + (rr / 4) * 16 + b) * 4 + rr % 4;
+            float sum = 0.0f;
+            #pragma unroll
+            for (int f = 0; f < kFinWaves; f++) {
+                float a = 0.0f;
+                for (int sg = f; sg < S; sg += kFinWaves)
+                    a += reinterpret_cast<const float*>(
+                        &smem.dec.rings[(rg / CH) * S + sg][0][0])[at];
+                sum = f ? sum + a : a;
+            }
+            if (row0 + r < R) y[(int64_t)b * R + row0 + r] = bf16_rne(sum * scale);
+        }
+    } else {
+        if (bn >= NB) return;
+        #pragma unroll
+        for (int j = 0; j < CH; j++) {
+            if (rg0 + j >= n_rg) break;
+            const int64_t r = (rg0 + j) * kGemmGroupRows + 4 * w.q;
+            *reinterpret_cast<v4f*>(ws + ((int64_t)s * NB + bn) * Rp + r) = w.acc[j];
+        }
     }
 }
 
-__device__ __forceinline__ uint16_t bf16_rne(float f) {
-    const uint32_t u = __builtin_bit_cast(uint32_t, f);
-    if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (uint16_t)((u >> 16) | 0x40u);   // quiet NaN
-    return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-}
 
 // y[b][r] = bf16(scale * sum over s of ws[s][b][r]).  A block of 4 waves
 // takes 64 consecutive outputs of one batch row: wave w sums segments
@@ -1863,7 +1943,6 @@ __device__ __forceinline__ uint16_t bf16_rne(float f) {
 // wave issues the loads of kFinBatch segments before it adds any of them,
 // so a call pays one memory round trip per kFinBatch segments instead of
 // one per segment.
-constexpr int kFinWaves = 4;
 constexpr int kFinBatch = 8;
 
 __global__ __launch_bounds__(kFinWaves * kLanes) void gemm_finalize_kernel(
@@ -2650,9 +2729,20 @@ int gemm_fused_launch(const void* comp, int64_t comp_bytes, const int64_t* offse
     const int cus = cu_count();
     if (cus <= 0) return fail(TANS_EHIP, "gemm_fused: cannot query the device's CU count");
     const int64_t pairs = (n_rg + kGemmChains - 1) / kGemmChains;
-    const int waves = spread_waves(pairs, (int)std::max<int64_t>(1, cus / S));
-    const int64_t row_blocks = (pairs + waves - 1) / waves;
-    const int64_t blocks = S * row_blocks;
+    // Every segment of a row group in one workgroup (WHOLE), where a wave per
+    // segment, x in all columns and a single round of workgroups fit: as many
+    // waves per CU as the other grid, and no second kernel.  Two kernels
+    // against one, per call: 2176 x 1280 at B = 3 (nibble) 17.4 -> 14.4 us (11.4
+    // + 3.9 us of kernels -> 13.5), 4096 x 4096 at B = 1 17.6 -> 14.7 us, 8192 x
+    // 1024 at B = 8 17.9 -> 14.8 us.  (17408 x 5120 would need 272 workgroups,
+    // two rounds; 5120 x 17408 has 25 segments.)
+    const int64_t whole_pairs = (pairs + cus - 1) / cus;
+    const bool whole = S * whole_pairs <= kDecWaves &&
+                       B * whole_x_stride((int)std::min<int64_t>(S * Nc, INT16_MAX)) * 2 <= kWholeXBytes;
+    const int waves = whole ? (int)(S * whole_pairs)
+                            : spread_waves(pairs, (int)std::max<int64_t>(1, cus / S));
+    const int64_t row_blocks = (pairs + (whole ? whole_pairs : waves) - 1) / (whole ? whole_pairs : waves);
+    const int64_t blocks = whole ? row_blocks : S * row_blocks;
     if (!grid_fits(blocks, kDecBlock) || !grid_fits(B * (Rp / kLanes), kFinWaves * kLanes))
         return fail(TANS_EINVAL, "gemm_fused: matrix too large");
     hipStream_t st = (hipStream_t)stream;
@@ -2660,9 +2750,13 @@ int gemm_fused_launch(const void* comp, int64_t comp_bytes, const int64_t* offse
         hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kDecBlock), 0, st,
                            (const uint32_t*)comp, comp_bytes / 4, offsets, states, (const v2u*)sm,
                            (const v2u*)table, Rp, C, (int)S, (int)Nc, (int)row_blocks, waves,
-                           (const uint16_t*)x, (int)B, (float*)workspace);
+                           (const uint16_t*)x, (int)B, (float*)workspace, R, scale, (uint16_t*)y);
     };
-    if (sps == 2) launch(gemm_fused_kernel<2>); else launch(gemm_fused_kernel<1>);
+    if (whole) {
+        if (sps == 2) launch(gemm_fused_kernel<2, true>); else launch(gemm_fused_kernel<1, true>);
+        return hip_check(hipGetLastError(), "gemm_fused_kernel launch");
+    }
+    if (sps == 2) launch(gemm_fused_kernel<2, false>); else launch(gemm_fused_kernel<1, false>);
     int rc = hip_check(hipGetLastError(), "gemm_fused_kernel launch");
     if (rc != TANS_OK) return rc;
     hipLaunchKernelGGL(gemm_finalize_kernel, dim3((unsigned)(B * (Rp / kLanes))),

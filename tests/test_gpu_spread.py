@@ -65,3 +65,25 @@ def test_gemm_row_groups_spread_over_cus(R, rows, cols, segments):
     same_nan = torch.isnan(y) == torch.isnan(y_raw)
     ok = (y - y_raw).abs() <= 2.0 ** -7 * y_raw.abs() + cols * 2.0 ** -23 * mag
     assert bool((same_nan & (ok | torch.isnan(y_raw))).all())
+
+
+# one workgroup per row block holding every segment (B small enough for x in
+# LDS) against one workgroup per segment and the separate sum (B = 8): the
+# same products in the same order, so equal to the bit.  Segments 1, 5, 8 and
+# 16, half tiles (width 32 mod 64), one to three pairs of row groups per
+# workgroup, ragged rows and columns, an odd pair count
+@pytest.mark.parametrize("alphabet", ["pair", "nibble"])
+@pytest.mark.parametrize("rows,cols,segments,batch", [(200, 2040, 8, 5), (48, 4096, 16, 2),
+                                                      (16, 1555, 5, 6), (1000, 1540, 16, 7),
+                                                      (17000, 1600, 5, 3), (8300, 1537, 7, 1)])
+def test_gemm_whole_rows_equal_the_segment_sums(R, alphabet, rows, cols, segments, batch):
+    from rans_vectoradd import tans_codec as T
+    _say(f"case: gemm whole rows {rows}x{cols} S={segments} B={batch} {alphabet}")
+    w = _bytes(R, rows * cols, rows + cols).view(rows, cols)
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    x = torch.randn(8, cols, generator=g, device="cuda").to(torch.bfloat16)
+    m = T.encode_matrix(w, torch.tensor(R.QWEN3_14B_FP8_EXP), segments=segments, alphabet=alphabet)
+    tbl = m.decode_table().cuda()
+    y8 = R.fp8_gemm_fused_tans(m, tbl, x, 2.0 ** -9)
+    y = R.fp8_gemm_fused_tans(m, tbl, x[:batch].contiguous(), 2.0 ** -9)
+    assert torch.equal(y.view(torch.int16), y8[:batch].view(torch.int16))
