@@ -323,6 +323,8 @@ constexpr int kMirrorWords = kLanes;
 constexpr int kRingAlloc = kRingWords + kMirrorWords;
 constexpr int kDecWaves = 16;              // waves per workgroup
 constexpr int kSmAhead = 4;                // sign/mantissa rows are loaded this many tiles ahead
+constexpr int kLowWaves = 4;               // ... where every wave gets a SIMD to itself
+constexpr int kMidWaves = 8;               // ... where two waves share a SIMD
 constexpr int kDecBlock = kDecWaves * kLanes;
 // At most kChecksPerStage * 64 words are handed out per stage.  A segment is
 // fetched once the one kSlots earlier in its slot is consumed; it can be
@@ -617,35 +619,35 @@ __device__ __forceinline__ void compose8(uint32_t ex_lo, uint32_t ex_hi, uint32_
 // bits than the refill schedule allows (nb > 10 in a 2^11-state table), are
 // replaced by a harmless one, so a malformed table gives wrong bytes, never
 // an out-of-range LDS access.
-template <uint32_t L>
+template <uint32_t L, int T = kDecBlock>   // T: threads of the workgroup
 struct TableRegs {
-    static_assert(L % kDecBlock == 0, "the table is split evenly over the workgroup");
-    v2u e[L / kDecBlock];
+    static_assert(L % T == 0, "the table is split evenly over the workgroup");
+    v2u e[L / T];
 };
 
-template <uint32_t L>
-__device__ __forceinline__ void table_fetch(TableRegs<L>& r, const v2u* __restrict__ table) {
+template <uint32_t L, int T>
+__device__ __forceinline__ void table_fetch(TableRegs<L, T>& r, const v2u* __restrict__ table) {
     #pragma unroll
-    for (uint32_t k = 0; k < L / kDecBlock; k++) r.e[k] = table[threadIdx.x + k * kDecBlock];
+    for (uint32_t k = 0; k < L / T; k++) r.e[k] = table[threadIdx.x + k * T];
 }
 
 // PACKED: the entries of the packed-layout decoders, whose word0 keeps nb
 // in bits 4:0 and moves the two exponents 8 bits up (bits 22:19 and
 // 30:27), so that bits 15:0 of a sum of word0s are the sum of their nb.
-template <uint32_t L, bool PACKED = false>
-__device__ __forceinline__ void table_store(v2u* lds, const TableRegs<L>& r) {
+template <uint32_t L, bool PACKED = false, int T>
+__device__ __forceinline__ void table_store(v2u* lds, const TableRegs<L, T>& r) {
     constexpr uint32_t log2L = 31 - __builtin_clz(L);
     constexpr uint32_t max_nb =
         log2L == tans_sched::kTripleLog2L ? tans_sched::kTripleMaxNb : log2L;
     #pragma unroll
-    for (uint32_t k = 0; k < L / kDecBlock; k++) {
+    for (uint32_t k = 0; k < L / T; k++) {
         v2u e = r.e[k];
         const uint32_t nb = e.x & 0xFFu;
         const uint32_t base = e.y >> 3;
         if (nb > max_nb || (e.x >> 27) != nb || (e.y & 7u) || base + (1u << nb) > L)
             e = v2u{e.x & 0x07FFFF00u, 0u};
         if constexpr (PACKED) e.x = (e.x & 0x1Fu) | ((e.x & 0x007FF800u) << 8);
-        lds[threadIdx.x + k * kDecBlock] = e;
+        lds[threadIdx.x + k * T] = e;
     }
 }
 
@@ -867,10 +869,10 @@ __device__ __forceinline__ void last_tile_sched(int64_t S, int n_tiles, int& las
 
 // LDS of a decoder workgroup.  The table comes first so that its entries'
 // byte offsets are their LDS addresses.
-template <int SPS, int C>
+template <int SPS, int C, int W = kDecWaves>   // W: waves of the workgroup
 struct DecSmem {
     v2u tbl[Alpha<SPS>::L];
-    uint32_t rings[kDecWaves][C][kRingAlloc];
+    uint32_t rings[W][C][kRingAlloc];
     uint32_t progress;   // tiles finished by all waves of the workgroup
     v2u sink;            // the table entry of lanes out of range (lane_init)
 
@@ -922,11 +924,12 @@ struct Chains {
 // table, and its bytes are discarded); fin_pos sets the final check
 // (check_last).  RESIDENT: the streams were loaded whole at their start
 // (feed_commit<NSEG>), so no stage fetches.
-template <int SPS, int C, bool LAST, bool RESIDENT = false>
+// beside: independent work put among the first stage's steps, where it can
+// issue while they wait on LDS.
+template <int SPS, int C, bool LAST, bool RESIDENT = false, class Beside>
 __device__ __forceinline__ void dec_tile(Chains<C>& ch, const v2u* __restrict__ tbl, int lane,
-                                         uint32_t (&ex)[C][4],
-                                         int last_segs = Alpha<SPS>::kSegsPerTile,
-                                         uint32_t fin_pos = Alpha<SPS>::kFinPosFullTile) {
+                                         uint32_t (&ex)[C][4], int last_segs, uint32_t fin_pos,
+                                         Beside&& beside) {
     using A = Alpha<SPS>;
     #pragma unroll
     for (int c = 0; c < C; c++) ch.l[c].q &= 0xF800001Fu;
@@ -936,6 +939,7 @@ __device__ __forceinline__ void dec_tile(Chains<C>& ch, const v2u* __restrict__ 
             #pragma unroll
             for (int c = 0; c < C; c++) feed_stage(ch.f[c], ch.p[c], lane);
         }
+        if constexpr (h == 0) beside();
         uint32_t e[C][8];
         static_for<0, A::kSegsPerStage>([&](auto Q) {
             constexpr int q = decltype(Q)::value;
@@ -974,6 +978,14 @@ __device__ __forceinline__ void dec_tile(Chains<C>& ch, const v2u* __restrict__ 
             }
         }
     });
+}
+
+template <int SPS, int C, bool LAST, bool RESIDENT = false>
+__device__ __forceinline__ void dec_tile(Chains<C>& ch, const v2u* __restrict__ tbl, int lane,
+                                         uint32_t (&ex)[C][4],
+                                         int last_segs = Alpha<SPS>::kSegsPerTile,
+                                         uint32_t fin_pos = Alpha<SPS>::kFinPosFullTile) {
+    dec_tile<SPS, C, LAST, RESIDENT>(ch, tbl, lane, ex, last_segs, fin_pos, [] {});
 }
 
 // ---------------------------------------------------------------------
@@ -1016,6 +1028,62 @@ struct FusedWave {
         if constexpr (PACKED) pk_tile<C, P == 0>(pk, preg, tbl, ex);
         else dec_tile<SPS, C, LAST, RES>(ch, tbl, lane, ex);
         pace(progress, lane, (uint32_t)(base + t), live);
+        finish<P>(t, ex);
+    }
+
+    // Decode tile t into ex while tile t - 1 (exponents in done) is finished.
+    template <int P, bool LAST>
+    __device__ __forceinline__ void overlapped(int t, uint32_t (&ex)[C][4],
+                                               const uint32_t (&done)[C][4]) {
+        dec_tile<SPS, C, LAST, RES>(ch, tbl, lane, ex, Alpha<SPS>::kSegsPerTile,
+                                    Alpha<SPS>::kFinPosFullTile,
+                                    [&] { finish<(P + kSmAhead - 1) % kSmAhead>(t - 1, done); });
+    }
+
+    // All tiles of a stream of n_tiles >= 2, each finished beside the next.
+    __device__ __forceinline__ void run_overlapped() {
+        static_assert(kSmAhead == 4 && !PACKED, "unrolled for kSmAhead == 4");
+        uint32_t a[C][4], b[C][4];
+        dec_tile<SPS, C, false, RES>(ch, tbl, lane, a);
+        const int body = n_tiles - 1;
+        int t = 1;
+        for (; t + 3 < body; t += 4) {
+            overlapped<1, false>(t, b, a);
+            overlapped<2, false>(t + 1, a, b);
+            overlapped<3, false>(t + 2, b, a);
+            overlapped<0, false>(t + 3, a, b);
+        }
+        // tiles t .. body, one to four of them (t mod 4 = 1)
+        switch (body - t) {
+            case 0:
+                overlapped<1, true>(t, b, a);
+                finish<1>(t, b);
+                break;
+            case 1:
+                overlapped<1, false>(t, b, a);
+                overlapped<2, true>(t + 1, a, b);
+                finish<2>(t + 1, a);
+                break;
+            case 2:
+                overlapped<1, false>(t, b, a);
+                overlapped<2, false>(t + 1, a, b);
+                overlapped<3, true>(t + 2, b, a);
+                finish<3>(t + 2, b);
+                break;
+            default:
+                overlapped<1, false>(t, b, a);
+                overlapped<2, false>(t + 1, a, b);
+                overlapped<3, false>(t + 2, b, a);
+                overlapped<0, true>(t + 3, a, b);
+                finish<0>(t + 3, a);
+                break;
+        }
+    }
+
+    // Compose, add and store tile t from its exponents, and load the
+    // sign/mantissa words four tiles ahead.
+    template <int P>
+    __device__ __forceinline__ void finish(int t, const uint32_t (&ex)[C][4]) {
         #pragma unroll
         for (int g = 0; g < G; g++) {
             uint32_t wa[4], wb[4];
@@ -1049,8 +1117,16 @@ struct FusedWave {
     }
 };
 
-template <int SPS, int G, int FIRST>
-__global__ __launch_bounds__(kDecBlock) void fused_add_kernel(
+// W: waves of a workgroup.  W < kDecWaves (streams of any length, one or two
+// waves per SIMD): each tile's compose, add and store are put among the next
+// tile's decode steps.  A wave alone on its SIMD waits on LDS for most of a
+// tile, and about 100 of the tile's 171 VALU instructions then issue in those
+// waits (106 VGPRs).  1024 per lane, pair: 256 groups 62 -> 50 us, 2048 groups
+// (8 waves per CU) 78 -> 72 us; 10007 x 1008 nibble 90 -> 73 us.  With 16 waves
+// the other waves fill the waits already, and the wider live ranges cost 1-2%.
+// 8-wave workgroups are slower than 4-wave ones where 4 are enough (53 us).
+template <int SPS, int G, int FIRST, int W>
+__global__ __launch_bounds__(W * kLanes) void fused_add_kernel(
     const uint32_t* __restrict__ a_comp, int64_t a_words, const int64_t* __restrict__ a_off,
     const uint16_t* __restrict__ a_st, const v2u* __restrict__ a_sm,
     const uint32_t* __restrict__ b_comp, int64_t b_words, const int64_t* __restrict__ b_off,
@@ -1058,13 +1134,15 @@ __global__ __launch_bounds__(kDecBlock) void fused_add_kernel(
     const v2u* __restrict__ table, int64_t K, int n_tiles, int waves, v4u* __restrict__ out) {
     constexpr uint32_t L = Alpha<SPS>::L;
     constexpr int C = 2 * G;
-    __shared__ DecSmem<SPS, C> smem;
+    __shared__ DecSmem<SPS, C, W> smem;
+    constexpr bool LOW = W < kDecWaves;
+    static_assert(!LOW || FIRST == 0, "streams of any length");
     v2u* tbl = smem.tbl;
     // issue the table, stream, state and sign/mantissa loads together; a
     // wave past the last group loads the last one and leaves after the
     // barrier
-    TableRegs<L> tr;
-    table_fetch<L>(tr, table);
+    TableRegs<L, W * kLanes> tr;
+    table_fetch(tr, table);
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
     const int64_t n_groups = (K + kLanes - 1) / kLanes;
@@ -1273,6 +1351,13 @@ __global__ __launch_bounds__(kDecBlock) void fused_add_kernel(
             next_offsets(g0 + 2 * grid_groups);
         }
         w.base = done;
+        if constexpr (LOW) {
+            w.run_overlapped();
+            g0 += grid_groups;
+            if (g0 >= n_groups) break;
+            setup(g0, false);
+            continue;
+        }
         // the first n_tiles - 1 tiles four per iteration, then the last one,
         // which ends the streams (its variant chosen by tile mod 4)
         const int body = n_tiles - 1;
@@ -1506,7 +1591,7 @@ __global__ __launch_bounds__(kDecBlock) void decode_kernel(
     v2u* tbl = smem.tbl;
     // loads issued together, as in fused_add_kernel
     TableRegs<L> tr;
-    table_fetch<L>(tr, table);
+    table_fetch(tr, table);
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
     const int64_t n_groups = (K + kLanes - 1) / kLanes;
@@ -1797,7 +1882,7 @@ __global__ __launch_bounds__(kDecBlock) void gemm_fused_kernel(
             xv[b] = (b < NB && x_in) ? x[(int64_t)b * C + xcol] : (uint16_t)0;
     }
     TableRegs<L> tr;
-    table_fetch<L>(tr, table);
+    table_fetch(tr, table);
     // the first `waves` waves decode, as in fused_add_kernel
     const int pairs = WHOLE ? waves / S : waves;   // row group pairs per workgroup
     const int pair = WHOLE ? wave / S : wave;
@@ -2420,8 +2505,9 @@ constexpr int kFusedGroups = 1;   // groups per wave in the fused kernel
 // us instead of 1.9, so pieces that do not fill the chip are spread over all
 // CUs rather than packed into a few.  Fused add, 1024 per lane, 16 waves per
 // workgroup against this rule: 256 groups 91.6 -> 61.6 us, 1024 groups 93.8
-// -> 67 us, 2048 groups 96.4 -> 78 us, 5000 groups (two rounds of 10 waves
-// per CU, not 16 and then 16 on a fifth of the CUs) 210 -> 180 us.
+// -> 67 us, 2048 groups 96.4 -> 78 us (with the kernels for few waves, see
+// fused_add_kernel, 50, 54 and 70 us), 5000 groups (two rounds of 10 waves per
+// CU, not 16 and then 16 on a fifth of the CUs) 210 -> 180 us.
 int spread_waves(int64_t units, int cus) {
     const int64_t per_round = (int64_t)cus * kDecWaves;
     const int64_t rounds = (units + per_round - 1) / per_round;
@@ -2578,13 +2664,14 @@ int tans_fp8_vecadd_fused(const void* a_comp, int64_t a_comp_bytes, const int64_
     const int waves = spread_waves(groups, cus);
     const int64_t blocks = std::min<int64_t>((groups + waves - 1) / waves, cus);
     const int n_tiles = (int)(N / kTile);
-#define TANS_LAUNCH_FUSED(S, FIRST)                                                               \
-    hipLaunchKernelGGL((fused_add_kernel<S, kFusedGroups, FIRST>), dim3((unsigned)blocks),       \
-                       dim3(kDecBlock), 0, (hipStream_t)stream, (const uint32_t*)a_comp,         \
+#define TANS_LAUNCH_FUSED_W(S, FIRST, W)                                                          \
+    hipLaunchKernelGGL((fused_add_kernel<S, kFusedGroups, FIRST, W>), dim3((unsigned)blocks),    \
+                       dim3(W * kLanes), 0, (hipStream_t)stream, (const uint32_t*)a_comp,        \
                        a_comp_bytes / 4, a_offsets, a_states, (const v2u*)a_sm,                  \
                        (const uint32_t*)b_comp, b_comp_bytes / 4, b_offsets, b_states,           \
                        (const v2u*)b_sm, (const v2u*)table, K, n_tiles, waves,      \
                        (v4u*)out)
+#define TANS_LAUNCH_FUSED(S, FIRST) TANS_LAUNCH_FUSED_W(S, FIRST, kDecWaves)
     // streams that fit the ring are loaded whole at their start
     if (packed) {
         switch (n_tiles) {
@@ -2596,13 +2683,18 @@ int tans_fp8_vecadd_fused(const void* a_comp, int64_t a_comp_bytes, const int64_
     } else if (sps == 2) {
         if (n_tiles == 1) TANS_LAUNCH_FUSED(2, Alpha<2>::kOneTileSegs);
         else if (n_tiles <= Alpha<2>::kResidentTiles) TANS_LAUNCH_FUSED(2, kSlots);
+        else if (waves <= kLowWaves) TANS_LAUNCH_FUSED_W(2, 0, kLowWaves);
+        else if (waves <= kMidWaves) TANS_LAUNCH_FUSED_W(2, 0, kMidWaves);
         else TANS_LAUNCH_FUSED(2, 0);
     } else {
         if (n_tiles == 1) TANS_LAUNCH_FUSED(1, Alpha<1>::kOneTileSegs);
         else if (n_tiles <= Alpha<1>::kResidentTiles) TANS_LAUNCH_FUSED(1, kSlots);
+        else if (waves <= kLowWaves) TANS_LAUNCH_FUSED_W(1, 0, kLowWaves);
+        else if (waves <= kMidWaves) TANS_LAUNCH_FUSED_W(1, 0, kMidWaves);
         else TANS_LAUNCH_FUSED(1, 0);
     }
 #undef TANS_LAUNCH_FUSED
+#undef TANS_LAUNCH_FUSED_W
     return hip_check(hipGetLastError(), "fused_add_kernel launch");
 }
 

@@ -27,9 +27,14 @@ def _bytes(R, n, seed):
 
 # groups of 64 lanes against 256 CUs: one, fewer than CUs, one more than CUs
 # (two waves on one), a whole round of 16 and one group more or less, two
-# rounds of 10 waves; the lane count ragged in each
-@pytest.mark.parametrize("alphabet,N", [("pair", 16), ("pair", 48), ("pair", 80), ("nibble", 48)])
-@pytest.mark.parametrize("groups", [1, 100, 257, 4095, 4096, 4097, 5000])
+# rounds of 10 waves; the lane count ragged in each.  Up to 4 and up to 8
+# waves per CU have kernels of their own for streams of any length (1500
+# groups: 6 waves), whose tiles overlap: every tile count mod 4
+@pytest.mark.parametrize("alphabet,N", [("pair", 16), ("pair", 48), ("pair", 80), ("pair", 96),
+                                        ("pair", 112), ("pair", 128), ("pair", 144),
+                                        ("nibble", 48), ("nibble", 64), ("nibble", 80),
+                                        ("nibble", 96)])
+@pytest.mark.parametrize("groups", [1, 100, 257, 1500, 4095, 4096, 4097, 5000])
 def test_groups_spread_over_cus(R, alphabet, N, groups):
     from rans_vectoradd import tans_codec as T
     K = groups * 64 - 3
