@@ -988,6 +988,62 @@ __device__ __forceinline__ void dec_tile(Chains<C>& ch, const v2u* __restrict__ 
     dec_tile<SPS, C, LAST, RESIDENT>(ch, tbl, lane, ex, last_segs, fin_pos, [] {});
 }
 
+// All tiles of wave w's streams (at least two), each finished (composed and
+// stored: w.finish<tile mod kSmAhead>) among the next one's decode steps.
+// For workgroups of few waves: see fused_add_kernel.
+template <class Wave>
+__device__ __forceinline__ void run_overlapped(Wave& w) {
+    static_assert(kSmAhead == 4, "unrolled for kSmAhead == 4");
+    constexpr int C = Wave::C;
+    uint32_t a[C][4], b[C][4];
+    // decode tile t (P = t mod 4) into `ex` beside the finish of tile t - 1
+    auto step = [&](auto P, auto LAST, int t, uint32_t (&ex)[C][4], const uint32_t (&done)[C][4]) {
+        w.template decode<decltype(LAST)::value>(ex, [&] {
+            w.template finish<(decltype(P)::value + kSmAhead - 1) % kSmAhead>(t - 1, done);
+        });
+    };
+    constexpr std::integral_constant<int, 0> p0{};
+    constexpr std::integral_constant<int, 1> p1{};
+    constexpr std::integral_constant<int, 2> p2{};
+    constexpr std::integral_constant<int, 3> p3{};
+    constexpr std::false_type mid{};
+    constexpr std::true_type last{};
+    w.template decode<false>(a, [] {});
+    const int body = w.n_tiles - 1;
+    int t = 1;
+    for (; t + 3 < body; t += 4) {
+        step(p1, mid, t, b, a);
+        step(p2, mid, t + 1, a, b);
+        step(p3, mid, t + 2, b, a);
+        step(p0, mid, t + 3, a, b);
+    }
+    // tiles t .. body, one to four of them (t mod 4 = 1)
+    switch (body - t) {
+        case 0:
+            step(p1, last, t, b, a);
+            w.template finish<1>(t, b);
+            break;
+        case 1:
+            step(p1, mid, t, b, a);
+            step(p2, last, t + 1, a, b);
+            w.template finish<2>(t + 1, a);
+            break;
+        case 2:
+            step(p1, mid, t, b, a);
+            step(p2, mid, t + 1, a, b);
+            step(p3, last, t + 2, b, a);
+            w.template finish<3>(t + 2, b);
+            break;
+        default:
+            step(p1, mid, t, b, a);
+            step(p2, mid, t + 1, a, b);
+            step(p3, mid, t + 2, b, a);
+            step(p0, last, t + 3, a, b);
+            w.template finish<0>(t + 3, a);
+            break;
+    }
+}
+
 // ---------------------------------------------------------------------
 // Fused decode + add.  A wave decodes G groups of A and the same G groups
 // of B (C = 2G chains) and writes their sums, tiled [N/16, K, 16].  The
@@ -1031,53 +1087,11 @@ struct FusedWave {
         finish<P>(t, ex);
     }
 
-    // Decode tile t into ex while tile t - 1 (exponents in done) is finished.
-    template <int P, bool LAST>
-    __device__ __forceinline__ void overlapped(int t, uint32_t (&ex)[C][4],
-                                               const uint32_t (&done)[C][4]) {
+    // Tile t's exponents, with `beside` put among its steps (run_overlapped).
+    template <bool LAST, class Beside>
+    __device__ __forceinline__ void decode(uint32_t (&ex)[C][4], Beside&& beside) {
         dec_tile<SPS, C, LAST, RES>(ch, tbl, lane, ex, Alpha<SPS>::kSegsPerTile,
-                                    Alpha<SPS>::kFinPosFullTile,
-                                    [&] { finish<(P + kSmAhead - 1) % kSmAhead>(t - 1, done); });
-    }
-
-    // All tiles of a stream of n_tiles >= 2, each finished beside the next.
-    __device__ __forceinline__ void run_overlapped() {
-        static_assert(kSmAhead == 4 && !PACKED, "unrolled for kSmAhead == 4");
-        uint32_t a[C][4], b[C][4];
-        dec_tile<SPS, C, false, RES>(ch, tbl, lane, a);
-        const int body = n_tiles - 1;
-        int t = 1;
-        for (; t + 3 < body; t += 4) {
-            overlapped<1, false>(t, b, a);
-            overlapped<2, false>(t + 1, a, b);
-            overlapped<3, false>(t + 2, b, a);
-            overlapped<0, false>(t + 3, a, b);
-        }
-        // tiles t .. body, one to four of them (t mod 4 = 1)
-        switch (body - t) {
-            case 0:
-                overlapped<1, true>(t, b, a);
-                finish<1>(t, b);
-                break;
-            case 1:
-                overlapped<1, false>(t, b, a);
-                overlapped<2, true>(t + 1, a, b);
-                finish<2>(t + 1, a);
-                break;
-            case 2:
-                overlapped<1, false>(t, b, a);
-                overlapped<2, false>(t + 1, a, b);
-                overlapped<3, true>(t + 2, b, a);
-                finish<3>(t + 2, b);
-                break;
-            default:
-                overlapped<1, false>(t, b, a);
-                overlapped<2, false>(t + 1, a, b);
-                overlapped<3, false>(t + 2, b, a);
-                overlapped<0, true>(t + 3, a, b);
-                finish<0>(t + 3, a);
-                break;
-        }
+                                    Alpha<SPS>::kFinPosFullTile, beside);
     }
 
     // Compose, add and store tile t from its exponents, and load the
@@ -1352,7 +1366,7 @@ __global__ __launch_bounds__(W * kLanes) void fused_add_kernel(
         }
         w.base = done;
         if constexpr (LOW) {
-            w.run_overlapped();
+            run_overlapped(w);
             g0 += grid_groups;
             if (g0 >= n_groups) break;
             setup(g0, false);
@@ -1405,6 +1419,8 @@ __global__ __launch_bounds__(W * kLanes) void fused_add_kernel(
 // complete (the tensor's last lanes) each store is checked against the
 // lanes in range, down to single bytes.
 // ---------------------------------------------------------------------
+// A wave with at most one other on its SIMD takes one group (NG = 1): its rows
+// of 64 columns go through 16 staging rows and out as half lines.
 constexpr int kDecodeGroups = 2;
 
 // Word d of lane i in a quad holds rows 4j..4j+3 of column i; the result
@@ -1432,19 +1448,24 @@ __device__ __forceinline__ void quad_selectors(int lane, uint32_t& sel1, uint32_
 constexpr int kXposeStride = 48;
 constexpr int kXposeWords = 7 * kXposeStride + kDecodeGroups * kLanes / 4;
 
-template <int SPS>
+// NG = 1: 16 rows x 64 columns, rows 20 dwords apart.
+constexpr int kXposeStride1 = 20;
+static_assert(16 * kXposeStride1 <= kXposeWords, "one group's 16 rows fit too");
+
+template <int SPS, int NG, int W>
 struct DecodeSmem {
-    DecSmem<SPS, kDecodeGroups> dec;
-    alignas(16) uint32_t xpose[kDecWaves][kXposeWords];
+    DecSmem<SPS, NG, W> dec;
+    alignas(16) uint32_t xpose[W][kXposeWords];
 };
-static_assert(sizeof(DecodeSmem<2>) <= 160 * 1024 && sizeof(DecodeSmem<1>) <= 160 * 1024,
+static_assert(sizeof(DecodeSmem<2, kDecodeGroups, kDecWaves>) <= 160 * 1024 &&
+                  sizeof(DecodeSmem<1, kDecodeGroups, kDecWaves>) <= 160 * 1024,
               "decoder LDS exceeds the 160 KiB of a gfx950 CU");
 
 // FIRST as in FusedWave: > 0 for streams loaded whole at their start,
 // < 0 for the packed layout.
-template <int SPS, int FIRST>
+template <int SPS, int FIRST, int NG>
 struct DecodeWave {
-    static constexpr int C = kDecodeGroups;
+    static constexpr int C = NG;   // groups of the wave: one chain each
     static constexpr bool PACKED = FIRST < 0;
     static constexpr bool RES = FIRST != 0;
     Chains<C> ch;
@@ -1464,9 +1485,10 @@ struct DecodeWave {
     uint32_t sel1, sel2;
     uint32_t* xp;           // this wave's staging rows (LDS)
     int n_tiles;
+    int n_last;             // elements per lane of the last tile
     int lane;
     int base;               // tiles this wave finished in earlier groups (pacing)
-    bool full;              // both groups have 64 lanes in range (wave-uniform)
+    bool full;              // all the wave's groups have 64 lanes in range (wave-uniform)
     bool lines;             // K % 16 == 0: rows start 16-byte aligned
     int last_segs;          // refill segments of the streams in the last tile
     uint32_t fin_pos;       // the final check's threshold (check_last)
@@ -1482,6 +1504,23 @@ struct DecodeWave {
         if constexpr (PACKED) pk_tile<C, P == 0>(pk, preg, tbl, ex);
         else dec_tile<SPS, C, LAST, RES>(ch, tbl, lane, ex, last_segs, fin_pos);
         pace(progress, lane, (uint32_t)(base + t), live);
+        finish<P>(t, ex, n);
+    }
+
+    // Tile t's exponents, with `beside` put among its steps (run_overlapped).
+    template <bool LAST, class Beside>
+    __device__ __forceinline__ void decode(uint32_t (&ex)[C][4], Beside&& beside) {
+        dec_tile<SPS, C, LAST, RES>(ch, tbl, lane, ex, last_segs, fin_pos, beside);
+    }
+    template <int P>
+    __device__ __forceinline__ void finish(int t, const uint32_t (&ex)[C][4]) {
+        finish<P>(t, ex, t == n_tiles - 1 ? n_last : kTile);
+    }
+
+    // Compose and store tile t (n elements per lane) from its exponents, and
+    // load the sign/mantissa words four tiles ahead.
+    template <int P>
+    __device__ __forceinline__ void finish(int t, const uint32_t (&ex)[C][4], int n) {
         uint32_t w[C][4];
         #pragma unroll
         for (int g = 0; g < C; g++) {
@@ -1494,6 +1533,16 @@ struct DecodeWave {
             // so each 8 lanes write one whole 128-byte line (non-temporal).
             // The wave's LDS accesses execute in order, so the writes of
             // half h = 1 come after the reads of half 0.
+            if constexpr (C == 1) {
+                // (one group: 4 lanes write 64 bytes of a row, cached so that
+                // the line's halves can meet)
+                #pragma unroll
+                for (int j = 0; j < 4; j++)
+                    xp[(4 * j + (lane & 3)) * kXposeStride1 + (lane >> 2)] =
+                        quad_transpose(w[0][j], sel1, sel2);
+                *reinterpret_cast<v4u*>(out_tile + (int64_t)(lane >> 2) * K + (lane & 3) * 16) =
+                    *reinterpret_cast<const v4u*>(xp + (lane >> 2) * kXposeStride1 + (lane & 3) * 4);
+            } else
             #pragma unroll
             for (int h = 0; h < 2; h++) {
                 #pragma unroll
@@ -1559,7 +1608,7 @@ struct DecodeWave {
     // All tiles: the first n_tiles - 1 four per iteration (the sign/mantissa
     // buffers rotate by four), then the last one, which holds n_last
     // elements and ends the streams.
-    __device__ __forceinline__ void run(int n_last) {
+    __device__ __forceinline__ void run() {
         static_assert(kSmAhead == 4, "the loop below is unrolled for kSmAhead == 4");
         const int body = n_tiles - 1;
         for (int t = 0; t < body; t += kSmAhead) {
@@ -1578,19 +1627,27 @@ struct DecodeWave {
 };
 
 
-template <int SPS, int FIRST>
-__global__ __launch_bounds__(kDecBlock) void decode_kernel(
+// W < kDecWaves (streams of any length): run_overlapped, as in
+// fused_add_kernel.  Per call with the table's build, two groups per wave and 16
+// waves per workgroup against this: 10007 x 1000 nibble 102 -> 77 us, 16384 x
+// 1024 pair 50 us (111 us before groups were spread over the CUs), 130000 x 512
+// 78 -> 42 us (8 waves of one group; 4 waves of two 52 us), 262144 x 512 72 -> 58
+// us (8 waves of two).
+template <int SPS, int FIRST, int NG, int W>
+__global__ __launch_bounds__(W * kLanes) void decode_kernel(
     const uint32_t* __restrict__ comp, int64_t words, const int64_t* __restrict__ off,
     const uint16_t* __restrict__ st, const v2u* __restrict__ sm,
     const v2u* __restrict__ table, int64_t K, int64_t N, int waves,
     uint8_t* __restrict__ out) {
     constexpr uint32_t L = Alpha<SPS>::L;
-    constexpr int C = kDecodeGroups;
-    __shared__ DecodeSmem<SPS> dsmem;
-    DecSmem<SPS, C>& smem = dsmem.dec;
+    constexpr int C = NG;
+    constexpr bool LOW = W < kDecWaves;
+    static_assert(!LOW || FIRST == 0, "streams of any length");
+    __shared__ DecodeSmem<SPS, NG, W> dsmem;
+    DecSmem<SPS, C, W>& smem = dsmem.dec;
     v2u* tbl = smem.tbl;
     // loads issued together, as in fused_add_kernel
-    TableRegs<L> tr;
+    TableRegs<L, W * kLanes> tr;
     table_fetch(tr, table);
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
@@ -1609,13 +1666,14 @@ __global__ __launch_bounds__(kDecBlock) void decode_kernel(
                       (PACKED && SPS == 2 && -FIRST <= kSmAhead),
                   "one-tile streams, streams of up to kResidentTiles tiles, any streams, or "
                   "packed streams of up to 4 tiles");
-    DecodeWave<SPS, FIRST> w;
+    DecodeWave<SPS, FIRST, NG> w;
     w.progress = &smem.progress;
     w.live = (uint32_t)(wg_groups >= (int64_t)waves * C ? waves : (wg_groups + C - 1) / C);
     w.lane = lane;
     w.K = K;
     const int rag = (int)(N % kTile);
     w.n_tiles = (int)(N / kTile) + (rag ? 1 : 0);
+    w.n_last = rag ? rag : kTile;
     last_tile_sched<SPS>(N / SPS, w.n_tiles, w.last_segs, w.fin_pos);
     w.tbl = tbl;
     w.sm_stride = K * 8;
@@ -1689,7 +1747,8 @@ __global__ __launch_bounds__(kDecBlock) void decode_kernel(
             }
         }
         w.base = done;
-        w.run(rag ? rag : kTile);
+        if constexpr (LOW) run_overlapped(w);
+        else w.run();
         done += w.n_tiles;
         g0 += grid_groups;
         if (g0 >= n_groups) break;
@@ -2721,26 +2780,35 @@ int tans_decode(const void* comp, int64_t comp_bytes, const int64_t* offsets,
     // the stores address 4 rows of a tile with 32-bit offsets
     if (K > (int64_t(1) << 30)) return fail(TANS_EINVAL, "decode: more than 2^30 lanes");
     const int64_t groups = (K + kLanes - 1) / kLanes;
-    // a wave takes two groups; those that do not fill the chip are spread
-    // over it (spread_waves)
+    // a wave takes two groups, or one where that gives no more than two waves
+    // per SIMD; those that do not fill the chip are spread over it
+    // (spread_waves)
     const int cus = cu_count();
     if (cus <= 0) return fail(TANS_EHIP, "decode: cannot query the device's CU count");
-    const int64_t pairs = (groups + kDecodeGroups - 1) / kDecodeGroups;
-    const int waves = spread_waves(pairs, cus);
-    int64_t blocks = (pairs + waves - 1) / waves;
+    const int64_t n_tiles = (N + kTile - 1) / kTile;
+    const bool any_length = n_tiles > (sps == 2 ? Alpha<2>::kResidentTiles : 1);
+    const int per_wave = any_length && groups <= (int64_t)kMidWaves * cus ? 1 : kDecodeGroups;
+    const int64_t units = (groups + per_wave - 1) / per_wave;
+    const int waves = spread_waves(units, cus);
+    int64_t blocks = (units + waves - 1) / waves;
     // Columns of one or two tiles: one workgroup per CU, the waves loop over
     // their group pairs (measured at 2^30 elements: 16 per column 923 ->
     // 616 us).  From 4 tiles on, one workgroup per 32 groups is as fast or
     // faster (64 per column: 472 vs 468 us; 256: 388 vs 400 us).
-    if ((N + kTile - 1) / kTile <= 2) blocks = std::min<int64_t>(blocks, cus);
+    if (n_tiles <= 2) blocks = std::min<int64_t>(blocks, cus);
     if (!grid_fits(blocks, kDecBlock)) return fail(TANS_EINVAL, "decode: K too large");
-#define TANS_LAUNCH_DECODE(S, FIRST)                                                              \
-    hipLaunchKernelGGL((decode_kernel<S, FIRST>), dim3((unsigned)blocks),                        \
-                       dim3(kDecBlock), 0, (hipStream_t)stream, (const uint32_t*)comp,           \
+#define TANS_LAUNCH_DECODE_W(S, FIRST, NG, W)                                                     \
+    hipLaunchKernelGGL((decode_kernel<S, FIRST, NG, W>), dim3((unsigned)blocks),                 \
+                       dim3(W * kLanes), 0, (hipStream_t)stream, (const uint32_t*)comp,           \
                        comp_bytes / 4, offsets, states, (const v2u*)sm, (const v2u*)table, K, N, \
                        waves, (uint8_t*)out)
+#define TANS_LAUNCH_DECODE(S, FIRST) TANS_LAUNCH_DECODE_W(S, FIRST, kDecodeGroups, kDecWaves)
+#define TANS_LAUNCH_DECODE_ANY(S)                                                                 \
+    if (per_wave == 1 && waves <= kLowWaves) TANS_LAUNCH_DECODE_W(S, 0, 1, kLowWaves);           \
+    else if (per_wave == 1) TANS_LAUNCH_DECODE_W(S, 0, 1, kMidWaves);                            \
+    else if (waves <= kMidWaves) TANS_LAUNCH_DECODE_W(S, 0, kDecodeGroups, kMidWaves);           \
+    else TANS_LAUNCH_DECODE(S, 0)
     // streams that fit the ring are loaded whole at their start
-    const int64_t n_tiles = (N + kTile - 1) / kTile;
     if (packed) {
         switch (n_tiles) {
             case 1: TANS_LAUNCH_DECODE(2, -1); break;
@@ -2751,12 +2819,14 @@ int tans_decode(const void* comp, int64_t comp_bytes, const int64_t* offsets,
     } else if (sps == 2) {
         if (n_tiles == 1) TANS_LAUNCH_DECODE(2, Alpha<2>::kOneTileSegs);
         else if (n_tiles <= Alpha<2>::kResidentTiles) TANS_LAUNCH_DECODE(2, kSlots);
-        else TANS_LAUNCH_DECODE(2, 0);
+        else { TANS_LAUNCH_DECODE_ANY(2); }
     } else {   // (the nibble decoder loaded whole at two tiles spills registers)
         if (n_tiles == 1) TANS_LAUNCH_DECODE(1, Alpha<1>::kOneTileSegs);
-        else TANS_LAUNCH_DECODE(1, 0);
+        else { TANS_LAUNCH_DECODE_ANY(1); }
     }
 #undef TANS_LAUNCH_DECODE
+#undef TANS_LAUNCH_DECODE_W
+#undef TANS_LAUNCH_DECODE_ANY
     return hip_check(hipGetLastError(), "decode_kernel launch");
 }
 

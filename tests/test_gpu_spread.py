@@ -51,6 +51,23 @@ def test_groups_spread_over_cus(R, alphabet, N, groups):
     assert torch.equal(dec, a.t())
 
 
+# the decoder's kernels for few waves (one group per wave up to 8 waves per CU,
+# then two): rows of whole 16-byte columns (K % 16 == 0, through the staging
+# rows) and others, whole and partial last groups, ragged last tiles of every
+# tile count mod 4
+@pytest.mark.parametrize("alphabet,N", [("pair", 82), ("pair", 104), ("pair", 128), ("pair", 130),
+                                        ("nibble", 34), ("nibble", 56), ("nibble", 64),
+                                        ("nibble", 90)])
+@pytest.mark.parametrize("K", [64, 6400, 6384, 6397, 96000, 95997, 192000 - 48, 192001])
+def test_decode_with_few_waves(R, alphabet, N, K):
+    from rans_vectoradd import tans_codec as T
+    _say(f"case: decode few waves {K} x {N} {alphabet}")
+    a = _bytes(R, K * N, K + N).view(K, N)
+    e = T.encode_gpu(a, torch.tensor(R.QWEN3_14B_FP8_EXP), alphabet=alphabet)
+    dec = R.gpu_tans_decode(e[0], e[2], e[1], e[3], e[4], e[6], e[5], N)
+    assert torch.equal(dec, a.t())
+
+
 # row groups of 16 rows per segment: one, an odd number, more than the CUs
 # of a segment's share hold in one round
 @pytest.mark.parametrize("rows,cols,segments", [(16, 512, 1), (1000, 2048, 8), (8272, 288, 1),
