@@ -201,6 +201,16 @@ int tans_decode(const void* comp, int64_t comp_bytes, const int64_t* offsets,
                 const uint32_t* table, int32_t log2L,
                 int64_t K, int64_t N, void* out, void* stream);
 
+/* tans_decode without a table: each workgroup builds its own in LDS from the
+ * device spread and freqs (those of tans_build_decode_table_device, which
+ * checks them; here a malformed pair decodes to wrong bytes, without
+ * out-of-range accesses).  Replaces gpu_tans_decode's table build and decode,
+ * csrc/tans_decode.cu:159-210, by one launch.                           */
+int tans_decode_spread(const void* comp, int64_t comp_bytes, const int64_t* offsets,
+                       const uint16_t* states, const void* sm, const int32_t* spread,
+                       const int32_t* freqs, int32_t log2L, int64_t K, int64_t N, void* out,
+                       void* stream);
+
 /* GPU encoder: the same bytes as tans_encode_begin/finish + tans_split_fp8
  * (the reference's tans_encode_interleaved, csrc/tans_codec.cpp:69-196, and
  * the split of rans_vectoradd/tans_codec.py:109-124), from FP8 bytes already

@@ -7,7 +7,7 @@
 //   fp8_add_kernel           uncompressed FP8 add (csrc/vecadd.cu:41-73)
 //   stream_probe_kernel      read-only / write-only / 2:1 streaming at the
 //                            add's launch shape (bandwidth ceilings)
-//   table_kernel             decode table from device spread/freqs
+//   table_kernel<SPS>        decode table from device spread/freqs
 //                            (csrc/tans_decode.cu:23-59 without the host trip)
 //   fused_add_kernel<SPS,G,FIRST> decode two encodings + FP8 add
 //                            (csrc/vecadd.cu:156-243)
@@ -176,121 +176,6 @@ __global__ __launch_bounds__(kBlock) void stream_probe_kernel(const v4u* __restr
                          : a[i] ^ b[i];
         if (NT) __builtin_nontemporal_store(v, c + i); else c[i] = v;
     }
-}
-
-// ---------------------------------------------------------------------
-// Decode table on the device: one workgroup of 16 waves.  The L slots are
-// cut into segments of 64 (wave w, round r: segment w * rounds + r, so
-// segments follow slot order).  A symbol's rank (its earlier slots, in
-// slot order) is its count in earlier segments plus its place among equal
-// symbols in its own segment.  The lanes holding a lane's symbol are the
-// AND over symbol bits of that bit's ballot (complemented where the lane's
-// own bit is 0); mbcnt of that mask is the place, its popcount the count,
-// and the last lane holding each symbol writes the count to LDS.  An exclusive prefix over segments (16
-// segments per thread, then 4 partial totals per symbol) gives the rest.
-//
-// The kernel checks what the host builder (codec.cpp) checks: frequencies
-// not negative and summing to L, every present symbol of a 2^11-state
-// table at a frequency of at least 2, spread symbols inside the alphabet
-// and each symbol's slot count equal to its frequency (a rank below it).
-// On any failure it sets *status (when given) to TANS_ETABLE; the table it
-// writes is then wrong but still in range: a symbol outside the alphabet is
-// folded into it, and the decoders' table_store replaces entries that
-// would step outside the table or read too many bits.
-// ---------------------------------------------------------------------
-constexpr int kTableWaves = 16;
-constexpr int kTableSegs = kTableWaves * 4;   // 64 segments of 64 slots at L = 4096
-
-__global__ __launch_bounds__(kTableWaves * 64) void table_kernel(
-    const int32_t* __restrict__ spread, const int32_t* __restrict__ freqs, int nsym, int log2L,
-    v2u* __restrict__ table, int32_t* __restrict__ status) {
-    __shared__ uint16_t cnt[kTableSegs][256];   // per segment: counts, then exclusive prefix
-    __shared__ uint16_t tot[4][256];            // prefix totals of segment quarters
-    __shared__ uint32_t fsum, bad;              // sum of the frequencies; any check failed
-    const uint32_t L = 1u << log2L;
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int rounds = (int)(L / (kTableWaves * 64));   // 4 (pair) or 2 (nibble)
-    const int sym_bits = 31 - __builtin_clz((uint32_t)nsym);
-    const int nseg = kTableWaves * rounds;
-    for (uint32_t i = threadIdx.x; i < kTableSegs * 256 / 2; i += blockDim.x)
-        reinterpret_cast<uint32_t*>(&cnt[0][0])[i] = 0u;
-    if (threadIdx.x == 0) { fsum = 0u; bad = 0u; }
-    __syncthreads();
-    uint32_t my_bad = 0u;
-    if ((int)threadIdx.x < nsym) {
-        const int32_t f = freqs[threadIdx.x];
-        const int32_t min_f = log2L == tans_sched::kTripleLog2L ? (int32_t)tans_sched::kTripleMinFreq : 1;
-        if (f < 0 || f > (int32_t)L || (f > 0 && f < min_f)) my_bad = 1u;
-        else atomicAdd(&fsum, (uint32_t)f);
-    }
-    uint32_t sym[4] = {0u, 0u, 0u, 0u}, rank[4] = {0u, 0u, 0u, 0u};
-    #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        if (r >= rounds) break;
-        const int seg = wave * rounds + r;
-        // a symbol outside the alphabet is folded into it (and reported)
-        const int32_t raw = spread[seg * 64 + lane];
-        if (raw < 0 || raw >= nsym) my_bad = 1u;
-        const uint32_t sv = (uint32_t)raw & (uint32_t)(nsym - 1);
-        sym[r] = sv;
-        // the lanes holding the same symbol: for each symbol bit, the ballot
-        // of lanes with that bit set, complemented where this lane's bit is 0
-        uint32_t mlo = 0xFFFFFFFFu, mhi = 0xFFFFFFFFu;
-        #pragma unroll
-        for (int bit = 0; bit < 8; bit++) {
-            if (bit >= sym_bits) break;
-            const uint64_t B = __ballot((sv >> bit) & 1u);
-            const uint32_t mine = (uint32_t)__builtin_amdgcn_sbfe((int)sv, bit, 1);   // 0 or ~0
-            mlo &= ~((uint32_t)B ^ mine);
-            mhi &= ~((uint32_t)(B >> 32) ^ mine);
-        }
-        const uint32_t rk = __builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, 0u));
-        const uint32_t tot = (uint32_t)__builtin_popcount(mlo) + (uint32_t)__builtin_popcount(mhi);
-        rank[r] = rk;
-        if (rk + 1u == tot) cnt[seg][sv] = (uint16_t)tot;
-    }
-    __syncthreads();
-    // exclusive prefix over segments: thread (q, s) scans segments [16q, 16q + 16)
-    const int s = threadIdx.x & 255;
-    const int q = threadIdx.x >> 8;
-    uint32_t run = 0;
-    if (s < nsym) {
-        uint16_t v[16];
-        #pragma unroll
-        for (int i = 0; i < 16; i++) v[i] = (16 * q + i < nseg) ? cnt[16 * q + i][s] : (uint16_t)0;
-        #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const uint32_t c = v[i];
-            v[i] = (uint16_t)run;
-            run += c;
-        }
-        tot[q][s] = (uint16_t)run;
-        #pragma unroll
-        for (int i = 0; i < 16; i++)
-            if (16 * q + i < nseg) cnt[16 * q + i][s] = v[i];
-    }
-    __syncthreads();
-    #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        if (r >= rounds) break;
-        const int seg = wave * rounds + r;
-        const uint32_t sv = sym[r];
-        uint32_t before = 0;
-        for (int qq = 0; qq < (seg >> 4); qq++) before += tot[qq][sv];
-        const uint32_t f = (uint32_t)freqs[sv];
-        const uint32_t rk = before + cnt[seg][sv] + rank[r];   // rank among sv's slots
-        if (rk >= f) my_bad = 1u;                              // more slots than its frequency
-        const uint32_t xp = f + rk;
-        const int top = xp ? 31 - __builtin_clz(xp) : log2L;
-        const int nb = top < log2L ? log2L - top : 0;
-        const uint32_t base = xp << nb;
-        const uint32_t ex = (nsym == 256) ? (((sv >> 4) << 11) | ((sv & 0xFu) << 19)) : (sv << 11);
-        table[seg * 64 + lane] = v2u{(uint32_t)nb | ex | ((uint32_t)nb << 27), (base - L) * 8u};
-    }
-    if (my_bad) bad = 1u;   // benign race: every writer stores 1
-    __syncthreads();
-    if (threadIdx.x == 0 && status && (bad || fsum != L)) *status = TANS_ETABLE;
 }
 
 // ---------------------------------------------------------------------
@@ -617,8 +502,8 @@ __device__ __forceinline__ void compose8(uint32_t ex_lo, uint32_t ex_hi, uint32_
 // thread, table_store writes them once they arrive.  Entries that would
 // step outside the table (nb > log2L or base + 2^nb > 2L), or read more
 // bits than the refill schedule allows (nb > 10 in a 2^11-state table), are
-// replaced by a harmless one, so a malformed table gives wrong bytes, never
-// an out-of-range LDS access.
+// replaced by a harmless one (lds_entry), so a malformed table gives wrong
+// bytes, never an out-of-range LDS access.
 template <uint32_t L, int T = kDecBlock>   // T: threads of the workgroup
 struct TableRegs {
     static_assert(L % T == 0, "the table is split evenly over the workgroup");
@@ -631,24 +516,193 @@ __device__ __forceinline__ void table_fetch(TableRegs<L, T>& r, const v2u* __res
     for (uint32_t k = 0; k < L / T; k++) r.e[k] = table[threadIdx.x + k * T];
 }
 
-// PACKED: the entries of the packed-layout decoders, whose word0 keeps nb
-// in bits 4:0 and moves the two exponents 8 bits up (bits 22:19 and
-// 30:27), so that bits 15:0 of a sum of word0s are the sum of their nb.
-template <uint32_t L, bool PACKED = false, int T>
-__device__ __forceinline__ void table_store(v2u* lds, const TableRegs<L, T>& r) {
+// A table entry as the decoders keep it in LDS: one that would step outside
+// the table or read too many bits becomes a harmless one.  PACKED: the
+// packed-layout decoders' word0, which keeps nb in bits 4:0 and moves the
+// two exponents 8 bits up (bits 22:19 and 30:27), so that bits 15:0 of a sum
+// of word0s are the sum of their nb.
+template <uint32_t L, bool PACKED>
+__device__ __forceinline__ v2u lds_entry(v2u e) {
     constexpr uint32_t log2L = 31 - __builtin_clz(L);
     constexpr uint32_t max_nb =
         log2L == tans_sched::kTripleLog2L ? tans_sched::kTripleMaxNb : log2L;
+    const uint32_t nb = e.x & 0xFFu;
+    const uint32_t base = e.y >> 3;
+    if (nb > max_nb || (e.x >> 27) != nb || (e.y & 7u) || base + (1u << nb) > L)
+        e = v2u{e.x & 0x07FFFF00u, 0u};
+    if constexpr (PACKED) e.x = (e.x & 0x1Fu) | ((e.x & 0x007FF800u) << 8);
+    return e;
+}
+
+template <uint32_t L, bool PACKED = false, int T>
+__device__ __forceinline__ void table_store(v2u* lds, const TableRegs<L, T>& r) {
     #pragma unroll
-    for (uint32_t k = 0; k < L / T; k++) {
-        v2u e = r.e[k];
-        const uint32_t nb = e.x & 0xFFu;
-        const uint32_t base = e.y >> 3;
-        if (nb > max_nb || (e.x >> 27) != nb || (e.y & 7u) || base + (1u << nb) > L)
-            e = v2u{e.x & 0x07FFFF00u, 0u};
-        if constexpr (PACKED) e.x = (e.x & 0x1Fu) | ((e.x & 0x007FF800u) << 8);
-        lds[threadIdx.x + k * T] = e;
+    for (uint32_t k = 0; k < L / T; k++)
+        lds[threadIdx.x + k * T] = lds_entry<L, PACKED>(r.e[k]);
+}
+
+// ---------------------------------------------------------------------
+// Decode table from (spread, freqs), by the W waves of a workgroup.  The L
+// slots are cut into segments of 64 (wave w takes a contiguous run of them).
+// A slot's rank (the earlier slots of its symbol, in slot order) is the
+// symbol's count in earlier segments plus the slot's place among equal
+// symbols in its own segment.  The lanes holding a lane's symbol are the
+// AND over symbol bits of that bit's ballot (complemented where the lane's
+// own bit is 0); mbcnt of that mask is the place, its popcount the count,
+// and the last lane holding each symbol writes the count to LDS.  An
+// exclusive prefix over segments (in up to four parts per symbol, whose
+// totals the last step adds) gives the rest.
+//
+// Used by table_kernel and by decode_kernel, which builds its own table in
+// LDS instead of waiting for a kernel that does (7 us; 100000 x 128 18.3 -> 14.9
+// us per call, 10007 x 1000 nibble 76.5 -> 71.7, 2^30 elements 375 -> 374).
+// ---------------------------------------------------------------------
+template <int SPS>
+struct TableShape {
+    static constexpr int kSyms = SPS == 2 ? 256 : 16;
+    static constexpr int kLog2L = SPS == 2 ? TANS_PAIR_LOG2L : TANS_NIBBLE_LOG2L;
+    static constexpr uint32_t L = 1u << kLog2L;
+    static constexpr int kSegs = (int)(L / 64);
+};
+
+template <int SPS, int W>
+struct TableScratch {
+    using S = TableShape<SPS>;
+    static constexpr int kParts = W * 64 / S::kSyms < 4 ? W * 64 / S::kSyms : 4;
+    uint16_t cnt[S::kSegs][S::kSyms];   // per segment: counts, then exclusive prefix in its part
+    uint16_t tot[kParts][S::kSyms];     // each part's total
+    uint32_t f[S::kSyms];
+};
+
+// The loads of a build: the thread's slots of the spread and a frequency.
+template <int SPS, int W>
+struct SpreadRegs {
+    static constexpr int kRounds = TableShape<SPS>::kSegs / W;   // segments per wave
+    int32_t s[kRounds];
+    int32_t f;
+};
+
+template <int SPS, int W>
+__device__ __forceinline__ void spread_fetch(SpreadRegs<SPS, W>& r,
+                                             const int32_t* __restrict__ spread,
+                                             const int32_t* __restrict__ freqs) {
+    constexpr int R = SpreadRegs<SPS, W>::kRounds;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    #pragma unroll
+    for (int i = 0; i < R; i++) r.s[i] = spread[(wave * R + i) * 64 + lane];
+    r.f = (int)threadIdx.x < TableShape<SPS>::kSyms ? freqs[threadIdx.x] : 0;
+}
+
+// Calls emit(slot, entry) for the thread's slots (the entry as the host
+// builder writes it).  Returns whether the thread saw a symbol outside the
+// alphabet (folded into it) or a slot past its symbol's frequency.  Every
+// thread of the workgroup takes part; sc must not be reused before the
+// caller's next barrier.
+template <int SPS, int W, class Emit>
+__device__ __forceinline__ bool table_build(TableScratch<SPS, W>& sc, const SpreadRegs<SPS, W>& r,
+                                            Emit&& emit) {
+    using S = TableShape<SPS>;
+    using Sc = TableScratch<SPS, W>;
+    constexpr int R = SpreadRegs<SPS, W>::kRounds;
+    constexpr int kBits = SPS == 2 ? 8 : 4;
+    constexpr int kPartSegs = S::kSegs / Sc::kParts;
+    static_assert(S::kSegs % W == 0 && S::kSegs % Sc::kParts == 0, "whole segments");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (uint32_t i = threadIdx.x; i < sizeof(sc.cnt) / 4; i += W * 64)
+        reinterpret_cast<uint32_t*>(&sc.cnt[0][0])[i] = 0u;
+    if ((int)threadIdx.x < S::kSyms) sc.f[threadIdx.x] = (uint32_t)r.f;
+    __syncthreads();
+    bool bad = false;
+    uint32_t sym[R], rank[R];
+    #pragma unroll
+    for (int i = 0; i < R; i++) {
+        if (r.s[i] < 0 || r.s[i] >= S::kSyms) bad = true;
+        const uint32_t sv = (uint32_t)r.s[i] & (uint32_t)(S::kSyms - 1);
+        uint32_t mlo = 0xFFFFFFFFu, mhi = 0xFFFFFFFFu;
+        #pragma unroll
+        for (int bit = 0; bit < kBits; bit++) {
+            const uint64_t B = __ballot((sv >> bit) & 1u);
+            const uint32_t mine = (uint32_t)__builtin_amdgcn_sbfe((int)sv, bit, 1);   // 0 or ~0
+            mlo &= ~((uint32_t)B ^ mine);
+            mhi &= ~((uint32_t)(B >> 32) ^ mine);
+        }
+        const uint32_t rk = __builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, 0u));
+        const uint32_t tot = (uint32_t)__builtin_popcount(mlo) + (uint32_t)__builtin_popcount(mhi);
+        sym[i] = sv;
+        rank[i] = rk;
+        if (rk + 1u == tot) sc.cnt[wave * R + i][sv] = (uint16_t)tot;
     }
+    __syncthreads();
+    if ((int)threadIdx.x < Sc::kParts * S::kSyms) {
+        const int s = threadIdx.x % S::kSyms, q = threadIdx.x / S::kSyms;
+        constexpr int kBatch = 8;
+        static_assert(kPartSegs % kBatch == 0, "whole batches");
+        uint32_t run = 0;
+        for (int b = 0; b < kPartSegs; b += kBatch) {
+            uint32_t v[kBatch];
+            #pragma unroll
+            for (int i = 0; i < kBatch; i++) v[i] = sc.cnt[q * kPartSegs + b + i][s];
+            #pragma unroll
+            for (int i = 0; i < kBatch; i++) {
+                sc.cnt[q * kPartSegs + b + i][s] = (uint16_t)run;
+                run += v[i];
+            }
+        }
+        sc.tot[q][s] = (uint16_t)run;
+    }
+    __syncthreads();
+    #pragma unroll
+    for (int i = 0; i < R; i++) {
+        const int seg = wave * R + i;
+        const uint32_t sv = sym[i];
+        uint32_t rk = sc.cnt[seg][sv] + rank[i];   // rank among sv's slots
+        #pragma unroll
+        for (int q = 0; q + 1 < Sc::kParts; q++)
+            if (q < seg / kPartSegs) rk += sc.tot[q][sv];   // wave-uniform
+        const uint32_t f = sc.f[sv];
+        if (rk >= f) bad = true;                   // more slots than its frequency
+        const uint32_t xp = f + rk;
+        const int top = xp ? 31 - __builtin_clz(xp) : S::kLog2L;
+        const int nb = top < S::kLog2L ? S::kLog2L - top : 0;
+        const uint32_t ex = SPS == 2 ? (((sv >> 4) << 11) | ((sv & 0xFu) << 19)) : (sv << 11);
+        emit(seg * 64 + lane,
+             v2u{(uint32_t)nb | ex | ((uint32_t)nb << 27), ((xp << nb) - S::L) * 8u});
+    }
+    return bad;
+}
+
+// The table in global memory, by one workgroup.  It checks what the host
+// builder (codec.cpp) checks: frequencies not negative and summing to L,
+// every present symbol of a 2^11-state table at a frequency of at least 2,
+// spread symbols inside the alphabet and each symbol's slot count equal to
+// its frequency (a rank below it).  On any failure it sets *status (when
+// given) to TANS_ETABLE; the table is then wrong but still in range: the
+// decoders replace entries that would step outside it or read too many bits
+// (lds_entry).
+constexpr int kTableWaves = 16;
+
+template <int SPS>
+__global__ __launch_bounds__(kTableWaves * 64) void table_kernel(
+    const int32_t* __restrict__ spread, const int32_t* __restrict__ freqs,
+    v2u* __restrict__ table, int32_t* __restrict__ status) {
+    using S = TableShape<SPS>;
+    __shared__ TableScratch<SPS, kTableWaves> sc;
+    __shared__ uint32_t fsum, any_bad;   // sum of the frequencies; any check failed
+    SpreadRegs<SPS, kTableWaves> r;
+    spread_fetch(r, spread, freqs);
+    if (threadIdx.x == 0) { fsum = 0u; any_bad = 0u; }
+    __syncthreads();
+    bool bad = false;
+    if ((int)threadIdx.x < S::kSyms) {
+        constexpr int32_t min_f =
+            S::kLog2L == tans_sched::kTripleLog2L ? (int32_t)tans_sched::kTripleMinFreq : 1;
+        if (r.f < 0 || r.f > (int32_t)S::L || (r.f > 0 && r.f < min_f)) bad = true;
+        else atomicAdd(&fsum, (uint32_t)r.f);
+    }
+    bad |= table_build<SPS, kTableWaves>(sc, r, [&](int slot, v2u e) { table[slot] = e; });
+    if (bad) any_bad = 1u;   // benign race: every writer stores 1
+    __syncthreads();
+    if (threadIdx.x == 0 && status && (any_bad || fsum != S::L)) *status = TANS_ETABLE;
 }
 
 // ---------------------------------------------------------------------
@@ -1456,6 +1510,15 @@ template <int SPS, int NG, int W>
 struct DecodeSmem {
     DecSmem<SPS, NG, W> dec;
     alignas(16) uint32_t xpose[W][kXposeWords];
+    // scratch of the table build: the stream rings where they are large
+    // enough (nothing is in them yet), else memory of its own
+    using Scratch = TableScratch<SPS, W>;
+    static constexpr bool kInRings = sizeof(dec.rings) >= sizeof(Scratch);
+    alignas(16) unsigned char more[kInRings ? 16 : sizeof(Scratch)];
+    __device__ __forceinline__ Scratch& scratch() {
+        return *reinterpret_cast<Scratch*>(kInRings ? reinterpret_cast<unsigned char*>(dec.rings)
+                                                    : more);
+    }
 };
 static_assert(sizeof(DecodeSmem<2, kDecodeGroups, kDecWaves>) <= 160 * 1024 &&
                   sizeof(DecodeSmem<1, kDecodeGroups, kDecWaves>) <= 160 * 1024,
@@ -1637,7 +1700,8 @@ template <int SPS, int FIRST, int NG, int W>
 __global__ __launch_bounds__(W * kLanes) void decode_kernel(
     const uint32_t* __restrict__ comp, int64_t words, const int64_t* __restrict__ off,
     const uint16_t* __restrict__ st, const v2u* __restrict__ sm,
-    const v2u* __restrict__ table, int64_t K, int64_t N, int waves,
+    const v2u* __restrict__ table, const int32_t* __restrict__ spread,
+    const int32_t* __restrict__ freqs, int64_t K, int64_t N, int waves,
     uint8_t* __restrict__ out) {
     constexpr uint32_t L = Alpha<SPS>::L;
     constexpr int C = NG;
@@ -1647,8 +1711,11 @@ __global__ __launch_bounds__(W * kLanes) void decode_kernel(
     DecSmem<SPS, C, W>& smem = dsmem.dec;
     v2u* tbl = smem.tbl;
     // loads issued together, as in fused_add_kernel
+    // (the table, or the spread that it is built from)
     TableRegs<L, W * kLanes> tr;
-    table_fetch(tr, table);
+    SpreadRegs<SPS, W> sr;
+    if (spread) spread_fetch(sr, spread, freqs);   // kernel-uniform
+    else table_fetch(tr, table);
     const int lane = threadIdx.x & (kLanes - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
     const int64_t n_groups = (K + kLanes - 1) / kLanes;
@@ -1731,7 +1798,11 @@ __global__ __launch_bounds__(W * kLanes) void decode_kernel(
         w.full = full;
     };
     setup(g0);
-    table_store<L, PACKED>(tbl, tr);
+    if (spread)
+        table_build<SPS, W>(dsmem.scratch(), sr,
+                            [&](int slot, v2u e) { tbl[slot] = lds_entry<L, PACKED>(e); });
+    else
+        table_store<L, PACKED>(tbl, tr);
     if (threadIdx.x == 0) smem.init();
     __syncthreads();
     if (!live) return;
@@ -2686,8 +2757,11 @@ int tans_build_decode_table_device(const int32_t* spread, const int32_t* freqs, 
     if (!((nsym == 256 && log2L == TANS_PAIR_LOG2L) || (nsym == 16 && log2L == TANS_NIBBLE_LOG2L)))
         return fail(TANS_EINVAL, "table: need (nsym 256, log2L 12) or (nsym 16, log2L 11)");
     if (status && !aligned(status, 4)) return fail(TANS_EINVAL, "table: status must be 4-byte aligned");
-    hipLaunchKernelGGL(table_kernel, dim3(1), dim3(kTableWaves * 64), 0, (hipStream_t)stream, spread, freqs,
-                       (int)nsym, (int)log2L, (v2u*)table, status);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(kTableWaves * 64), 0, (hipStream_t)stream, spread,
+                           freqs, (v2u*)table, status);
+    };
+    if (nsym == 256) launch(table_kernel<2>); else launch(table_kernel<1>);
     return hip_check(hipGetLastError(), "table_kernel launch");
 }
 
@@ -2757,14 +2831,21 @@ int tans_fp8_vecadd_fused(const void* a_comp, int64_t a_comp_bytes, const int64_
     return hip_check(hipGetLastError(), "fused_add_kernel launch");
 }
 
-int tans_decode(const void* comp, int64_t comp_bytes, const int64_t* offsets,
-                const uint16_t* states, const void* sm, const uint32_t* table, int32_t log2L,
-                int64_t K, int64_t N, void* out, void* stream) {
+}  // extern "C"
+
+namespace {
+
+// tans_decode with its table, or with the spread and frequencies it is built
+// from (table null)
+int decode_launch(const void* comp, int64_t comp_bytes, const int64_t* offsets,
+                  const uint16_t* states, const void* sm, const uint32_t* table,
+                  const int32_t* spread, const int32_t* freqs, int32_t log2L, int64_t K, int64_t N,
+                  void* out, void* stream) {
     const int sps = sps_for(log2L);
     if (!sps) return fail(TANS_EINVAL, "decode: log2L must be 12 (pair) or 11 (nibble)");
     if (K < 0 || N < 0 || N % 2) return fail(TANS_EINVAL, "decode: N must be even");
     if (K == 0 || N == 0) return TANS_OK;
-    if (!comp || !offsets || !sm || !table || !out)
+    if (!comp || !offsets || !sm || !(table || (spread && freqs)) || !out)
         return fail(TANS_EINVAL, "decode: null pointer");
     // no state array: the packed layout of short streams
     const bool packed = !states;
@@ -2774,7 +2855,7 @@ int tans_decode(const void* comp, int64_t comp_bytes, const int64_t* offsets,
     if (comp_bytes < 0 || comp_bytes % 4)
         return fail(TANS_EINVAL, "decode: compressed size must be a multiple of 4 bytes");
     if (!aligned(comp, 16) || !aligned(sm, 8) || !aligned(offsets, 8) || !aligned(states, 2) ||
-        !aligned(table, 8) || !aligned(out, 4))
+        !aligned(table, 8) || !aligned(spread, 4) || !aligned(freqs, 4) || !aligned(out, 4))
         return fail(TANS_EINVAL, "decode: misaligned buffer (comp 16, sm 8, out 4 bytes)");
     if ((N + kTile - 1) / kTile > INT32_MAX) return fail(TANS_EINVAL, "decode: N too large");
     // the stores address 4 rows of a tile with 32-bit offsets
@@ -2800,7 +2881,8 @@ int tans_decode(const void* comp, int64_t comp_bytes, const int64_t* offsets,
 #define TANS_LAUNCH_DECODE_W(S, FIRST, NG, W)                                                     \
     hipLaunchKernelGGL((decode_kernel<S, FIRST, NG, W>), dim3((unsigned)blocks),                 \
                        dim3(W * kLanes), 0, (hipStream_t)stream, (const uint32_t*)comp,           \
-                       comp_bytes / 4, offsets, states, (const v2u*)sm, (const v2u*)table, K, N, \
+                       comp_bytes / 4, offsets, states, (const v2u*)sm, (const v2u*)table,       \
+                       spread, freqs, K, N,                                                      \
                        waves, (uint8_t*)out)
 #define TANS_LAUNCH_DECODE(S, FIRST) TANS_LAUNCH_DECODE_W(S, FIRST, kDecodeGroups, kDecWaves)
 #define TANS_LAUNCH_DECODE_ANY(S)                                                                 \
@@ -2828,6 +2910,25 @@ int tans_decode(const void* comp, int64_t comp_bytes, const int64_t* offsets,
 #undef TANS_LAUNCH_DECODE_W
 #undef TANS_LAUNCH_DECODE_ANY
     return hip_check(hipGetLastError(), "decode_kernel launch");
+}
+
+}  // namespace
+
+extern "C" {
+
+int tans_decode(const void* comp, int64_t comp_bytes, const int64_t* offsets,
+                const uint16_t* states, const void* sm, const uint32_t* table, int32_t log2L,
+                int64_t K, int64_t N, void* out, void* stream) {
+    return decode_launch(comp, comp_bytes, offsets, states, sm, table, nullptr, nullptr, log2L, K,
+                         N, out, stream);
+}
+
+int tans_decode_spread(const void* comp, int64_t comp_bytes, const int64_t* offsets,
+                       const uint16_t* states, const void* sm, const int32_t* spread,
+                       const int32_t* freqs, int32_t log2L, int64_t K, int64_t N, void* out,
+                       void* stream) {
+    return decode_launch(comp, comp_bytes, offsets, states, sm, nullptr, spread, freqs, log2L, K,
+                         N, out, stream);
 }
 
 int tans_fp8_gemm_fused(const void* comp, int64_t comp_bytes, const int64_t* offsets,

@@ -139,6 +139,9 @@ def _check_packed(packed: bool, N: int, log2L: int, K: int) -> None:
                  f"and at most {TANS_PACKED_MAX_N} elements per stream")
 
 
+# the most lanes for which a decode's workgroups build their own tables
+_BUILD_EACH_MAX_LANES = 1 << 20
+
 # (spread, freqs) pairs whose device table build reported no inconsistency:
 # id pair -> (weak references, data pointers and version counters).  A pair
 # is read back (one host synchronisation) only the first time it is seen and
@@ -203,15 +206,22 @@ def gpu_tans_decode(compressed: torch.Tensor, offsets: torch.Tensor, states: tor
     if K == 0 or N == 0:
         return out
     with _on(dev):
-        table = torch.empty(2 << log2L, dtype=torch.int32, device=dev)
+        stream = _stream(dev)
         verify = (not _table_known_valid(spread, freqs)
                   and not torch.cuda.is_current_stream_capturing())
-        status = torch.zeros(1, dtype=torch.int32, device=dev) if verify else None
-        stream = _stream(dev)
-        check(lib.tans_build_decode_table_device(_ptr(spread), _ptr(freqs), nsym, log2L,
-                                                 _ptr(table),
-                                                 _ptr(status) if verify else None, stream),
-              "gpu_tans_decode")
+        # Columns of more than two rounds of workgroups (32 groups on each of 256
+        # CUs) read a table built once; otherwise each workgroup builds its
+        # own, about 1 us per round against a kernel of 7 us and its launch.
+        # (Columns of one or two tiles run in one round at any lane count.)
+        # A verified table is there already.
+        build_once = verify or (K > _BUILD_EACH_MAX_LANES and N > 2 * TANS_TILE)
+        if build_once:
+            table = torch.empty(2 << log2L, dtype=torch.int32, device=dev)
+            status = torch.zeros(1, dtype=torch.int32, device=dev) if verify else None
+            check(lib.tans_build_decode_table_device(_ptr(spread), _ptr(freqs), nsym, log2L,
+                                                     _ptr(table),
+                                                     _ptr(status) if verify else None, stream),
+                  "gpu_tans_decode")
         if verify:
             rc = int(status.item())
             _require(rc == 0, "gpu_tans_decode: spread and freqs do not form a valid decode "
@@ -219,9 +229,15 @@ def gpu_tans_decode(compressed: torch.Tensor, offsets: torch.Tensor, states: tor
                               "spread's symbol counts, and be >= 2 for every present symbol "
                               "of a 2^11-state table)")
             _remember_valid_table(spread, freqs)
-        check(lib.tans_decode(_ptr(compressed), compressed.numel(), _ptr(offsets), _ptr(states),
-                              _ptr(sign_mantissa), _ptr(table), log2L, K, N, _ptr(out), stream),
-              "gpu_tans_decode")
+        if build_once:
+            check(lib.tans_decode(_ptr(compressed), compressed.numel(), _ptr(offsets),
+                                  _ptr(states), _ptr(sign_mantissa), _ptr(table), log2L, K, N,
+                                  _ptr(out), stream), "gpu_tans_decode")
+        else:
+            check(lib.tans_decode_spread(_ptr(compressed), compressed.numel(), _ptr(offsets),
+                                         _ptr(states), _ptr(sign_mantissa), _ptr(spread),
+                                         _ptr(freqs), log2L, K, N, _ptr(out), stream),
+                  "gpu_tans_decode")
     return out
 
 

@@ -26,6 +26,7 @@ EXPORTS = (
     "tans_build_decode_table_device",
     "tans_fp8_vecadd_fused",
     "tans_decode",
+    "tans_decode_spread",
     "tans_fp8_gemm_fused",
     "tans_fp8_gemm_fused_noalloc",
     "tans_fp8_gemm_raw",
@@ -75,6 +76,7 @@ for _name, _args in {
     "tans_fp8_vecadd_fused": [_P, _I64, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _I32,
                               _I64, _I64, _P, _P],
     "tans_decode": [_P, _I64, _P, _P, _P, _P, _I32, _I64, _I64, _P, _P],
+    "tans_decode_spread": [_P, _I64, _P, _P, _P, _P, _P, _I32, _I64, _I64, _P, _P],
     "tans_fp8_gemm_fused": [_P, _I64, _P, _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _P, _I64,
                             ctypes.c_float, _P, _I64, _P, _P],
     "tans_fp8_gemm_fused_noalloc": [_P, _I64, _P, _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _P,

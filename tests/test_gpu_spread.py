@@ -109,3 +109,31 @@ def test_gemm_whole_rows_equal_the_segment_sums(R, alphabet, rows, cols, segment
     y8 = R.fp8_gemm_fused_tans(m, tbl, x, 2.0 ** -9)
     y = R.fp8_gemm_fused_tans(m, tbl, x[:batch].contiguous(), 2.0 ** -9)
     assert torch.equal(y.view(torch.int16), y8[:batch].view(torch.int16))
+
+
+# the table built in each workgroup (tans_decode_spread) against a host-built
+# one (tans_decode): every decoder kernel, by alphabet, layout, tiles and waves
+@pytest.mark.parametrize("alphabet,layout,N,groups", [
+    ("pair", "auto", 16, 40), ("pair", "auto", 32, 40), ("pair", "auto", 48, 40),
+    ("pair", "auto", 64, 40), ("pair", "words", 16, 40), ("pair", "words", 64, 40),
+    ("pair", "words", 96, 40), ("pair", "words", 96, 1500), ("pair", "words", 96, 3000),
+    ("pair", "words", 96, 6000), ("nibble", "words", 16, 40), ("nibble", "words", 40, 40),
+    ("nibble", "words", 40, 1500), ("nibble", "words", 40, 3000), ("nibble", "words", 40, 6000)])
+def test_decode_builds_the_host_table(R, alphabet, layout, N, groups):
+    from rans_vectoradd import tans_codec as T
+    from rans_vectoradd._lib import lib
+    K = 64 * groups - 5
+    _say(f"case: decode_spread {K} x {N} {alphabet} {layout}")
+    a = _bytes(R, K * N, K + N).view(K, N)
+    comp, st, off, _, sm, fr, sp = T.encode_gpu(a, torch.tensor(R.QWEN3_14B_FP8_EXP),
+                                                alphabet=alphabet, layout=layout)
+    tbl = T.build_decode_table(sp.cpu().numpy(), fr.cpu().numpy()).cuda()
+    log2L = 12 if alphabet == "pair" else 11
+    stream = torch.cuda.current_stream().cuda_stream
+    outs = [torch.zeros((N, K), dtype=torch.uint8, device="cuda") for _ in range(2)]
+    args = (comp.data_ptr(), comp.numel(), off.data_ptr(), st.data_ptr() if st.numel() else None,
+            sm.data_ptr())
+    assert lib.tans_decode(*args, tbl.data_ptr(), log2L, K, N, outs[0].data_ptr(), stream) == 0
+    assert lib.tans_decode_spread(*args, sp.data_ptr(), fr.data_ptr(), log2L, K, N,
+                                  outs[1].data_ptr(), stream) == 0
+    assert torch.equal(outs[0], a.t()) and torch.equal(outs[1], a.t())
