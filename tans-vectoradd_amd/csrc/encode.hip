@@ -654,11 +654,24 @@ __device__ __forceinline__ uint32_t rank_in(Mask m) {
 // A tile's bits are appended to the unfinished word by one 64-bit shift per
 // word; the words come out of them in order, one at most per segment.  Words
 // taken past the lane's bits, and the group's padding to 4 words, are zero.
-// The stores go through a buffer resource bounded by the group's length.
 //
-// What bounds it: the vector-memory path, by its instructions: one scattered
-// store per segment.  2^29 elements at 1024 per lane, 0.58 GB: 142 us (201 us
-// with a 2-byte load per step and the bits joined step by step).
+// Words go to a ring of kRingBytes in LDS that holds the stream from byte
+// `flushed` on, and whole KiBs of it are stored 16 bytes per lane.  A place is
+// filled two crossings of its lane after it was taken, so by the time the
+// ring moves on, hundreds of words later, it is nearly always full.  A lane so
+// far behind that its place has left the ring stores the word itself, after
+// the wave's earlier stores have completed (they wrote what the ring held
+// there).  The stores go through a buffer resource bounded by the group's
+// length.
+//
+// What bounds it: memory and the vector-memory path.  2^29 elements at 1024 per
+// lane, 0.58 GB: 128 us, 142 us with one scattered store per segment (201 us
+// with a 2-byte load per step and the bits joined step by step).  Records and
+// words are non-temporal, as nothing reads them again: with cached words this
+// kernel takes 124 us, and the next call's walk, which then has to write them
+// back, 267 instead of 251.
+constexpr int kRingBytes = 4096;
+constexpr int kFlushBytes = 16 * kLanes;
 constexpr int kPlaceAhead = 4;   // tiles whose records are in flight
 
 template <int SPS>
@@ -667,6 +680,10 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_kernel(
     const int64_t* __restrict__ offsets, uint32_t* __restrict__ comp, int64_t words_total) {
     using F = TileFmt<SPS>;
     constexpr int NQ = (F::kTriple ? 160 : 96) / 32 + 1;   // words a tile's bits can touch
+    constexpr uint32_t kTileBytes = F::kSegs * kLanes * 4;   // the most a tile can hand out
+    static_assert(kRingBytes >= (int)kTileBytes + 2 * kFlushBytes && kRingBytes % kFlushBytes == 0,
+                  "a tile's words fit in the ring beside a flush");
+    __shared__ alignas(16) unsigned char rings[kEncBlock / kLanes][kRingBytes];
     const int lane = threadIdx.x & (kLanes - 1);
     // the group (wave-uniform, so the output resource stays in SGPRs)
     const int64_t g = (int64_t)blockIdx.x * (kEncBlock / kLanes) +
@@ -678,7 +695,9 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_kernel(
     const bool active = (uint32_t)lane < lanes;
     const int64_t base = offsets[g];
     const int64_t glen = offsets[g + 1] - base;
-    const Rsrc out = rsrc(comp + base, glen > 0x1FFFFFFF ? 0x7FFFFFFFu : (uint32_t)(glen * 4));
+    // the stream's bytes (a multiple of 16, as every length is of 4 words)
+    const uint32_t end = glen < 0 ? 0u : glen > 0x1FFFFFF0 ? 0x7FFFFFC0u : (uint32_t)(glen * 4);
+    const Rsrc out = rsrc(comp + base, end);
     const int64_t S = N / SPS;
     const int nt = (int)((N + kTile - 1) / kTile);   // S <= 2^24 (checked by the launcher)
     const int last_segs = (int)tans_sched::last_tile_segments(S, F::kTriple);
@@ -689,6 +708,42 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_kernel(
     uint32_t acc = 0;     // those bits
     uint32_t f0 = (uint32_t)lane * 4u, f1 = (lanes + (uint32_t)lane) * 4u;   // places (bytes)
     uint32_t handed = 8u * lanes;   // bytes handed out
+    uint32_t flushed = 0;           // bytes of the stream that have left the ring
+    bool unwaited = false;          // a flush's stores may still be on their way
+    unsigned char* ring = rings[__builtin_amdgcn_readfirstlane(threadIdx.x / kLanes)];
+    // the calling lane's word for place f (STALE: the place may have left the ring)
+    auto put = [&](uint32_t v, uint32_t f, auto STALE) {
+        if constexpr (decltype(STALE)::value) {
+            if (f < flushed) {
+                __builtin_amdgcn_raw_buffer_store_b32(v, out, f, 0, 0);
+                return;
+            }
+        }
+        *reinterpret_cast<uint32_t*>(ring + (f & (uint32_t)(kRingBytes - 1))) = v;
+    };
+    // the next KiB of the ring (bytes past the stream's end are dropped)
+    auto flush = [&]() {
+        const uint32_t at = flushed + (uint32_t)lane * 16u;
+        // (compiler barriers: the ring is written as words and read as
+        // vectors, which type-based alias analysis would let it reorder)
+        asm volatile("" ::: "memory");
+        const v4u v = *reinterpret_cast<const v4u*>(ring + (at & (uint32_t)(kRingBytes - 1)));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_raw_buffer_store_b128(v, out, at, 0, kNT);
+        flushed += (uint32_t)kFlushBytes;
+        unwaited = true;
+    };
+    // before a tile: room in the ring for all it can hand out; true if a lane
+    // of the wave holds a place that has left the ring
+    auto make_room = [&]() {
+        while (handed + kTileBytes > flushed + (uint32_t)kRingBytes) flush();   // wave-uniform
+        const bool stale = __any(active && f0 < flushed);
+        if (stale && unwaited) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            unwaited = false;
+        }
+        return stale;
+    };
     // tile t's record (zero past the last tile and in lanes out of range)
     const int64_t rec_stride = K * (kRecWords * 4);
     auto load = [&](int t) {
@@ -697,7 +752,7 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_kernel(
             rsrc(reinterpret_cast<const char*>(rec) + (int64_t)tt * rec_stride +
                      k0 * (kRecWords * 4),
                  t < nt ? lanes * (kRecWords * 4) : 0u),
-            (uint32_t)lane * (kRecWords * 4), 0, 0);
+            (uint32_t)lane * (kRecWords * 4), 0, kNT);
     };
     // the words tile t's bits make, the unfinished one first
     auto words_of = [&](const v3u& r, int t, uint32_t (&q)[NQ]) {
@@ -728,14 +783,11 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_kernel(
             q[2 + F::kOvf] = (uint32_t)(((uint64_t)prev << n) >> 32);
         }
     };
-    auto tile = [&](const v3u& r, int t) {
-        uint32_t q[NQ];
-        words_of(r, t, q);
+    auto steps = [&](const v3u& r, uint32_t (&q)[NQ], auto STALE) {
         static_for<0, F::kSegs>([&](auto I) {
             constexpr int s = decltype(I)::value;
             const Mask m = add_carry(pos, (r.x << (27 - 5 * s)) & 0xF8000000u);
-            if (__builtin_amdgcn_inverse_ballot_w64(m))
-                __builtin_amdgcn_raw_buffer_store_b32(q[0], out, f0, 0, 0);
+            if (__builtin_amdgcn_inverse_ballot_w64(m)) put(q[0], f0, STALE);
             f0 = select(m, f1, f0);
             f1 = select(m, rank_in(m) * 4u + handed, f1);
             handed += 4u * (uint32_t)__popcll(m);
@@ -744,6 +796,12 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_kernel(
             for (int i = 0; i < F::kSegs - s && i + 1 < NQ; i++) q[i] = select(m, q[i + 1], q[i]);
         });
         acc = q[0];
+    };
+    auto tile = [&](const v3u& r, int t) {
+        uint32_t q[NQ];
+        words_of(r, t, q);
+        if (make_room()) steps(r, q, std::true_type{});
+        else steps(r, q, std::false_type{});
     };
     v3u r[kPlaceAhead];
     #pragma unroll
@@ -767,6 +825,7 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_kernel(
         }
         uint32_t q[NQ];
         words_of(r[i], nt - 1, q);
+        make_room();
         #pragma unroll
         for (int s = 0; s < F::kSegs; s++) {
             if (s >= last_segs) break;   // wave-uniform
@@ -777,8 +836,7 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_kernel(
                               : s == last_segs - 2
                                   ? m & __ballot((int32_t)(pos >> 27) > (int32_t)fin_pos)
                                   : m;
-            if (__builtin_amdgcn_inverse_ballot_w64(m))
-                __builtin_amdgcn_raw_buffer_store_b32(q[0], out, f0, 0, 0);
+            if (__builtin_amdgcn_inverse_ballot_w64(m)) put(q[0], f0, std::true_type{});
             f0 = select(m, f1, f0);
             f1 = select(take, rank_in(take) * 4u + handed, f1);
             fc -= select(m & ~take, 1u, 0u);
@@ -790,16 +848,18 @@ __global__ __launch_bounds__(kEncBlock) void enc_place_kernel(
     }
     if (active) {
         if (pos >> 27) {   // the last, partial word
-            __builtin_amdgcn_raw_buffer_store_b32(acc, out, f0, 0, 0);
+            put(acc, f0, std::true_type{});
             f0 = f1;
             fc--;
         }
-        if (fc >= 1) __builtin_amdgcn_raw_buffer_store_b32(0u, out, f0, 0, 0);
-        if (fc >= 2) __builtin_amdgcn_raw_buffer_store_b32(0u, out, f1, 0, 0);
+        if (fc >= 1) put(0u, f0, std::true_type{});
+        if (fc >= 2) put(0u, f1, std::true_type{});
     }
-    // padding up to the 4-word boundary
-    if ((int64_t)handed + 4 * lane < glen * 4)
-        __builtin_amdgcn_raw_buffer_store_b32(0u, out, handed + 4u * (uint32_t)lane, 0, 0);
+    // padding up to the 4-word boundary, which the ring has room for: the last
+    // tile handed out no word after its last segment
+    if (lane < 4 && handed + 4u * (uint32_t)lane < end)
+        put(0u, handed + 4u * (uint32_t)lane, std::true_type{});
+    while (flushed < end) flush();   // wave-uniform
 }
 
 // The packed layout: one wave per group.  Each lane reads its bit count

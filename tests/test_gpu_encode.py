@@ -92,19 +92,23 @@ def test_gpu_encode_packed_config_data(R, N):
 
 
 @pytest.mark.parametrize("alphabet", ALPHABETS)
+@pytest.mark.parametrize("steep", [1.0, 14.0])
 @pytest.mark.parametrize("K,N", [(300, 16), (130, 64), (65, 30), (70, 130), (200, 400),
-                                 (64, 128), (127, 1042)])
-def test_gpu_encode_tiles_past_64_bits(R, alphabet, K, N):
+                                 (64, 128), (127, 1042), (100, 4096)])
+def test_gpu_encode_tiles_past_64_bits(R, alphabet, K, N, steep):
     """Rows that cost up to the table's longest codes (uniform bytes, steep
     histogram) beside rows that cost almost nothing (one exponent): tiles
     of more than 64 bits, whose records overflow, and lanes that cross word
-    boundaries in every segment or in hardly any, in one group.  Whole and
+    boundaries in every segment or in hardly any, in one group.  With the
+    steeper histogram a row of one exponent costs almost no bits, so its
+    words' places fall thousands of words behind the others'.  Whole and
     ragged last tiles, one and several 8-tile blocks.  Bytes equal the CPU
     encoder's."""
     from rans_vectoradd import tans_codec as T
     _say(f"case: encode_gpu overflowing tiles K={K} N={N} {alphabet}")
     torch.manual_seed(K + N)
     hist = 2.0 ** -torch.arange(16, dtype=torch.float64)
+    hist[1:] *= 2.0 ** -(steep - 1.0)
     fp8 = torch.randint(0, 256, (K, N), dtype=torch.uint8)
     fp8[::3] &= 0x87                                  # exponent 0: the shortest code
     half = torch.arange(K) % 5 == 1                   # rows that change halfway
