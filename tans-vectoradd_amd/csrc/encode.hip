@@ -418,20 +418,33 @@ struct MatSrc {
 // workspace's state array.
 constexpr int kBlockTiles = 8;   // tiles per 128-byte block of a row
 
-template <int SPS, bool PACKED, class Src>
-__global__ __launch_bounds__(kEncBlock) void enc_walk_kernel(
+// LINES (rows of whole 128-byte lines, RowSrc): a load instruction takes 8 rows'
+// lines, 8 lanes each, not 16 bytes of 64 lines; the wave turns them over
+// through 8 KiB of LDS (a row's chunks permuted by its index, so that neither
+// side conflicts).  Each line is then touched once, and the loads can be
+// non-temporal, which leaves the cache to the records.  Workgroups of 16
+// waves, so that they share the tables beside 128 KiB of rows.  2^29 elements at
+// 1024 per lane: 251 -> 204 us.
+constexpr int kLinesBlock = 1024;
+constexpr int64_t kLinesRound = 4096;   // groups of one round: 16 on each of 256 CUs
+
+template <int SPS, bool PACKED, class Src, bool LINES>
+__global__ __launch_bounds__(LINES ? kLinesBlock : kEncBlock) void enc_walk_kernel(
     Src src, int64_t K, int64_t N, const uint32_t* __restrict__ enc_tab,
     const uint16_t* __restrict__ next, int log2L, uint32_t* __restrict__ rec,
     uint32_t* __restrict__ ovf, uint16_t* __restrict__ states, uint32_t* __restrict__ glen,
     uint32_t* __restrict__ sm, uint16_t* __restrict__ plen) {
     using F = TileFmt<SPS>;
+    constexpr int kWaves = (LINES ? kLinesBlock : kEncBlock) / kLanes;
     static_assert(kEncBlock % kLanes == 0, "blocks hold whole groups");
+    static_assert(!LINES || std::is_same_v<Src, RowSrc>, "lines of a tensor's rows");
+    __shared__ alignas(16) v4u lines[LINES ? kWaves : 1][LINES ? kBlockTiles * kLanes : 1];
     __shared__ EncTab<SPS> tab;
     load_tables<SPS>(tab, enc_tab, next, log2L);
     __syncthreads();
     const int lane = threadIdx.x & (kLanes - 1);
-    const int64_t g = (int64_t)blockIdx.x * (kEncBlock / kLanes) +
-                      __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int64_t g = (int64_t)blockIdx.x * kWaves + wave;
     const int64_t k0 = g * kLanes;
     if (k0 >= K) return;
     const uint32_t lanes = (uint32_t)(K - k0 < kLanes ? K - k0 : kLanes);
@@ -496,25 +509,60 @@ __global__ __launch_bounds__(kEncBlock) void enc_walk_kernel(
     };
     v4u cur[kBlockTiles], nxt[kBlockTiles];
     int b = (nt - 1) / kBlockTiles;
-    const int full = nt - (rag ? 1 : 0);   // whole tiles
-    #pragma unroll
-    for (int c = kBlockTiles - 1; c >= 0; c--)
-        if (b * kBlockTiles + c < full) cur[c] = src.tile(b * kBlockTiles + c);   // wave-uniform
-    v4u ragged = {0u, 0u, 0u, 0u};
-    if (rag) ragged = src.last(nt - 1, rag);
-    if (b > 0) load(nxt, b - 1);
-    #pragma unroll
-    for (int c = kBlockTiles - 1; c >= 0; c--) {
-        const int t = b * kBlockTiles + c;
-        if (t < nt) tile(rag && t == nt - 1 ? ragged : cur[c], t, std::true_type{});
-    }
-    for (b--; b >= 0; b--) {
-        #pragma unroll
-        for (int c = 0; c < kBlockTiles; c++) cur[c] = nxt[c];
-        if (b > 0) load(nxt, b - 1);
+    if constexpr (LINES) {
+        // load i of a block: rows 8 i .. 8 i + 7; lane l takes the chunk of row
+        // 8 i + l / 8 that belongs at LDS place l of those rows, chunk c of
+        // row r being at place c ^ (r mod 8) of its 8
+        const int rsub = lane >> 3, chunk = (lane & 7) ^ rsub;
+        const uint8_t* first = src.fp8 + k0 * N + chunk * kTile;
+        auto load_lines = [&](int blk) {
+            #pragma unroll
+            for (int i = 0; i < kBlockTiles; i++) {
+                const uint32_t r = (uint32_t)(8 * i + rsub);
+                nxt[i] = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(
+                    first + (int64_t)(r < lanes ? r : lanes - 1) * N + blk * (kBlockTiles * kTile)));
+            }
+        };
+        v4u* stage = lines[wave];
+        auto turn = [&]() {   // the wave's LDS accesses execute in order
+            #pragma unroll
+            for (int i = 0; i < kBlockTiles; i++) stage[i * kLanes + lane] = nxt[i];
+        };
+        auto get = [&](int c) { return stage[lane * kBlockTiles + (c ^ (lane & 7))]; };
+        load_lines(b);
+        turn();
+        if (b > 0) load_lines(b - 1);
         #pragma unroll
         for (int c = kBlockTiles - 1; c >= 0; c--)
-            tile(cur[c], b * kBlockTiles + c, std::false_type{});
+            tile(get(c), b * kBlockTiles + c, std::true_type{});
+        for (b--; b >= 0; b--) {
+            turn();
+            if (b > 0) load_lines(b - 1);
+            #pragma unroll
+            for (int c = kBlockTiles - 1; c >= 0; c--)
+                tile(get(c), b * kBlockTiles + c, std::false_type{});
+        }
+    } else {
+        const int full = nt - (rag ? 1 : 0);   // whole tiles
+        #pragma unroll
+        for (int c = kBlockTiles - 1; c >= 0; c--)
+            if (b * kBlockTiles + c < full) cur[c] = src.tile(b * kBlockTiles + c);   // wave-uniform
+        v4u ragged = {0u, 0u, 0u, 0u};
+        if (rag) ragged = src.last(nt - 1, rag);
+        if (b > 0) load(nxt, b - 1);
+        #pragma unroll
+        for (int c = kBlockTiles - 1; c >= 0; c--) {
+            const int t = b * kBlockTiles + c;
+            if (t < nt) tile(rag && t == nt - 1 ? ragged : cur[c], t, std::true_type{});
+        }
+        for (b--; b >= 0; b--) {
+            #pragma unroll
+            for (int c = 0; c < kBlockTiles; c++) cur[c] = nxt[c];
+            if (b > 0) load(nxt, b - 1);
+            #pragma unroll
+            for (int c = kBlockTiles - 1; c >= 0; c--)
+                tile(cur[c], b * kBlockTiles + c, std::false_type{});
+        }
     }
     uint32_t words = 0;
     if (active) {
@@ -1008,17 +1056,30 @@ int gpu_encode_begin(const Src& src, const void* data, int64_t K, int64_t N,
     uint16_t* plen = reinterpret_cast<uint16_t*>(ws + l.plen);
     uint16_t* st_out = packed ? reinterpret_cast<uint16_t*>(ws + l.pstate) : states;
     hipStream_t st = (hipStream_t)stream;
-    const dim3 grid((unsigned)((G + kEncBlock / kLanes - 1) / (kEncBlock / kLanes)));
-    auto walk = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(kEncBlock), 0, st, src, K, N, enc_tab, enc_next,
+    auto walk = [&](auto kernel, int block = kEncBlock) {
+        const int64_t per = block / kLanes;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((G + per - 1) / per)), dim3((unsigned)block), 0,
+                           st, src, K, N, enc_tab, enc_next,
                            (int)log2L, rec, ovf, st_out, glen, (uint32_t*)sm, plen);
     };
+    bool done = false;
     if constexpr (std::is_same_v<Src, RowSrc>) {
-        if (packed) walk(enc_walk_kernel<2, true, Src>);
+        // rows of whole lines, and rounds of 16-wave workgroups that are at
+        // least three quarters full in all (the other kernel's smaller
+        // workgroups fill a part round better).  Calls with it against
+        // without, 1024 per lane: 256 groups 121 / 90 us, 2048 groups 134 / 128,
+        // 4096 groups 185 / 205, 4160 groups 249 / 226, 6250 groups 291 / 315, 8192
+        // groups 360 / 398; 62500 groups of 128 per lane 404 / 422 us.
+        const int64_t rounds = (G + kLinesRound - 1) / kLinesRound;
+        const bool lines = N % (kBlockTiles * kTile) == 0 && 4 * G >= 3 * rounds * kLinesRound;
+        done = packed || lines;
+        if (packed) walk(enc_walk_kernel<2, true, Src, false>);
+        else if (lines && sps == 2) walk(enc_walk_kernel<2, false, Src, true>, kLinesBlock);
+        else if (lines) walk(enc_walk_kernel<1, false, Src, true>, kLinesBlock);
     }
-    if (!packed) {
-        if (sps == 2) walk(enc_walk_kernel<2, false, Src>);
-        else walk(enc_walk_kernel<1, false, Src>);
+    if (!done) {
+        if (sps == 2) walk(enc_walk_kernel<2, false, Src, false>);
+        else walk(enc_walk_kernel<1, false, Src, false>);
     }
     if ((rc = hip_check(hipGetLastError(), "enc_walk_kernel launch"))) return rc;
     hipLaunchKernelGGL(enc_scan_kernel, dim3(1), dim3(kScanBlock), 0, st, glen, G, offsets,

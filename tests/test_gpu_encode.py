@@ -117,6 +117,21 @@ def test_gpu_encode_tiles_past_64_bits(R, alphabet, K, N, steep):
         _compare(T, fp8, hist, alphabet, layout)
 
 
+@pytest.mark.parametrize("alphabet", ALPHABETS)
+@pytest.mark.parametrize("groups,N", [(3072, 128), (4096, 256), (3071, 128)])
+def test_gpu_encode_rows_of_whole_lines(R, alphabet, groups, N):
+    """Tensors that fill the chip with 16-wave workgroups and whose rows are
+    whole 128-byte lines (one and two blocks of 8 tiles, a partial last
+    group), and one group fewer, which takes the other kernel: the bytes equal
+    the CPU encoder's."""
+    _say(f"case: encode_gpu whole lines {groups} groups x {N} {alphabet}")
+    from rans_vectoradd import tans_codec as T
+    K = groups * 64 - 7
+    torch.manual_seed(N)
+    fp8 = R.random_fp8_bytes(K * N, device="cpu").reshape(K, N)
+    _compare(T, fp8, torch.tensor(R.QWEN3_14B_FP8_EXP), alphabet)
+
+
 def test_gpu_encode_edge_cases(R):
     from rans_vectoradd import tans_codec as T
     exp = torch.tensor(R.QWEN3_14B_FP8_EXP)
