@@ -42,10 +42,9 @@ CASES = ([(a, K, N, "auto") for a in ALPHABETS for K, N in SHAPES]
 
 @pytest.mark.parametrize("alphabet,K,N,layout", CASES)
 def test_gpu_encode_matches_cpu(R, alphabet, K, N, layout):
-    """N % 16 == 0 takes the backward pass that reads rows in 128-byte blocks
-    (whole blocks at N = 128, 4096; a partial last block at 208, 48, 16) and
-    writes the sign/mantissa tiles itself; the other widths read one step's
-    bytes at a time and leave the tiles to enc_sm_kernel.  K % 64 != 0 and
+    """The walk reads rows in 8-tile blocks (whole blocks at N = 128, 4096; a
+    partial last block at 208, 48, 16); N % 16 != 0 reads unaligned tiles and
+    a masked last one.  K % 64 != 0 and
     K < 64 give groups with lanes out of range; N = 2 (pair) is one step.
     N = 18, 20, 34, 36 end in a tile of one refill segment (18, 34 with both
     alphabets, 20, 36 with pairs), where the check before it is the plain
