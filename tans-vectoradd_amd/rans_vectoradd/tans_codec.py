@@ -457,13 +457,15 @@ def _encode_lanes_gpu(begin, K: int, N: int, exp_freqs, alphabet: str, dev: torc
         # scan writes: one wait for the stream, no copies or launches for it
         result = torch.empty(2, dtype=torch.int64, device="cpu", pin_memory=True)
         stream = torch.cuda.current_stream(dev)
-        check(begin(log2L, tab_d.data_ptr(), next_d.data_ptr(), ws, offsets.data_ptr(),
-                    states.data_ptr(), sm.data_ptr(), result.data_ptr(), stream.cuda_stream),
-              "encode_gpu")
-        # (device copies of the cached tables, made while the passes run)
-        freqs_d, spread_d = freqs.clone(), spread.clone()
-        partial = torch.empty(0, dtype=torch.uint8, device=dev)
-        stream.synchronize()
+        try:
+            check(begin(log2L, tab_d.data_ptr(), next_d.data_ptr(), ws, offsets.data_ptr(),
+                        states.data_ptr(), sm.data_ptr(), result.data_ptr(), stream.cuda_stream),
+                  "encode_gpu")
+            # (device copies of the cached tables, made while the passes run)
+            freqs_d, spread_d = freqs.clone(), spread.clone()
+            partial = torch.empty(0, dtype=torch.uint8, device=dev)
+        finally:
+            stream.synchronize()   # also on an error: the scan writes `result`
         total, bad = result.tolist()
         if bad:
             raise RuntimeError("encode_gpu: data holds a symbol whose frequency is 0")
