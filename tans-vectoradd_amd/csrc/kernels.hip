@@ -9,13 +9,14 @@
 //                            add's launch shape (bandwidth ceilings)
 //   table_kernel<SPS>        decode table from device spread/freqs
 //                            (csrc/tans_decode.cu:23-59 without the host trip)
-//   fused_add_kernel<SPS,G,FIRST> decode two encodings + FP8 add
+//   fused_add_kernel<SPS,G,FIRST,W> decode two encodings + FP8 add
 //                            (csrc/vecadd.cu:156-243)
-//   decode_kernel<SPS,FIRST> decode to FP8 bytes [N, K]
+//   decode_kernel<SPS,FIRST,NG,W> decode to FP8 bytes [N, K]
 //                            (csrc/tans_decode.cu:125-155)
-//   gemm_fused_kernel<SPS>   decode W + skinny GEMM partial sums on the
-//                            matrix cores (no counterpart in the
-//                            reference), with gemm_finalize_kernel and the
+//   gemm_fused_kernel<SPS,WHOLE> decode W + skinny GEMM on the matrix cores
+//                            (no counterpart in the reference): partial sums
+//                            and gemm_finalize_kernel, or (WHOLE) the
+//                            product in one kernel; and the
 //                            uncompressed baselines gemm_raw_xs_kernel
 //                            (rows of up to 8192 columns), and for longer
 //                            rows gemm_raw_dot2_kernel (B = 1) and
