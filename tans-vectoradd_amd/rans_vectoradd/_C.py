@@ -19,6 +19,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 
 import torch
 
@@ -139,8 +140,27 @@ def _check_packed(packed: bool, N: int, log2L: int, K: int) -> None:
                  f"and at most {TANS_PACKED_MAX_N} elements per stream")
 
 
-# the most lanes for which a decode's workgroups build their own tables
-_BUILD_EACH_MAX_LANES = 1 << 20
+# A decode's workgroups build their own tables up to this many rounds of them
+# (32 groups on each CU), see _builds_each
+_BUILD_EACH_ROUNDS = 2
+
+
+@functools.lru_cache(maxsize=None)
+def _cu_count(device_index: int) -> int:
+    return torch.cuda.get_device_properties(device_index).multi_processor_count
+
+
+def _builds_each(K: int, N: int, cus: int) -> bool:
+    """Whether each workgroup of a decode of K lanes of N elements builds its
+    own table on `cus` CUs, or all read one that a kernel built before.  The
+    kernel is paid for once, the own tables by every round of workgroups
+    (columns of one or two tiles run in one round at any lane count).  On 256
+    CUs, us per call, kernel / own tables: pair 128 per lane, 1 round 30.5 /
+    28.4, 2 rounds 59.4 / 59.5, 3 rounds 83.2 / 86.0, 8 rounds 219.6 / 233.7;
+    1024 per lane, 2 rounds 378.8 / 378.0; nibble 128 per lane, 2 rounds 62.4 /
+    61.3, 4 rounds 124.8 / 123.6, 8 rounds 243.0 / 247.7."""
+    return N <= 2 * TANS_TILE or K <= _BUILD_EACH_ROUNDS * 32 * TANS_LANES * cus
+
 
 # (spread, freqs) pairs whose device table build reported no inconsistency:
 # id pair -> (weak references, data pointers and version counters).  A pair
@@ -209,12 +229,8 @@ def gpu_tans_decode(compressed: torch.Tensor, offsets: torch.Tensor, states: tor
         stream = _stream(dev)
         verify = (not _table_known_valid(spread, freqs)
                   and not torch.cuda.is_current_stream_capturing())
-        # Columns of more than two rounds of workgroups (32 groups on each of 256
-        # CUs) read a table built once; otherwise each workgroup builds its
-        # own, about 1 us per round against a kernel of 7 us and its launch.
-        # (Columns of one or two tiles run in one round at any lane count.)
-        # A verified table is there already.
-        build_once = verify or (K > _BUILD_EACH_MAX_LANES and N > 2 * TANS_TILE)
+        # (a verified table is there already)
+        build_once = verify or not _builds_each(K, N, _cu_count(dev.index))
         if build_once:
             table = torch.empty(2 << log2L, dtype=torch.int32, device=dev)
             status = torch.zeros(1, dtype=torch.int32, device=dev) if verify else None
