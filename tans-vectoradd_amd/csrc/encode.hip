@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "../../include/tans_amd.h"
+#include "launch.h"
 #include "schedule.h"
 
 extern "C" void tans_internal_set_error(const char* msg);  // codec.cpp
@@ -425,8 +426,8 @@ constexpr int kBlockTiles = 8;   // tiles per 128-byte block of a row
 // non-temporal, which leaves the cache to the records.  Workgroups of 16
 // waves, so that they share the tables beside 128 KiB of rows.  2^29 elements at
 // 1024 per lane: 251 -> 204 us.
-constexpr int kLinesBlock = 1024;
-constexpr int64_t kLinesRound = 4096;   // groups of one round: 16 on each of 256 CUs
+constexpr int kLinesBlock = (int)tans_launch::kLineWaves * kLanes;
+static_assert(kBlockTiles * kTile == tans_launch::kLineBytes, "a block of tiles is a line");
 
 template <int SPS, bool PACKED, class Src, bool LINES>
 __global__ __launch_bounds__(LINES ? kLinesBlock : kEncBlock) void enc_walk_kernel(
@@ -1064,14 +1065,9 @@ int gpu_encode_begin(const Src& src, const void* data, int64_t K, int64_t N,
     };
     bool done = false;
     if constexpr (std::is_same_v<Src, RowSrc>) {
-        // rows of whole lines, and rounds of 16-wave workgroups that are at
-        // least three quarters full in all (the other kernel's smaller
-        // workgroups fill a part round better).  Calls with it against
-        // without, 1024 per lane: 256 groups 121 / 90 us, 2048 groups 134 / 128,
-        // 4096 groups 185 / 205, 4160 groups 249 / 226, 6250 groups 291 / 315, 8192
-        // groups 360 / 398; 62500 groups of 128 per lane 404 / 422 us.
-        const int64_t rounds = (G + kLinesRound - 1) / kLinesRound;
-        const bool lines = N % (kBlockTiles * kTile) == 0 && 4 * G >= 3 * rounds * kLinesRound;
+        const int cus = tans_internal_cu_count();
+        if (cus <= 0) return fail(TANS_EHIP, "gpu_encode: cannot query the device's CU count");
+        const bool lines = tans_launch::whole_lines(G, N, cus);
         done = packed || lines;
         if (packed) walk(enc_walk_kernel<2, true, Src, false>);
         else if (lines && sps == 2) walk(enc_walk_kernel<2, false, Src, true>, kLinesBlock);

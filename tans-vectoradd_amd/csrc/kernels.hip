@@ -68,6 +68,7 @@
 #include <type_traits>
 
 #include "../../include/tans_amd.h"
+#include "launch.h"
 #include "schedule.h"
 
 extern "C" void tans_internal_set_error(const char* msg);  // codec.cpp
@@ -2682,6 +2683,8 @@ int scratch_address(void** out) {
 }  // namespace
 
 extern "C" {
+
+int tans_internal_cu_count() { return cu_count(); }
 
 int tans_fp8_memcpy(const void* a, void* c, int64_t n, void* stream) {
     if (n < 0 || n % 16 || ((!a || !c) && n)) return fail(TANS_EINVAL, "memcpy: n must be a multiple of 16");
