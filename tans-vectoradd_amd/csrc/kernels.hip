@@ -208,10 +208,11 @@ constexpr int kSlots = kDelay + 2;
 constexpr int kRingWords = kSlots * kSegWords;
 constexpr int kMirrorWords = kLanes;
 constexpr int kRingAlloc = kRingWords + kMirrorWords;
-constexpr int kDecWaves = 16;              // waves per workgroup
+constexpr int kDecWaves = tans_launch::kDecWaves;   // waves per workgroup
 constexpr int kSmAhead = 4;                // sign/mantissa rows are loaded this many tiles ahead
 constexpr int kLowWaves = 4;               // ... where every wave gets a SIMD to itself
 constexpr int kMidWaves = 8;               // ... where two waves share a SIMD
+static_assert(kMidWaves <= kDecWaves / 2, "the kernels for few waves run one round (spread_waves)");
 constexpr int kDecBlock = kDecWaves * kLanes;
 // At most kChecksPerStage * 64 words are handed out per stage.  A segment is
 // fetched once the one kSlots earlier in its slot is consumed; it can be
@@ -1421,12 +1422,9 @@ __global__ __launch_bounds__(W * kLanes) void fused_add_kernel(
             next_offsets(g0 + 2 * grid_groups);
         }
         w.base = done;
-        if constexpr (LOW) {
+        if constexpr (LOW) {   // one round (spread_waves)
             run_overlapped(w);
-            g0 += grid_groups;
-            if (g0 >= n_groups) break;
-            setup(g0, false);
-            continue;
+            return;
         }
         // the first n_tiles - 1 tiles four per iteration, then the last one,
         // which ends the streams (its variant chosen by tile mod 4)
@@ -1820,8 +1818,11 @@ __global__ __launch_bounds__(W * kLanes) void decode_kernel(
             }
         }
         w.base = done;
-        if constexpr (LOW) run_overlapped(w);
-        else w.run();
+        if constexpr (LOW) {   // one round (spread_waves)
+            run_overlapped(w);
+            return;
+        }
+        w.run();
         done += w.n_tiles;
         g0 += grid_groups;
         if (g0 >= n_groups) break;
@@ -2630,22 +2631,6 @@ int sps_for(int32_t log2L) {
 
 constexpr int kFusedGroups = 1;   // groups per wave in the fused kernel
 
-// Waves of each workgroup that decode, for `units` wave-sized pieces of work
-// (a wave takes one at a time) on `cus` workgroups, one per CU: as few as
-// keep the number of rounds.  The 16 waves of a full workgroup share the
-// CU's issue slots, and a wave with a SIMD to itself decodes a tile in 0.85
-// us instead of 1.9, so pieces that do not fill the chip are spread over all
-// CUs rather than packed into a few.  Fused add, 1024 per lane, 16 waves per
-// workgroup against this rule: 256 groups 91.6 -> 61.6 us, 1024 groups 93.8
-// -> 67 us, 2048 groups 96.4 -> 78 us (with the kernels for few waves, see
-// fused_add_kernel, 50, 54 and 70 us), 5000 groups (two rounds of 10 waves per
-// CU, not 16 and then 16 on a fifth of the CUs) 210 -> 180 us.
-int spread_waves(int64_t units, int cus) {
-    const int64_t per_round = (int64_t)cus * kDecWaves;
-    const int64_t rounds = (units + per_round - 1) / per_round;
-    return (int)((units + cus * rounds - 1) / (cus * rounds));
-}
-
 int gemm_fused_launch(const void* comp, int64_t comp_bytes, const int64_t* offsets,
                       const uint16_t* states, const void* sm, const uint32_t* table,
                       int32_t log2L, int64_t R, int64_t C, int64_t S, int64_t Nc, const void* x,
@@ -2798,7 +2783,7 @@ int tans_fp8_vecadd_fused(const void* a_comp, int64_t a_comp_bytes, const int64_
     // one workgroup per CU at most; the waves loop over the groups
     const int cus = cu_count();
     if (cus <= 0) return fail(TANS_EHIP, "vecadd_fused: cannot query the device's CU count");
-    const int waves = spread_waves(groups, cus);
+    const int waves = tans_launch::spread_waves(groups, cus);
     const int64_t blocks = std::min<int64_t>((groups + waves - 1) / waves, cus);
     const int n_tiles = (int)(N / kTile);
 #define TANS_LAUNCH_FUSED_W(S, FIRST, W)                                                          \
@@ -2874,7 +2859,7 @@ int decode_launch(const void* comp, int64_t comp_bytes, const int64_t* offsets,
     const bool any_length = n_tiles > (sps == 2 ? Alpha<2>::kResidentTiles : 1);
     const int per_wave = any_length && groups <= (int64_t)kMidWaves * cus ? 1 : kDecodeGroups;
     const int64_t units = (groups + per_wave - 1) / per_wave;
-    const int waves = spread_waves(units, cus);
+    const int waves = tans_launch::spread_waves(units, cus);
     int64_t blocks = (units + waves - 1) / waves;
     // Columns of one or two tiles: one workgroup per CU, the waves loop over
     // their group pairs (measured at 2^30 elements: 16 per column 923 ->
@@ -3007,7 +2992,7 @@ int gemm_fused_launch(const void* comp, int64_t comp_bytes, const int64_t* offse
     const bool whole = S * whole_pairs <= kDecWaves &&
                        B * whole_x_stride((int)std::min<int64_t>(S * Nc, INT16_MAX)) * 2 <= kWholeXBytes;
     const int waves = whole ? (int)(S * whole_pairs)
-                            : spread_waves(pairs, (int)std::max<int64_t>(1, cus / S));
+                            : tans_launch::spread_waves(pairs, (int)std::max<int64_t>(1, cus / S));
     const int64_t row_blocks = (pairs + (whole ? whole_pairs : waves) - 1) / (whole ? whole_pairs : waves);
     const int64_t blocks = whole ? row_blocks : S * row_blocks;
     if (!grid_fits(blocks, kDecBlock) || !grid_fits(B * (Rp / kLanes), kFinWaves * kLanes))

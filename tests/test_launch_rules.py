@@ -19,12 +19,14 @@ def rules(tmp_path_factory):
 extern "C" int whole_lines(int64_t G, int64_t N, int cus) {
     return tans_launch::whole_lines(G, N, cus);
 }
+extern "C" int spread_waves(int64_t units, int cus) { return tans_launch::spread_waves(units, cus); }
 ''')
     out = d / "librules.so"
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{CSRC}",
                     str(src), "-o", str(out)], check=True)
     lib = ctypes.CDLL(str(out))
     lib.whole_lines.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    lib.spread_waves.argtypes = [ctypes.c_int64, ctypes.c_int]
     return lib
 
 
@@ -56,3 +58,20 @@ def test_encoder_loads_lines_in_rounds_of_this_device(rules, cus):
         assert not rules.whole_lines(full, 192, cus) and not rules.whole_lines(full, 130, cus)
     assert not rules.whole_lines(1, 1024, cus)
     assert not rules.whole_lines(round_ + 1, 1024, cus)   # half of two rounds
+
+
+@pytest.mark.parametrize("cus", [1, 32, 256, 304])
+def test_waves_are_as_few_as_keep_the_rounds(rules, cus):
+    """1..16 waves, the rounds of 16-wave workgroups, no wave fewer; and up to 8
+    waves one round with no more workgroups than CUs, so that the kernels for
+    few waves, which take one piece per wave, leave none over."""
+    full = 16 * cus
+    around = (1, 2, cus, 8 * cus, full, 2 * full, 3 * full, 17 * full)
+    for units in sorted({u + d for u in around for d in (-1, 0, 1, 5)} - {0, -1}):
+        w = rules.spread_waves(units, cus)
+        rounds = -(-units // full)
+        assert 1 <= w <= 16
+        assert -(-units // (w * cus)) == rounds
+        assert w == 1 or -(-units // ((w - 1) * cus)) > rounds
+        if w <= 8:
+            assert rounds == 1 and -(-units // w) <= cus
