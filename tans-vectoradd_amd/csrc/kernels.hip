@@ -70,6 +70,7 @@
 #include "../../include/tans_amd.h"
 #include "launch.h"
 #include "schedule.h"
+#include "table_entry.h"
 
 extern "C" void tans_internal_set_error(const char* msg);  // codec.cpp
 
@@ -503,10 +504,9 @@ __device__ __forceinline__ void compose8(uint32_t ex_lo, uint32_t ex_hi, uint32_
 // The decode table is copied into LDS by the kDecBlock threads of a
 // decoder workgroup in two halves: table_fetch issues every load of the
 // thread, table_store writes them once they arrive.  Entries that would
-// step outside the table (nb > log2L or base + 2^nb > 2L), or read more
-// bits than the refill schedule allows (nb > 10 in a 2^11-state table), are
-// replaced by a harmless one (lds_entry), so a malformed table gives wrong
-// bytes, never an out-of-range LDS access.
+// step outside the table or read too many bits are replaced by a harmless one
+// (tans_table::lds_entry), so a malformed table gives wrong bytes, never an
+// out-of-range LDS access.
 template <uint32_t L, int T = kDecBlock>   // T: threads of the workgroup
 struct TableRegs {
     static_assert(L % T == 0, "the table is split evenly over the workgroup");
@@ -519,22 +519,11 @@ __device__ __forceinline__ void table_fetch(TableRegs<L, T>& r, const v2u* __res
     for (uint32_t k = 0; k < L / T; k++) r.e[k] = table[threadIdx.x + k * T];
 }
 
-// A table entry as the decoders keep it in LDS: one that would step outside
-// the table or read too many bits becomes a harmless one.  PACKED: the
-// packed-layout decoders' word0, which keeps nb in bits 4:0 and moves the
-// two exponents 8 bits up (bits 22:19 and 30:27), so that bits 15:0 of a sum
-// of word0s are the sum of their nb.
 template <uint32_t L, bool PACKED>
 __device__ __forceinline__ v2u lds_entry(v2u e) {
-    constexpr uint32_t log2L = 31 - __builtin_clz(L);
-    constexpr uint32_t max_nb =
-        log2L == tans_sched::kTripleLog2L ? tans_sched::kTripleMaxNb : log2L;
-    const uint32_t nb = e.x & 0xFFu;
-    const uint32_t base = e.y >> 3;
-    if (nb > max_nb || (e.x >> 27) != nb || (e.y & 7u) || base + (1u << nb) > L)
-        e = v2u{e.x & 0x07FFFF00u, 0u};
-    if constexpr (PACKED) e.x = (e.x & 0x1Fu) | ((e.x & 0x007FF800u) << 8);
-    return e;
+    constexpr int log2L = 31 - __builtin_clz(L);
+    const tans_table::Entry r = tans_table::lds_entry(log2L, PACKED, {e.x, e.y});
+    return v2u{r.x, r.y};
 }
 
 template <uint32_t L, bool PACKED = false, int T>
@@ -664,12 +653,8 @@ __device__ __forceinline__ bool table_build(TableScratch<SPS, W>& sc, const Spre
             if (q < seg / kPartSegs) rk += sc.tot[q][sv];   // wave-uniform
         const uint32_t f = sc.f[sv];
         if (rk >= f) bad = true;                   // more slots than its frequency
-        const uint32_t xp = f + rk;
-        const int top = xp ? 31 - __builtin_clz(xp) : S::kLog2L;
-        const int nb = top < S::kLog2L ? S::kLog2L - top : 0;
-        const uint32_t ex = SPS == 2 ? (((sv >> 4) << 11) | ((sv & 0xFu) << 19)) : (sv << 11);
-        emit(seg * 64 + lane,
-             v2u{(uint32_t)nb | ex | ((uint32_t)nb << 27), ((xp << nb) - S::L) * 8u});
+        const tans_table::Entry e = tans_table::entry(S::kLog2L, sv, f, rk);
+        emit(seg * 64 + lane, v2u{e.x, e.y});
     }
     return bad;
 }
