@@ -176,3 +176,55 @@ def test_misaligned_buffers_are_rejected_before_launch():
     assert lib.tans_decode(m, 1024, d, d, d, d, 12, 64, 16, d, None) == -1
     f = ctypes.c_float(1.0)
     assert lib.tans_fp8_gemm_raw(d, 128, 96, m, 1, f, d, None) == -1
+
+
+def test_encoder_sources_and_decode_spread_validate_before_launch():
+    """The encoder's begins that report through `result`, and the decode that
+    builds its own table, reject what they cannot take with TANS_EINVAL before
+    touching the device."""
+    from rans_vectoradd._lib import lib
+    P = ctypes.c_void_p
+    d = P(4096)
+    big = 1 << 30
+
+    def rejects(fn, ok, cases):
+        for i, v, message in cases:
+            args = list(ok)
+            args[i] = v
+            assert fn(*args) == -1, (i, v)
+            assert message in lib.tans_last_error(), (i, v, lib.tans_last_error())
+
+    # lanes_begin(fp8, K, N, packed, tab, next, log2L, ws, ws_bytes, off, st, sm, result, stream)
+    ok = (d, 64, 32, 0, d, d, 12, d, big, d, d, d, d, None)
+    rejects(lib.tans_gpu_encode_lanes_begin, ok,
+            [(12, None, b"null result"), (0, P(4104), b"16-byte aligned"), (2, 15, b"even N"),
+             (2, 0, b"positive"), (6, 10, b"log2L"), (8, 16, b"workspace too small"),
+             (1, 1 << 31, b"too small")] +
+            [(i, None, b"null pointer") for i in (0, 4, 5, 7, 9, 10, 11)])
+    packed = (d, 64, 32, 1, d, d, 12, d, big, d, None, d, d, None)
+    rejects(lib.tans_gpu_encode_lanes_begin, packed,
+            [(2, 66, b"N <= 64"), (6, 11, b"log2L 12"), (12, None, b"null result"),
+             (11, None, b"null pointer")])
+    huge = list(ok)
+    huge[8] = 1 << 60
+    rejects(lib.tans_gpu_encode_lanes_begin, huge,
+            [(1, 1 << 31, b"too large"), (2, (2 << 24) + 2, b"too large")])
+    # matrix_begin(w, R, C, S, Nc, pad, tab, next, log2L, ws, ws_bytes, off, st, sm, result, stream)
+    ok = (d, 100, 100, 2, 64, 8, d, d, 12, d, 1 << 60, d, d, d, d, None)
+    rejects(lib.tans_gpu_encode_matrix_begin, ok,
+            [(14, None, b"null result"), (1, 0, b"R > 0"), (1, -1, b"R > 0"), (2, 15, b"C >= 16"),
+             (4, 0, b"multiple of 32"), (4, 48, b"multiple of 32"), (4, 1056, b"1024"),
+             (3, 0, b"R > 0"), (3, 1, b"cover C"), (3, 3, b"cover C"), (3, 1 << 31, b"cover C"),
+             (5, -1, b"a byte"), (5, 256, b"a byte"), (1, 1 << 31, b"too large"),
+             (1, (1 << 31) - 1, b"too large"), (8, 10, b"log2L"), (10, 16, b"workspace too small")] +
+            [(i, None, b"null pointer") for i in (0, 6, 7, 9, 11, 12, 13)])
+    # decode_spread(comp, bytes, off, st, sm, spread, freqs, log2L, K, N, out, stream)
+    ok = (d, 1024, d, d, d, d, d, 12, 64, 32, d, None)
+    rejects(lib.tans_decode_spread, ok,
+            [(i, None, b"null pointer") for i in (0, 2, 4, 5, 6, 10)] +
+            [(i, P(4098), b"misaligned") for i in (0, 4, 5, 6, 10)] +
+            [(1, 1022, b"multiple of 4"), (7, 10, b"log2L"), (9, 31, b"even")])
+    no_states = list(ok)
+    no_states[3] = None
+    rejects(lib.tans_decode_spread, no_states, [(9, 66, b"packed"), (7, 11, b"packed")])
+    assert lib.tans_decode_spread(*ok[:8], 0, 16, d, None) == 0
