@@ -225,3 +225,117 @@ def test_checkpoint_container_on_gpu(R, tmp_path):
     y = R.fp8_gemm_fused_tans(m, m.decode_table().cuda(), x, scale).float()
     y_raw = R.fp8_gemm_raw(w.reshape(1024, 512).cuda(), x, scale).float()
     assert bool(((y - y_raw).abs() <= 2.0 ** -7 * y_raw.abs() + 1e-6).all())
+
+
+def _tables(T, lib, hist, alphabet):
+    freqs = T.symbol_freqs(hist.numpy(), alphabet)
+    spread = T.build_spread(freqs)
+    nsym, L, _ = T.ALPHABETS[alphabet]
+    tab, nxt = torch.empty(nsym, dtype=torch.int32), torch.empty(L, dtype=torch.int16)
+    assert lib.tans_build_encode_table(spread.ctypes.data, freqs.ctypes.data, nsym,
+                                       L.bit_length() - 1, tab.data_ptr(), nxt.data_ptr()) == 0
+    return tab.cuda(), nxt.cuda(), L.bit_length() - 1
+
+
+@pytest.mark.parametrize("alphabet,layout", [("pair", "words"), ("pair", "packed"),
+                                             ("nibble", "words")])
+def test_gpu_encode_begin_reports_through_status(R, alphabet, layout):
+    """tans_gpu_encode_begin and tans_gpu_encode_packed_begin with their
+    finish: the bytes of encode_gpu; the status word stays 0 on good data and
+    becomes TANS_ESYMBOL (-3) for a symbol of frequency 0; no lanes give
+    offsets {0}."""
+    from rans_vectoradd import tans_codec as T
+    from rans_vectoradd._lib import lib
+    packed = layout == "packed"
+    K, N = 517, 64
+    _say(f"case: encode begin with status {alphabet} {layout}")
+    hist = torch.tensor(R.QWEN3_14B_FP8_EXP)
+    hist[0] = 0.0
+    torch.manual_seed(3)
+    good = R.random_fp8_bytes(K * N, device="cpu").reshape(K, N)
+    good[((good >> 3) & 15) == 0] |= 1 << 3       # (no exponent 0)
+    want = T.encode_gpu(good.cuda(), hist, alphabet=alphabet, layout=layout)
+    bad = good.clone()
+    bad[516, 63] &= 0x87                          # the last lane's last element
+    tab, nxt, log2L = _tables(T, lib, hist, alphabet)
+    stream = torch.cuda.current_stream().cuda_stream
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+    off = torch.empty(-(-K // 64) + 1, dtype=torch.int64, device="cuda")
+    st = torch.empty(0 if packed else K, dtype=torch.uint16, device="cuda")
+    sm = torch.empty_like(want[4])
+
+    def begin(x, status, lanes=K):
+        args = (x.data_ptr(), lanes, N, tab.data_ptr(), nxt.data_ptr(), log2L, ws.data_ptr(),
+                ws.numel(), off.data_ptr())
+        out = (sm.data_ptr(), status.data_ptr(), stream)
+        if packed:
+            return lib.tans_gpu_encode_packed_begin(*args, *out)
+        return lib.tans_gpu_encode_begin(*args, st.data_ptr(), *out)
+
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    x = good.cuda()
+    assert begin(x, status) == 0 and status.item() == 0
+    comp = torch.empty((int(off[-1]) + 256) * 4, dtype=torch.uint8, device="cuda")
+    finish = lib.tans_gpu_encode_packed_finish if packed else lib.tans_gpu_encode_finish
+    assert finish(K, N, log2L, ws.data_ptr(), off.data_ptr(), comp.data_ptr(), comp.numel(),
+                  stream) == 0
+    for a, b in zip((comp, st, off, sm), (want[0], want[1], want[2], want[4])):
+        assert torch.equal(a.cpu(), b.cpu())
+    x = bad.cuda()
+    assert begin(x, status) == 0 and status.item() == -3
+    status.zero_()
+    off.fill_(9)
+    assert begin(x, status, 0) == 0 and status.item() == 0 and off[0].item() == 0
+
+
+# every walk that marks a symbol of frequency 0: a tensor's rows per lane and
+# as whole lines, with both alphabets, ragged rows, the packed layout; the mark
+# is set by the first and by the last lane, in the walk's first tile (the row's
+# last) and in its last one, and cleared for the same data without the symbol
+@pytest.mark.parametrize("alphabet,K,N,layout", [
+    ("pair", 300, 208, "words"), ("pair", 65, 18, "words"), ("pair", 300, 64, "packed"),
+    ("pair", 130, 2, "packed"), ("pair", 3072 * 64 - 7, 128, "words"), ("nibble", 130, 90, "words"),
+    ("nibble", 3072 * 64 - 7, 128, "words")])
+def test_gpu_encode_marks_frequency_zero(R, alphabet, K, N, layout):
+    from rans_vectoradd import tans_codec as T
+    _say(f"case: frequency 0 K={K} N={N} {alphabet} {layout}")
+    hist = torch.zeros(16)
+    hist[5:9] = torch.tensor([1.0, 2.0, 3.0, 4.0])
+    g = torch.Generator().manual_seed(K)
+    x = torch.randint(0, 256, (K, N), dtype=torch.uint8, generator=g)
+    x = ((x & 0x87) | (5 + ((x >> 3) & 3)) << 3).cuda()
+    want = [t.cpu() for t in T.encode_gpu(x, hist, alphabet=alphabet, layout=layout)]
+    for k, n in ((0, 0), (K - 1, N - 1), (K // 2, N // 2), (K - 1, 0)):
+        kept = x[k, n].clone()
+        x[k, n] = 12 << 3
+        with pytest.raises(RuntimeError, match="frequency is 0"):
+            T.encode_gpu(x, hist, alphabet=alphabet, layout=layout)
+        x[k, n] = kept
+    for a, b in zip(want, T.encode_gpu(x, hist, alphabet=alphabet, layout=layout)):
+        assert torch.equal(a, b.cpu())
+
+
+# the same for a matrix: its corners and the last column of a segment, where
+# rows and columns are padded and the last block is a half tile
+@pytest.mark.parametrize("alphabet", ALPHABETS)
+@pytest.mark.parametrize("rows,cols,segments", [(70, 95, 1), (64, 256, 2), (10, 8, 1)])
+def test_encode_matrix_marks_frequency_zero(R, alphabet, rows, cols, segments):
+    from rans_vectoradd import tans_codec as T
+    _say(f"case: matrix frequency 0 {rows}x{cols} {alphabet}")
+    hist = torch.zeros(16)
+    hist[5:9] = torch.tensor([1.0, 2.0, 3.0, 4.0])
+    g = torch.Generator().manual_seed(rows)
+    w = torch.randint(0, 256, (rows, cols), dtype=torch.uint8, generator=g)
+    w = ((w & 0x87) | (5 + ((w >> 3) & 3)) << 3).cuda()
+    want = T.encode_matrix(w, hist, segments=segments, alphabet=alphabet)
+    for r, c in ((0, 0), (rows - 1, cols - 1), (0, want.seg_cols - 1), (rows - 1, cols // 2)):
+        if c >= cols:
+            continue
+        kept = w[r, c].clone()
+        w[r, c] = 12 << 3
+        with pytest.raises(RuntimeError, match="frequency is 0"):
+            T.encode_matrix(w, hist, segments=segments, alphabet=alphabet)
+        w[r, c] = kept
+    again = T.encode_matrix(w, hist, segments=segments, alphabet=alphabet)
+    for part in ("comp", "states", "offsets", "sm"):
+        assert torch.equal(getattr(want, part).cpu(), getattr(again, part).cpu()), part
