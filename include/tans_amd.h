@@ -215,7 +215,10 @@ int tans_decode_spread(const void* comp, int64_t comp_bytes, const int64_t* offs
  * (the reference's tans_encode_interleaved, csrc/tans_codec.cpp:69-196, and
  * the split of rans_vectoradd/tans_codec.py:109-124), from FP8 bytes already
  * on the device.  Three calls:
- *   workspace  bytes of device scratch begin and finish need for [K, N]
+ *   workspace  bytes of device scratch begin and finish need for [K, N]:
+ *              16 (pair) or 24 (nibble) per lane and started 16-element
+ *              tile, and 4 per lane and per 64 lanes, each part rounded up
+ *              to 256.  Rows shorter than a tile need as much as a whole one
  *   begin      fp8 [K, N] (device, 16-byte aligned, N even), enc_tab/enc_next from
  *              tans_build_encode_table (device copies), log2L 12 (pair) or
  *              11 (nibble).  Writes offsets [ceil(K/64) + 1] (int64 words),

@@ -403,14 +403,15 @@ struct MatSrc {
 // row is fetched in one go (the lanes' rows are N bytes apart, so a line
 // read piecewise over many steps could leave the cache in between).
 //
-// What bounds it: memory.  2^29 elements at 1024 per lane take 252 us (284 us
-// with 2-byte chunks stored per step, 0.54 GB of them) for 1.21 GB read and
-// written; the same accesses without the walk take 230 us, the walk without
-// its loads and stores 97 us.  Conflict-free table reads change nothing.  The
-// sign/mantissa stores are non-temporal: nothing here reads them again, and
-// the place pass, which finds more of the records still cached, takes 142
-// instead of 149 us.  Non-temporal records: this kernel 268, the place pass
-// 131 us.
+// What bounds it: memory.  2^29 elements at 1024 per lane, 1.21 GB read and
+// written, take 202 us (6.0 TB/s) with the whole-line loads below.  Without them
+// it was 251 us (284 us with 2-byte chunks stored per step, 0.54 GB of them): the
+// same accesses without the walk took 230 us, the walk without its loads and
+// stores 97 us, conflict-free table reads changed nothing, and non-temporal
+// records cost this kernel 16 us and gave the place pass 11.  The sign/mantissa
+// stores are non-temporal: nothing here reads them again, and the place pass
+// finds more of the records still cached (142 instead of 149 us before its LDS
+// ring).
 //
 // The lanes' word counts are summed into glen[group], padded to a multiple
 // of 4.  PACKED (the packed layout): plen[k] gets the lane's bits (12 for

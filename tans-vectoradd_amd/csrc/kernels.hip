@@ -547,7 +547,9 @@ __device__ __forceinline__ void table_store(v2u* lds, const TableRegs<L, T>& r) 
 //
 // Used by table_kernel and by decode_kernel, which builds its own table in
 // LDS instead of waiting for a kernel that does (7 us; 100000 x 128 18.3 -> 14.9
-// us per call, 10007 x 1000 nibble 76.5 -> 71.7, 2^30 elements 375 -> 374).
+// us per call, 10007 x 1000 nibble 76.5 -> 71.7).  Every round of workgroups
+// builds it again, about 2.5 us each (pair; 1 us nibble), so columns of many
+// rounds read one built once (rans_vectoradd._C._builds_each).
 // ---------------------------------------------------------------------
 template <int SPS>
 struct TableShape {
@@ -1177,7 +1179,7 @@ struct FusedWave {
 // waves per SIMD): each tile's compose, add and store are put among the next
 // tile's decode steps.  A wave alone on its SIMD waits on LDS for most of a
 // tile, and about 100 of the tile's 171 VALU instructions then issue in those
-// waits (106 VGPRs).  1024 per lane, pair: 256 groups 62 -> 50 us, 2048 groups
+// waits (96 VGPRs).  1024 per lane, pair: 256 groups 62 -> 49 us, 2048 groups
 // (8 waves per CU) 78 -> 72 us; 10007 x 1008 nibble 90 -> 73 us.  With 16 waves
 // the other waves fill the waits already, and the wider live ranges cost 1-2%.
 // 8-wave workgroups are slower than 4-wave ones where 4 are enough (53 us).
@@ -1827,17 +1829,19 @@ __global__ __launch_bounds__(W * kLanes) void decode_kernel(
 // columns: the 8 columns 8 q .. 8 q + 7).  So one tile of a lane (16
 // elements) is exactly what v_mfma_f32_16x16x32_bf16 takes from that lane
 // as its A operand, split in two k-blocks of 8: the wave's 64 lanes hold a
-// 16-row x 64-column block of W.  x comes from an LDS stage of the
-// segment's columns (zero past the segment or the matrix), as the B
+// 16-row x 64-column block of W.  x comes from an LDS stage (zero past the
+// matrix; the segment's columns, or WHOLE: all columns), as the B
 // operand: lane j reads x[j % 16][the same 8 columns] (lanes j % 16 >= B
-// read a row whose products are never stored).  The 4 fp32 accumulators of
+// read a row whose sums are never stored).  The 4 fp32 accumulators of
 // lane j hold rows 4 (j / 16) .. 4 (j / 16) + 3 of the group for batch row
 // j % 16.  The batch size does not change the work per tile.
 //
 // A workgroup takes one segment and up to 32 row groups (two per wave, two
-// chains per lane).  Partial sums go to a workspace [S][B][Rp] and
-// gemm_finalize_kernel adds the S segments in a fixed order, scales and
-// rounds to bf16 (round to nearest even).
+// chains per lane; fewer where that spreads them over more CUs).  Partial
+// sums go to a workspace [S][B][Rp] and gemm_finalize_kernel adds the S
+// segments in a fixed order, scales and rounds to bf16 (round to nearest
+// even).  Or (WHOLE, where the launcher finds that it fits) a workgroup takes
+// a few row groups in all segments and does that itself.
 // ---------------------------------------------------------------------
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
@@ -2137,7 +2141,6 @@ __global__ __launch_bounds__(kDecBlock) void gemm_fused_kernel(
         }
     }
 }
-
 
 // y[b][r] = bf16(scale * sum over s of ws[s][b][r]).  A block of 4 waves
 // takes 64 consecutive outputs of one batch row: wave w sums segments

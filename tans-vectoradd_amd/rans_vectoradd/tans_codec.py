@@ -239,7 +239,7 @@ def compressed_bytes(comp, states, offsets, partial, sm) -> int:
 # ---------------------------------------------------------------------------
 
 GEMM_GROUP_ROWS = 16          # rows of a lane group of the GEMM layout
-GEMM_BLOCK_ROW_GROUPS = 32    # row groups per workgroup of the GEMM kernel
+GEMM_BLOCK_ROW_GROUPS = 32    # row groups of a full workgroup of the GEMM kernel
 GEMM_COL_UNIT = 32            # segment widths are multiples of this
 GEMM_MIN_SEG_COLS = 256       # default segments are at least this wide (64 elements per lane)
 GEMM_TARGET_BLOCKS = 256      # workgroups that fill MI355X once (one per CU)
@@ -373,10 +373,10 @@ _ENC_TABLES_MAX = 16
 
 
 def _encode_tables(exp_freqs, alphabet: str, dev: torch.device):
-    """(freqs, spread, enc_tab, enc_next) on dev for a histogram.  The
-    quantization costs about a millisecond of host time, so the tables of the
-    last few (histogram, alphabet, device) keys are kept; callers get copies
-    of freqs and spread."""
+    """(freqs, spread, enc_tab, enc_next) on dev for a histogram.  Making and
+    uploading them takes about 0.5 ms (pair; 0.13 ms nibble) of host time, so
+    the tables of the last _ENC_TABLES_MAX (histogram, alphabet, device) keys
+    are kept; callers get copies of freqs and spread."""
     h = np.ascontiguousarray(np.asarray(exp_freqs, dtype=np.float64))
     key = (alphabet, h.shape, h.tobytes(), str(dev))
     hit = _ENC_TABLES.get(key)
@@ -410,8 +410,10 @@ def encode_gpu(fp8_bytes: torch.Tensor, exp_freqs, tile: int = 0, *, alphabet: s
     the 7-tuple of encode() with the same arguments, byte for byte, as
     device tensors (freqs and spread included, ready for gpu_tans_decode).
     ``layout`` as in encode(): the packed layout of short streams by
-    default where it applies (pair alphabet, N <= 64; states empty).  Reads the stream length
-    back from the device once (the size of the compressed tensor)."""
+    default where it applies (pair alphabet, N <= 64; states empty).  Waits
+    for the device once, for the stream length (the size of the compressed
+    tensor).  A histogram that the last few calls did not have costs about
+    0.5 ms of host time for its tables (pair; 0.13 ms nibble)."""
     if not (isinstance(fp8_bytes, torch.Tensor) and fp8_bytes.dim() == 2
             and fp8_bytes.dtype == torch.uint8):
         raise ValueError("fp8_bytes must be a 2-D uint8 tensor [K, N]")
