@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes
 import dataclasses
+import threading
 
 import numpy as np
 import torch
@@ -370,6 +371,7 @@ def encode_matrix(w_fp8: torch.Tensor, exp_freqs, *, segments: int | None = None
 
 _ENC_TABLES: dict = {}
 _ENC_TABLES_MAX = 16
+_ENC_TABLES_LOCK = threading.Lock()   # several threads may encode
 
 
 def _encode_tables(exp_freqs, alphabet: str, dev: torch.device):
@@ -398,9 +400,10 @@ def _encode_tables(exp_freqs, alphabet: str, dev: torch.device):
         # may read the tables)
         tables = tuple(torch.from_numpy(t).to(dev) for t in
                        (freqs, spread, enc_tab.view(np.int32), enc_next.view(np.int16)))
-    if len(_ENC_TABLES) >= _ENC_TABLES_MAX:
-        _ENC_TABLES.pop(next(iter(_ENC_TABLES)))
-    _ENC_TABLES[key] = tables
+    with _ENC_TABLES_LOCK:
+        if key not in _ENC_TABLES and len(_ENC_TABLES) >= _ENC_TABLES_MAX:
+            _ENC_TABLES.pop(next(iter(_ENC_TABLES)))
+        _ENC_TABLES[key] = tables
     return tables
 
 

@@ -339,3 +339,40 @@ def test_encode_matrix_rejects_bad_input(T):
         T.encode_matrix(torch.zeros((4, 2000), dtype=torch.uint8), D.QWEN3_14B_FP8_EXP, segments=1)
     with pytest.raises(ValueError):
         T.encode_matrix(torch.zeros((0, 16), dtype=torch.uint8), D.QWEN3_14B_FP8_EXP)
+
+
+def test_encode_tables_of_several_threads_stay_bounded(monkeypatch):
+    """Threads that encode with more histograms than are kept: each gets its
+    tables, and no more than the limit stay."""
+    import contextlib
+    import sys
+    import threading
+
+    from rans_vectoradd import tans_codec as T
+    f = T.symbol_freqs([1.0] * 16, "nibble")
+    sp = T.build_spread(f)
+    monkeypatch.setattr(T, "_ENC_TABLES", {})
+    monkeypatch.setattr(T, "symbol_freqs", lambda *a: f)   # (the same tables, quickly)
+    monkeypatch.setattr(T, "build_spread", lambda *a: sp)
+    monkeypatch.setattr(torch.cuda, "device", lambda d: contextlib.nullcontext())
+    failed = []
+
+    def work(i):
+        try:
+            for j in range(400):
+                got = T._encode_tables([i + 1.0] + [j + 1.0] * 15, "nibble", torch.device("cpu"))
+                assert torch.equal(got[0], torch.from_numpy(f))
+        except BaseException as e:   # noqa: BLE001  (reported by the main thread)
+            failed.append(repr(e)[:80])
+
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    try:
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(8)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(interval)
+    assert not failed and len(T._ENC_TABLES) == T._ENC_TABLES_MAX
